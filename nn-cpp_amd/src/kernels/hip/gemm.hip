@@ -242,8 +242,9 @@ int64_t gemm_workspace_floats(const GemmCall& g) {
 // Configurations kNumConfigs .. kNumConfigs + kValuShapes - 1 are the VALU kernel's lane blocks (gemm_valu.hip).
 // Configuration kNumConfigs + kValuShapes forces the VALU pieces kernel on a cut product it can take,
 // kNumConfigs + kValuShapes + 1 the 16x16x4 MFMA pieces kernel, and kNumConfigs + kValuShapes + 2 the whole-depth
-// 16x16x4 chain kernel on a product that is not cut.
-int gemm_config_count() { return kNumConfigs + kValuShapes + 3; }
+// 16x16x4 chain kernel on a product that is not cut; the kRingConfigs after those are the ring kernel's tiles.
+constexpr int kFirstRing = kNumConfigs + kValuShapes + 3;
+int gemm_config_count() { return kFirstRing + kRingConfigs; }
 const char* gemm_config_name(int config) {
 	if (config == kNumConfigs + kValu2x2) return "valu 32x32 (2x2 chains per lane)";
 	if (config == kNumConfigs + kValu1x2) return "valu 16x32 (1x2 chains per lane)";
@@ -254,6 +255,7 @@ const char* gemm_config_name(int config) {
 	if (config == kNumConfigs + kValuShapes) return "valu pieces 16x16 (every piece of a cut output in one lane)";
 	if (config == kNumConfigs + kValuShapes + 1) return "mfma pieces 16x16x4 (a wave per piece, 16x16 tiles)";
 	if (config == kNumConfigs + kValuShapes + 2) return "mfma chain 16x16x4 (32x32 tiles, no LDS)";
+	if (config >= kFirstRing && config < kFirstRing + kRingConfigs) return ring_config_name(config - kFirstRing);
 
 	return (config >= 0 && config < kNumConfigs) ? configs()[config].name : "";
 }
@@ -270,8 +272,11 @@ hipError_t gemm_launch(const GemmCall& g, hipStream_t s, int config, float* work
 	if (valu_ok && config >= kNumConfigs && config < kNumConfigs + kValuShapes)
 		return gemm_valu_launch(g, config - kNumConfigs, s);
 	if (config == kNumConfigs + kValuShapes + 2 && chain4_ok(g)) return gemm_chain4_launch(g, s);
+	if (config >= kFirstRing && config < kFirstRing + kRingConfigs && ring_ok(g))
+		return gemm_ring_launch(g, s, config - kFirstRing);
 	if (config < 0 && chain4_takes(g)) return gemm_chain4_launch(g, s);
 	if ((config < 0 || config >= kNumConfigs) && valu_ok && valu_takes(g)) return gemm_valu_launch(g, valu_shape(g), s);
+	if (config < 0 && ring_takes(g)) return gemm_ring_launch(g, s);
 	if (config < 0 || config >= kNumConfigs) config = pick_config(g);
 	const Config& cf = configs()[config];
 
@@ -341,6 +346,7 @@ hipError_t gemm_launch_pair(const GemmCall& g0, const GemmCall& g1, hipStream_t 
 	if (g0.batch_count != 1 || g1.batch_count != 1 || g0.batch.ndim != 0 || g1.batch.ndim != 0) return hipSuccess;
 	if (g0.m == 0 || g0.n == 0 || g1.m == 0 || g1.n == 0) return hipSuccess;
 	if (depth_cut(g0.m, g0.n, g0.k) || depth_cut(g1.m, g1.n, g1.k)) return hipSuccess;
+	if (ring_takes(g0) || ring_takes(g1)) return hipSuccess;
 	const int c0 = pick_config(g0), c1 = pick_config(g1);
 	if (c0 != c1) return hipSuccess;
 	const Config& cf = configs()[c0];

@@ -92,6 +92,13 @@ hipError_t gemm_chain4_launch(const GemmCall& g, hipStream_t s);
 bool chain4_vec(const GemmCall& g);       // 16-byte loads of its k-contiguous operands
 GemmArgs chain4_args(const GemmCall& g);  // the chain kernel's arguments (32 x 32 tiles)
 hipError_t gemm_pieces4_launch(const GemmCall& g, hipStream_t s);
+// Whole-depth products on the ring kernel (gemm_ring.hpp): no gather, leading dimensions below 2^21, row sums (one
+// ordered sum) or the GELU epilogue (A B^T) allowed. config < 0 picks the tile by shape.
+constexpr int kRingConfigs = 4;
+bool ring_ok(const GemmCall& g);
+bool ring_takes(const GemmCall& g);  // the shapes it is routed for (measured)
+hipError_t gemm_ring_launch(const GemmCall& g, hipStream_t s, int config = -1);
+const char* ring_config_name(int config);
 // A B on the chain kernel and A^T B (row sums allowed) on the pieces kernel in one launch (gemm_pieces.hip): single
 // matrices, each taken by its own kernel's route (chain4_takes, a depth cut and pieces4_takes) and at most
 // 768 threads for the pieces' workgroup. The caller guarantees that neither product writes what the other reads or

@@ -1,0 +1,151 @@
+// gemm_ring.hip - which products run on the ring kernel (gemm_ring.hpp), on which tile, and their launch.
+#include "gemm_ring.hpp"
+
+#include <cmath>
+#include <mutex>
+
+#include "gemm.hpp"
+
+namespace nnh {
+
+namespace {
+
+enum { kRing256x128 = 0, kRing128x128 = 1, kRing64x64 = 2, kRing64x64Deep = 3 };
+
+const RingConfig* ring_configs() {
+	static const RingConfig table[kRingConfigs] = {ring_config_256x128(), ring_config_128x128(), ring_config_64x64(),
+	                                               ring_config_64x64_deep()};
+	return table;
+}
+
+// Raises the kernels' dynamic LDS limit once per device.
+hipError_t prepare_ring() {
+	static std::mutex mu;
+	static bool done[64] = {};
+	int dev = 0;
+	hipError_t e = hipGetDevice(&dev);
+	if (e != hipSuccess) return e;
+	if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
+	std::lock_guard<std::mutex> lock(mu);
+	if (done[dev]) return hipSuccess;
+	for (int i = 0; i < kRingConfigs; ++i) {
+		const RingConfig& c = ring_configs()[i];
+		for (int v = 0; v < 2; ++v)
+			for (int f = 0; f < 6; ++f) {
+				const auto fn = f < 4 ? c.fn[f][v] : f == 4 ? c.rowsum_fn[v] : c.gelu_fn[v];
+				e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+				                        c.lds_bytes);
+				if (e != hipSuccess) return e;
+			}
+	}
+	done[dev] = true;
+	return hipSuccess;
+}
+
+bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+// 16-byte operand loads: aligned rows whose contiguous length is whole chunks of four, so that no chunk crosses it.
+bool ring_vec(const GemmCall& g) {
+	bool ok = aligned16(g.a) && aligned16(g.b) && g.lda % 4 == 0 && g.ldb % 4 == 0 && (g.ta ? g.m : g.k) % 4 == 0 &&
+	          (g.tb ? g.k : g.n) % 4 == 0;
+	for (int d = 0; d < g.batch.ndim; ++d) ok = ok && g.batch.sa[d] % 4 == 0 && g.batch.sb[d] % 4 == 0;
+	return ok;
+}
+
+// The time of `tiles` workgroups on a chip of 256 CUs, in cycles of a 32-deep step. Measured per step (4096 x 4096 x
+// 2048, every layout within 3%): 256 x 128 8790 cycles (8192 of them MFMAs), 128 x 128 4610 (4096), 64 x 64 2380 for
+// the two workgroups a CU holds (2048) and 1450 for one alone (1024; 64-deep stages 1350). A workgroup's start and
+// end (first loads, stores) cost about as much as 1 to 2 steps of its own.
+double ring_cost(double tiles, double steps, int config) {
+	const double rounds = tiles / 256;
+	switch (config) {
+		case kRing256x128: return std::ceil(rounds) * (8790 * steps + 12000);
+		case kRing128x128: return std::ceil(rounds) * (4610 * steps + 9000);
+		case kRing64x64: {
+			const double pairs = std::floor(rounds / 2), rest = std::ceil(rounds - 2 * pairs);
+			return pairs * (2380 * steps + 6000) + (rest > 1 ? 2380 * steps + 6000 : rest > 0 ? 1450 * steps + 4500 : 0);
+		}
+		default: return std::ceil(rounds) * (1350 * steps + 4500);
+	}
+}
+
+int ring_pick(const GemmCall& g) {
+	const double steps = (double)((g.k + 31) / 32);
+	int best = kRing64x64;
+	double cost = 0;
+	for (int i = 0; i < kRingConfigs; ++i) {
+		// one float a lane takes the 256 x 128 tile's load addresses past its registers
+		if (i == kRing256x128 && !ring_vec(g)) continue;
+		const RingConfig& c = ring_configs()[i];
+		const double tiles = (double)((g.m + c.bm - 1) / c.bm) * (double)((g.n + c.bn - 1) / c.bn) * (double)g.batch_count;
+		const double t = ring_cost(tiles, steps, i);
+		if (i == 0 || cost == 0 || t < cost) {
+			cost = t;
+			best = i;
+		}
+	}
+	return best;
+}
+
+}  // namespace
+
+bool ring_ok(const GemmCall& g) {
+	// the offsets of a tile's rows are 32-bit byte counts: 256 rows of 2^21 floats stay below 2^31
+	constexpr int64_t kMaxLd = int64_t(1) << 21;
+	if (g.gather || g.k <= 0 || depth_cut(g.m, g.n, g.k) || g.lda >= kMaxLd || g.ldb >= kMaxLd) return false;
+	return !g.rowsum || (g.ta && !g.tb && g.rowsum_outer == 0 && g.batch_count == 1 && g.batch.ndim == 0);
+}
+
+bool ring_takes(const GemmCall& g) {
+	// Products with a 64 x 64 tile for at least half the CUs and a depth of a few stages. Measured against the tile
+	// kernels (us): 4096^3 NN 1106 -> 995, 2048^3 157 -> 137, 1024^3 28.8 -> 23.4, 8192 x 512 x 2048 NT 152 -> 136,
+	// 2048 x 512 x 8192 TN 205 -> 157, 1021 x 771 x 1533 NN (one float a lane) 79 -> 42, 300 x 3000 x 500 24 -> 15.
+	// With fewer tiles the 32 x 32 tiles' shorter chains win (768^3, 144 tiles: 16.7 us against 18.4), and products
+	// narrower than 128 with 2^22 outputs or more (attention's 256 x 64 per head) keep their 128 x 64 tiles (256 of
+	// them, 256 deep: 26 to 31 us against 29 to 33).
+	if (!ring_ok(g) || g.k < 96) return false;
+	if (g.m >= 128 && g.n < 128 && (double)g.m * (double)g.n * (double)g.batch_count >= 512.0 * 128 * 64) return false;
+	const double tiles = (double)((g.m + 63) / 64) * (double)((g.n + 63) / 64) * (double)g.batch_count;
+	return tiles >= 176;
+}
+
+hipError_t gemm_ring_launch(const GemmCall& g, hipStream_t s, int config) {
+	if (!ring_ok(g)) return hipErrorInvalidValue;
+	hipError_t e = prepare_ring();
+	if (e != hipSuccess) return e;
+	const RingConfig& c = ring_configs()[config >= 0 ? config : ring_pick(g)];
+	GemmArgs p{};
+	p.a = g.a;
+	p.b = g.b;
+	p.c = g.c;
+	p.lda = g.lda;
+	p.ldb = g.ldb;
+	p.ldc = g.ldc;
+	p.m = (int)g.m;
+	p.n = (int)g.n;
+	p.k = (int)g.k;
+	p.accumulate = g.accumulate;
+	p.tiles_m = (int)((g.m + c.bm - 1) / c.bm);
+	p.tiles_n = (int)((g.n + c.bn - 1) / c.bn);
+	p.batch_count = (int)g.batch_count;
+	p.batch = g.batch;
+	p.ep = g.ep;
+	p.pieces = 1;
+	p.piece_k = (int)g.k;
+	p.rowsum = g.rowsum;
+	p.rowsum_combine = g.rowsum_combine;
+	bool c_vec = g.ldc % 4 == 0 && aligned16(g.c) && (!g.ep.gelu_y || (aligned16(g.ep.gelu_y) && aligned16(g.ep.gelu_t)));
+	for (int d = 0; d < g.batch.ndim; ++d) c_vec = c_vec && g.batch.sc[d] % 4 == 0;
+	p.c_vec = c_vec ? 1 : 0;
+	const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * p.batch_count;
+	if (blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+	if (g.ep.gelu_y && (g.ta || !g.tb || g.rowsum)) return hipErrorInvalidValue;
+	const int v = ring_vec(g) ? 1 : 0;
+	const auto fn = g.ep.gelu_y ? c.gelu_fn[v] : g.rowsum ? c.rowsum_fn[v] : c.fn[(g.ta ? 2 : 0) + (g.tb ? 1 : 0)][v];
+	hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3((unsigned)c.threads), (size_t)c.lds_bytes, s, p);
+	return hipGetLastError();
+}
+
+const char* ring_config_name(int config) { return ring_configs()[config].name; }
+
+}  // namespace nnh

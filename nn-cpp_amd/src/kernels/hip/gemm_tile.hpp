@@ -147,6 +147,7 @@ struct GemmArgs {
 	int pieces;        // > 1: depth cut, each piece writes partial[(batch*pieces + piece)][m][n]
 	int piece_k;       // depth of one piece
 	int vec_ok;        // lda, ldb, strides multiples of 4 and a, b 16-byte aligned
+	int c_vec;         // the ring kernel only: C (and every buffer the epilogue addresses like C) takes 16-byte accesses
 	float* partial;
 	BatchDesc batch;
 	Epilogue ep;

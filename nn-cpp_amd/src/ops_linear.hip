@@ -120,10 +120,13 @@ int nnh_linear_gelu_forward(const float* x, size_t M, size_t K, const float* w, 
 	GemmCall g;
 	int rc = build_gemm(0, 1, M, n, K, x, K, w, K, h, n, 0, nullptr, &ep, g);
 	if (rc != NNH_OK || M == 0 || n == 0) return rc;
-	if (chain4_ok(g)) {  // the chain kernel applies the GELU in its epilogue
+	// the ring kernel (large products) and the chain kernel (small ones) apply the GELU in their epilogue
+	const bool on_ring = ring_takes(g) && !chain4_takes(g);
+	if (on_ring || chain4_ok(g)) {
 		g.ep.gelu_y = y;
 		g.ep.gelu_t = tanh_saved;
-		return hip_status(gemm_chain4_launch(g, reinterpret_cast<hipStream_t>(stream)), "linear gelu");
+		hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+		return hip_status(on_ring ? gemm_ring_launch(g, s) : gemm_chain4_launch(g, s), "linear gelu");
 	}
 	rc = run_gemm(g, stream, -1);
 	if (rc != NNH_OK) return rc;

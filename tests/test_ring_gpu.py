@@ -1,0 +1,84 @@
+"""The ring GEMM (gemm_ring.hpp) where it can go wrong, bit for bit against the oracle: every tile shape forced at one
+row and column below, at and past its tile, depths around its stages (fewer stages than the ring holds, a partial last
+stage of every remainder class, the accumulate point at 256), 16-byte and 4-byte loads; and, through its own route, row
+sums, the GELU epilogue and batches. The outputs are whole sums in a fixed order, so the tolerance is zero."""
+import numpy as np
+import pytest
+
+from helpers import SENTINEL, Problem, assert_same, gpu_sgemm, oracle_sgemm
+from nnh import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def ring_configs():
+    import nnh
+    return {nm: i for i, nm in enumerate(nnh.gemm_configs()) if nm.startswith("ring ")}
+
+
+def host(t):
+    import torch
+    torch.cuda.synchronize()
+    return t.cpu().numpy()
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_ring_edges(gpu, oracle, ta, tb):
+    seed = 91000
+    for name, cfg in ring_configs().items():
+        bm, bn = (int(v) for v in name.split()[1].split("_")[0].split("x"))
+        # (m, n, k, pad): pad 0 with sizes a multiple of four takes 16-byte loads, the others one float a lane
+        for m, n, k, pad in ((bm, bn, 32, 0), (bm + 4, bn - 4, 100, 0), (bm - 1, bn + 1, 33, 0), (4, 8, 4, 0), (1, 1, 1, 0),
+                             (bm, bn + 4, 256, 4), (5, bn, 288, 0), (bm + 16, 12, 300, 0), (7, 9, 95, 1), (bm + 1, 3, 161, 3),
+                             (20, 24, 500, 0)):
+            for acc in (0, 1):
+                p = Problem(ta, tb, m, n, k, pad, seed)
+                seed += 1
+                want = oracle_sgemm(oracle, p, acc)
+                assert_same(gpu_sgemm(p, acc, config=cfg), want, (name, ta, tb, m, n, k, pad, acc))
+
+
+@pytest.mark.parametrize("M,K,n", [(200, 904, 900), (133, 901, 899)])
+def test_ring_row_sums(gpu, oracle, M, K, n):
+    """A 2-D weight gradient that takes the ring: dW = G^T X with db folded in, fresh and added."""
+    import torch
+
+    import nnh
+    x, w, g = synth.normal(1, (M, K)), synth.normal(2, (n, K)), synth.normal(3, (M, n))
+    dw0, db0 = synth.normal(4, (n, K)), synth.normal(5, (n,))
+    for first in (True, False):
+        want = oracle.linear_backward(g, x, w, dw=dw0, dw_first=first, db=db0, db_first=first)
+        dw, db = torch.from_numpy(dw0).cuda(), torch.from_numpy(db0).cuda()
+        nnh.linear_backward(*(torch.from_numpy(a).cuda() for a in (g, x, w)), dw=dw, dw_first=first, db=db, db_first=first)
+        assert_same(host(dw), want[1], ("dw", M, K, n, first))
+        assert_same(host(db), want[2], ("db", M, K, n, first))
+
+
+@pytest.mark.parametrize("M,K,n", [(1000, 128, 900), (777, 99, 1021)])
+def test_ring_gelu(gpu, oracle, M, K, n):
+    import torch
+
+    import nnh
+    L, P = nnh.lib(), nnh._ptr
+    x, w, b = synth.normal(11, (M, K)), synth.normal(12, (n, K)), synth.normal(13, (n,))
+    h0 = oracle.linear_forward(x, w, b)
+    y0, t0 = oracle.gelu_forward(h0)
+    xd, wd, bd = (torch.from_numpy(a).cuda() for a in (x, w, b))
+    h, y, t = (torch.full((M, n), float(SENTINEL), device="cuda") for _ in range(3))
+    nnh.check(L.nnh_linear_gelu_forward(P(xd), M, K, P(wd), n, P(bd), P(h), P(y), P(t), nnh._stream(None)))
+    for got, want, what in ((h, h0, "h"), (y, y0, "y"), (t, t0, "tanh")):
+        assert_same(host(got), want, (what, M, K, n))
+
+
+@pytest.mark.parametrize("shape", [(3, 500, 100, 450), (5, 449, 130, 451)])
+def test_ring_batches(gpu, oracle, shape):
+    """A batch of products, the right operand broadcast; the tiles of different matrices share one launch."""
+    import torch
+
+    import nnh
+    nb, m, k, n = shape
+    a, b = synth.normal(21, (nb, m, k)), synth.normal(22, (nb, k, n))
+    got = host(nnh.matmul(torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()))
+    for i in range(nb):
+        want = oracle.sgemm(0, 0, m, n, k, a[i], k, b[i], n, np.zeros((m, n), np.float32), n, 0)
+        assert_same(got[i], want, (shape, i))
