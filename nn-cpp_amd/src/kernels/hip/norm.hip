@@ -18,6 +18,7 @@
 #include "norm.hpp"
 
 #include <algorithm>
+#include <mutex>
 
 #include "fastdiv.hpp"
 
@@ -544,82 +545,50 @@ __global__ void __launch_bounds__(256) ln_backward_kernel(const LnBwdArgs a) {
 	if (a.dbeta) a.dbeta[col] = a.db_first ? 0.0f + sb : a.dbeta[col] + sb;
 }
 
-// ---- layernorm with its rows staged in LDS ----
-// A workgroup owns `rw` consecutive rows (a contiguous block of rw * D floats): its 256 threads copy the block into
-// LDS with 16-byte coalesced loads, all issued before the first LDS store (row pitch D + 1, so lane r walking row r
-// hits bank (r + j) mod 64), lane r of wave 0 runs row r's chains over LDS and writes its outputs back into its LDS
-// row, and the 256 threads copy the block out with coalesced stores. The LDS budget is 64 KB of floats (16384):
-// rw = min(64, 16384 / (D + 1)) rows for the forward, about half of that for the backward (g and x), and no more
-// than R / 256 rows when that leaves about 256 workgroups on a small input.
+// ---- layernorm, a few rows per workgroup ----
+// A workgroup of 256 threads owns `rw` consecutive rows (a contiguous block of rw * D floats) and keeps them in
+// registers from the load to the store. Only the row chains (one dependent add per element, the reference's order) run
+// over LDS: all threads put the terms there, element-wise, and one lane per chain adds them in order, sixteen at a time
+// from 16-byte reads two blocks ahead, about 7 cycles an add (4.3 from registers; the reads take the rest). The rows of
+// LDS are padded to a multiple of four floats plus four, so that the lanes of a read (one row each) use different banks.
+// What bounds it: the two (forward) or one (backward) chain of D adds, 1.3 us at D = 512, between the load and the store;
+// rw is chosen so that 2 to 4 workgroups share a CU and one's chain runs beside another's memory traffic. Measured
+// over [8192, 512]: forward 22.8 -> 12.4 us, dx alone 37.2 -> 12.0, against a version that also ran the element-wise
+// passes in the chain lanes.
+// PER: 16-byte groups (VEC) or quadruples of floats a thread holds: rw * D <= 1024 PER.
 
-constexpr int kLnLdsFloats = 16384;
-constexpr int kLnLoadPer = kLnLdsFloats / 4 / 256;  // float4 loads per thread for a full block (16)
+constexpr int kLnMaxRows = 32;  // chains of one kind in a wave: lanes 0 .. 31, the backward's second kind lanes 32 .. 63
 
-__device__ __forceinline__ void ln_block_load(const float* __restrict__ src, int nr, int D, int pitch, int vec,
-                                              const FastDiv& dq, float* dst) {
-	const int tid = threadIdx.x;
-	const int total = nr * D;
-	if (vec) {
-		const int q4 = D >> 2, tot = total >> 2;
-		if (tot == 0) return;
-		f32x4 v[kLnLoadPer];
+__device__ __host__ __forceinline__ int ln_pitch(int D) { return ((D + 3) & ~3) + 4; }
+
+// acc + v[0] + v[1] + ... + v[n - 1] in order; v is 16-byte aligned LDS.
+__device__ __forceinline__ float lds_chain(const float* v, int n, float acc = 0.0f) {
+	const f32x4* q = reinterpret_cast<const f32x4*>(v);
+	const int nb = n / 16;
+	if (nb > 0) {
+		f32x4 t[3][4];
 #pragma unroll
-		for (int u = 0; u < kLnLoadPer; ++u) {
-			const int q = min(tid + 256 * u, tot - 1);
-			v[u] = *reinterpret_cast<const f32x4*>(src + 4 * q);
-		}
+		for (int e = 0; e < 4; ++e) t[0][e] = q[e];
 #pragma unroll
-		for (int u = 0; u < kLnLoadPer; ++u) {
-			const int q = tid + 256 * u;
-			if (q < tot) {
-				const int r = (int)fdiv((unsigned)q, dq), c = 4 * (q - r * q4);
+		for (int e = 0; e < 4; ++e) t[1][e] = q[4 * min(1, nb - 1) + e];
+		for (int b = 0; b < nb; b += 3) {
 #pragma unroll
-				for (int i = 0; i < 4; ++i) dst[r * pitch + c + i] = v[u][i];
-			}
-		}
-	} else {
-		for (int b = 0; b < total; b += 256 * 16) {
-			float v[16];
+			for (int k = 0; k < 3; ++k) {
+				// past the end a redundant read of the last block: no branch around a read
 #pragma unroll
-			for (int u = 0; u < 16; ++u) v[u] = src[min(b + tid + 256 * u, total - 1)];
+				for (int e = 0; e < 4; ++e) t[(k + 2) % 3][e] = q[4 * min(b + k + 2, nb - 1) + e];
+				__builtin_amdgcn_sched_barrier(0);  // keeps the reads ahead of the adds they run beside
+				if (b + k < nb) {
 #pragma unroll
-			for (int u = 0; u < 16; ++u) {
-				const int e = b + tid + 256 * u;
-				if (e < total) {
-					const int r = (int)fdiv((unsigned)e, dq);
-					dst[r * pitch + e - r * D] = v[u];
+					for (int e = 0; e < 4; ++e)
+#pragma unroll
+						for (int i = 0; i < 4; ++i) acc = acc + t[k][e][i];
 				}
 			}
 		}
 	}
-}
-
-// dst (global) = block in LDS; with add, dst = old + block (the backward's accumulate).
-__device__ __forceinline__ void ln_block_store(float* __restrict__ dst, int nr, int D, int pitch, int vec,
-                                               const FastDiv& dq, const float* src, bool add) {
-	const int tid = threadIdx.x;
-	const int total = nr * D;
-	if (vec) {
-		const int q4 = D >> 2, tot = total >> 2;
-		for (int q = tid; q < tot; q += 256) {
-			const int r = (int)fdiv((unsigned)q, dq), c = 4 * (q - r * q4);
-			f32x4 v;
-#pragma unroll
-			for (int i = 0; i < 4; ++i) v[i] = src[r * pitch + c + i];
-			if (add) {
-				const f32x4 o = *reinterpret_cast<const f32x4*>(dst + 4 * q);
-#pragma unroll
-				for (int i = 0; i < 4; ++i) v[i] = o[i] + v[i];
-			}
-			*reinterpret_cast<f32x4*>(dst + 4 * q) = v;
-		}
-	} else {
-		for (int e = tid; e < total; e += 256) {
-			const int r = (int)fdiv((unsigned)e, dq);
-			const float v = src[r * pitch + e - r * D];
-			dst[e] = add ? dst[e] + v : v;
-		}
-	}
+	for (int j = 16 * nb; j < n; ++j) acc = acc + v[j];
+	return acc;
 }
 
 struct LnArgs {
@@ -633,264 +602,310 @@ struct LnArgs {
 	float* mean;           // forward
 	float* inv;            // forward
 	int64_t R;
-	int D, rw, vec, first;
+	int D, rw, first;
 	float fd, eps;
-	FastDiv dq;            // D / 4 (vec) or D
-	FastDiv dd;            // D
+	FastDiv dq;            // D / 4 (VEC) or D
 };
 
-// layernorm forward (ops.cpp:1017-1030) on rw rows per workgroup.
-__global__ void __launch_bounds__(256) ln_forward_lds_kernel(const LnArgs a) {
-	extern __shared__ __align__(16) float lds[];
-	const int pitch = a.D + 1;
-	const int64_t r0 = (int64_t)blockIdx.x * a.rw;
-	const int nr = (int)(a.R - r0 < a.rw ? a.R - r0 : a.rw);
-	ln_block_load(a.x + r0 * a.D, nr, a.D, pitch, a.vec, a.dq, lds);
-	__syncthreads();
-	const int r = threadIdx.x;
-	if (r < nr) {
-		float* row = lds + r * pitch;
-		const int D16 = a.D & ~15;
-		float sum = 0.0f;
-		for (int j = 0; j < D16; j += 16) {  // 16 LDS reads issued, then the 16 dependent adds
-			float v[16];
+// The workgroup's elements as units of four consecutive floats of a row (VEC) or single floats (four to a slot): unit
+// e of slot u. Calls f(slot, element in the slot, row, column, index in the block) for every element of the block, and
+// with 16-byte units the elements of a slot share a row.
+template <int PER, bool VEC, class F>
+__device__ __forceinline__ void ln_each(int total, int D, const FastDiv& dq, F&& f) {
+	const int tid = threadIdx.x;
 #pragma unroll
-			for (int u = 0; u < 16; ++u) v[u] = row[j + u];
+	for (int u = 0; u < PER; ++u) {
+		if constexpr (VEC) {
+			const int q = tid + 256 * u;
+			if (4 * q < total) {
+				const int r = (int)fdiv((unsigned)q, dq), c = 4 * (q - r * (D >> 2));
+				f(u, r, c, 4 * q);
+			}
+		} else {
 #pragma unroll
-			for (int u = 0; u < 16; ++u) sum = sum + v[u];
+			for (int i = 0; i < 4; ++i) {
+				const int e = tid + 256 * (4 * u + i);
+				if (e < total) {
+					const int r = (int)fdiv((unsigned)e, dq);
+					f(4 * u + i, r, e - r * D, e);
+				}
+			}
 		}
-		for (int j = D16; j < a.D; ++j) sum = sum + row[j];
-		const float mu = sum / a.fd;
-		float sq = 0.0f;
-		for (int j = 0; j < D16; j += 16) {
-			float v[16];
-#pragma unroll
-			for (int u = 0; u < 16; ++u) v[u] = row[j + u];
-#pragma unroll
-			for (int u = 0; u < 16; ++u) sq = sq + (v[u] - mu) * (v[u] - mu);
-		}
-		for (int j = D16; j < a.D; ++j) sq = sq + (row[j] - mu) * (row[j] - mu);
-		const float inv = 1.0f / sqrtf(sq / a.fd + a.eps);
-		a.mean[r0 + r] = mu;
-		a.inv[r0 + r] = inv;
-		for (int j = 0; j < D16; j += 16) {
-			float v[16];
-#pragma unroll
-			for (int u = 0; u < 16; ++u) v[u] = row[j + u];
-#pragma unroll
-			for (int u = 0; u < 16; ++u) row[j + u] = (v[u] - mu) * inv * a.gm[j + u] + a.bt[j + u];
-		}
-		for (int j = D16; j < a.D; ++j) row[j] = (row[j] - mu) * inv * a.gm[j] + a.bt[j];
 	}
-	__syncthreads();
-	ln_block_store(a.y + r0 * a.D, nr, a.D, pitch, a.vec, a.dq, lds, false);
 }
 
-// layernorm backward's dx (ops.cpp:1043-1060) on rw rows per workgroup. g and x are staged in LDS; all 256 threads
-// form the products dxhat * ((x - mean) * inv_std) of the second sum elementwise, so the lane that owns a row only
-// runs its two addition chains (sa over g * gamma, sb over the products, both in column order); then all threads
-// write dx = k * (D * dxhat - sa - xhat * sb) elementwise, straight to HBM.
-__device__ __forceinline__ void ln_dx_body(const LnArgs& a, int block, float* lds) {
-	const int pitch = a.D + 1;
-	float* gs = lds;
-	float* xs = gs + a.rw * pitch;
-	float* gms = xs + a.rw * pitch;
-	float* st = gms + a.D;  // per row: mean, inv_std, sa, sb
+// The block's elements into registers, every load issued at an index clamped into the block.
+template <int PER, bool VEC>
+__device__ __forceinline__ void ln_load(const float* __restrict__ src, int total, f32x4 (&v)[PER]) {
 	const int tid = threadIdx.x;
+#pragma unroll
+	for (int u = 0; u < PER; ++u) {
+		if constexpr (VEC) {
+			v[u] = *reinterpret_cast<const f32x4*>(src + 4 * min(tid + 256 * u, total / 4 - 1));
+		} else {
+#pragma unroll
+			for (int i = 0; i < 4; ++i) v[u][i] = src[min(tid + 256 * (4 * u + i), total - 1)];
+		}
+	}
+}
+
+// layernorm forward (ops.cpp:1017-1030) on rw rows per workgroup.
+template <int PER, bool VEC>
+__global__ void __launch_bounds__(256) ln_forward_rows_kernel(const LnArgs a) {
+	extern __shared__ __align__(16) float lds[];
+	const int D = a.D, pitch = ln_pitch(D), tid = threadIdx.x;
+	float* st = lds + a.rw * pitch;  // per row: mean, inv_std
+	const int64_t r0 = (int64_t)blockIdx.x * a.rw;
+	const int nr = (int)(a.R - r0 < a.rw ? a.R - r0 : a.rw), total = nr * D;
+	f32x4 v[PER];
+	ln_load<PER, VEC>(a.x + r0 * D, total, v);
+	ln_each<PER, VEC>(total, D, a.dq, [&](int s, int r, int c, int) {
+		if constexpr (VEC) *reinterpret_cast<f32x4*>(lds + r * pitch + c) = v[s];
+		else lds[r * pitch + c] = v[s / 4][s % 4];
+	});
+	__syncthreads();
+	if (tid < nr) st[2 * tid] = lds_chain(lds + tid * pitch, D) / a.fd;
+	__syncthreads();
+	ln_each<PER, VEC>(total, D, a.dq, [&](int s, int r, int c, int) {
+		const float mu = st[2 * r];
+		if constexpr (VEC) {
+			f32x4 sq;
+#pragma unroll
+			for (int i = 0; i < 4; ++i) sq[i] = (v[s][i] - mu) * (v[s][i] - mu);
+			*reinterpret_cast<f32x4*>(lds + r * pitch + c) = sq;
+		} else {
+			lds[r * pitch + c] = (v[s / 4][s % 4] - mu) * (v[s / 4][s % 4] - mu);
+		}
+	});
+	__syncthreads();
+	if (tid < nr) {
+		const float inv = 1.0f / sqrtf(lds_chain(lds + tid * pitch, D) / a.fd + a.eps);
+		st[2 * tid + 1] = inv;
+		a.mean[r0 + tid] = st[2 * tid];
+		a.inv[r0 + tid] = inv;
+	}
+	__syncthreads();
+	float* out = a.y + r0 * D;
+	ln_each<PER, VEC>(total, D, a.dq, [&](int s, int r, int c, int e) {
+		const float mu = st[2 * r], inv = st[2 * r + 1];
+		if constexpr (VEC) {
+			f32x4 o;
+#pragma unroll
+			for (int i = 0; i < 4; ++i) o[i] = (v[s][i] - mu) * inv * a.gm[c + i] + a.bt[c + i];
+			*reinterpret_cast<f32x4*>(out + e) = o;
+		} else {
+			out[e] = (v[s / 4][s % 4] - mu) * inv * a.gm[c] + a.bt[c];
+		}
+	});
+}
+
+// layernorm backward's dx (ops.cpp:1043-1060) on rw rows per workgroup: the terms g gamma and (g gamma) ((x - mean)
+// inv_std) go to LDS for the row's two chains and stay in registers, as dxhat and xhat, for
+// dx = k (D dxhat - sa - xhat sb).
+template <int PER, bool VEC>
+__device__ __forceinline__ void ln_dx_body(const LnArgs& a, int block, float* lds) {
+	const int D = a.D, pitch = ln_pitch(D), tid = threadIdx.x;
+	float* la = lds;
+	float* lb = la + a.rw * pitch;
+	float* st = lb + a.rw * pitch;  // per row: mean, inv_std, sa, sb
 	const int64_t r0 = (int64_t)block * a.rw;
-	const int nr = (int)(a.R - r0 < a.rw ? a.R - r0 : a.rw);
-	ln_block_load(a.g + r0 * a.D, nr, a.D, pitch, a.vec, a.dq, gs);
-	ln_block_load(a.x + r0 * a.D, nr, a.D, pitch, a.vec, a.dq, xs);
-	for (int j = tid; j < a.D; j += 256) gms[j] = a.gm[j];
+	const int nr = (int)(a.R - r0 < a.rw ? a.R - r0 : a.rw), total = nr * D;
+	f32x4 dxh[PER], xh[PER];
+	ln_load<PER, VEC>(a.g + r0 * D, total, dxh);
+	ln_load<PER, VEC>(a.x + r0 * D, total, xh);
 	if (tid < nr) {
 		st[4 * tid] = a.mean_in[r0 + tid];
 		st[4 * tid + 1] = a.inv_in[r0 + tid];
 	}
 	__syncthreads();
-	if (tid < nr) {
-		// the row's two chains (ops.cpp:1040-1047): sa += g gamma, sb += (g gamma) ((x - mean) inv_std), each
-		// product formed as the reference forms it, 16 steps' LDS reads issued before their arithmetic
-		const float* gr = gs + tid * pitch;
-		const float* xr = xs + tid * pitch;
-		const float mu = st[4 * tid], iv = st[4 * tid + 1];
-		const int D16 = a.D & ~15;
-		float sa = 0.0f, sb = 0.0f;
-		for (int j = 0; j < D16; j += 16) {
-			float gv[16], mv[16], xv[16];
+	ln_each<PER, VEC>(total, D, a.dq, [&](int s, int r, int c, int) {
+		const float mu = st[4 * r], iv = st[4 * r + 1];
+		if constexpr (VEC) {
+			f32x4 p;
 #pragma unroll
-			for (int u = 0; u < 16; ++u) {
-				gv[u] = gr[j + u];
-				mv[u] = gms[j + u];
-				xv[u] = xr[j + u];
+			for (int i = 0; i < 4; ++i) {
+				dxh[s][i] = dxh[s][i] * a.gm[c + i];
+				xh[s][i] = (xh[s][i] - mu) * iv;
+				p[i] = dxh[s][i] * xh[s][i];
 			}
-#pragma unroll
-			for (int u = 0; u < 16; ++u) {
-				const float dxhat = gv[u] * mv[u];
-				sa = sa + dxhat;
-				sb = sb + dxhat * ((xv[u] - mu) * iv);
-			}
+			*reinterpret_cast<f32x4*>(la + r * pitch + c) = dxh[s];
+			*reinterpret_cast<f32x4*>(lb + r * pitch + c) = p;
+		} else {
+			float& d = reinterpret_cast<float(&)[4 * PER]>(dxh)[s];
+			float& h = reinterpret_cast<float(&)[4 * PER]>(xh)[s];
+			d = d * a.gm[c];
+			h = (h - mu) * iv;
+			la[r * pitch + c] = d;
+			lb[r * pitch + c] = d * h;
 		}
-		for (int j = D16; j < a.D; ++j) {
-			const float dxhat = gr[j] * gms[j];
-			sa = sa + dxhat;
-			sb = sb + dxhat * ((xr[j] - mu) * iv);
-		}
-		st[4 * tid + 2] = sa;
-		st[4 * tid + 3] = sb;
+	});
+	__syncthreads();
+	if (tid < 64 && (tid & (kLnMaxRows - 1)) < nr) {
+		const int r = tid & (kLnMaxRows - 1), second = tid / kLnMaxRows;
+		st[4 * r + 2 + second] = lds_chain((second ? lb : la) + r * pitch, D);
 	}
 	__syncthreads();
 	const float fd = a.fd;
-	float* dst = a.y + r0 * a.D;
-	const int total = nr * a.D;
-	for (int e = tid; e < total; e += 256) {
-		const int r = (int)fdiv((unsigned)e, a.dd), j = e - r * a.D;
-		const float mu = st[4 * r], inv = st[4 * r + 1], sa = st[4 * r + 2], sb = st[4 * r + 3];
-		const float k = inv / fd;
-		const float dxhat = gs[r * pitch + j] * gms[j];
-		const float term = k * (fd * dxhat - sa - ((xs[r * pitch + j] - mu) * inv) * sb);
-		dst[e] = a.first ? term + 0.0f : dst[e] + term;
-	}
+	float* dst = a.y + r0 * D;
+	ln_each<PER, VEC>(total, D, a.dq, [&](int s, int r, int, int e) {
+		const float k = st[4 * r + 1] / fd, sa = st[4 * r + 2], sb = st[4 * r + 3];
+		if constexpr (VEC) {
+			f32x4 o;
+			if (!a.first) o = *reinterpret_cast<const f32x4*>(dst + e);
+#pragma unroll
+			for (int i = 0; i < 4; ++i) {
+				const float term = k * (fd * dxh[s][i] - sa - xh[s][i] * sb);
+				o[i] = a.first ? term + 0.0f : o[i] + term;
+			}
+			*reinterpret_cast<f32x4*>(dst + e) = o;
+		} else {
+			const float term = k * (fd * dxh[s / 4][s % 4] - sa - xh[s / 4][s % 4] * sb);
+			dst[e] = a.first ? term + 0.0f : dst[e] + term;
+		}
+	});
 }
 
-__global__ void __launch_bounds__(256) ln_dx_lds_kernel(const LnArgs a) {
-	extern __shared__ __align__(16) float lds[];
-	ln_dx_body(a, (int)blockIdx.x, lds);
-}
+struct LnColArgs {
+	const float* g;
+	const float* x;
+	const float* mean;
+	const float* inv;
+	int64_t R;
+	int D;
+	float* dgamma;
+	int dg_first;
+	float* dbeta;
+	int db_first;
+	int blocks;  // workgroups of the column chains
+};
 
 // layernorm backward's dgamma and dbeta (ops.cpp:1061-1076): each is a chain down a column in row order, so the
-// columns are the only parallelism. A workgroup owns 32 columns and streams the rows in chunks of 120. Waves 1-15
-// produce: each thread loads four rows of its column (or, VEC, one row's four columns with 16-byte loads) with the
-// rows' mean and inv_std, four chunks ahead in a register ring, and writes g * ((x - mean) * inv_std), formed
-// exactly as the reference forms it, and g into the chunk's LDS buffer (a row of 64 floats: the products, then g,
-// so wave 0 reads 64 consecutive words). Wave 0 consumes one chunk behind: lanes 0-31 add the products down their
-// column (dgamma), lanes 32-63 add g (dbeta), 24 rows' LDS reads in flight while they add eight. One barrier per
-// chunk; two buffers. Measured at [32, 256, 512]: 53 us (the chains of 8192 rows bound it near 23 us; 8-column
-// blocks, 4x the workgroups, and a raised wave priority for the chains measured no faster).
-constexpr int kLnCols = 32, kLnProducers = 960, kLnThreads = 64 + kLnProducers, kLnAhead = 4, kLnPer = 4;
-constexpr int kLnRowStride = kLnProducers / kLnCols;  // 30: a scalar producer's rows are rr + 30 u
-constexpr int kLnChunk = kLnRowStride * kLnPer;       // 120 rows
-constexpr int kLnVecPerRow = kLnCols / 4;             // 8 16-byte loads cover a row's columns
+// columns are the only parallelism, and about 7 cycles a row (24 us for 8192 rows) the least time. A workgroup of
+// four waves, one a SIMD, owns 16 columns: waves 1-3 load the rows in chunks of 192, three chunks ahead in a register
+// ring, form g * ((x - mean) * inv_std) exactly as the reference does and write it and g to LDS column by column (a
+// column's rows back to back); wave 0, one chunk behind, adds: lanes 0-15 the products down their column (dgamma),
+// lanes 16-31 g (dbeta), four rows per 16-byte read. One barrier a chunk, two buffers. 16 columns a workgroup keep the
+// loads (64 bytes a row) at a third of what a CU can take. Measured for 8192 rows of 512: 37 us, and 41 with dx beside it
+// (52 and 90 in two launches with 32 columns and fifteen producer waves, where the chain wave shared its SIMD with three
+// producers and read one row at a time); of 64: 30 us against 51.
+constexpr int kLnCols = 16, kLnAhead = 3, kLnWaveRows = 64, kLnChunk = 3 * kLnWaveRows;
+constexpr int kLnColPitch = kLnChunk + 4;  // 4 mod 64: the chain lanes' 16-byte reads use different banks
+constexpr int kLnColBuf = 2 * kLnCols * kLnColPitch;
+constexpr size_t kLnColLds = 2 * kLnColBuf * sizeof(float);
 
 template <bool VEC>
-__global__ void __launch_bounds__(kLnThreads) ln_dgamma_kernel(const float* __restrict__ g,
-                                                               const float* __restrict__ x,
-                                                               const float* __restrict__ mean,
-                                                               const float* __restrict__ inv, int64_t R, int D,
-                                                               float* dgamma, int dg_first, float* dbeta,
-                                                               int db_first) {
-	__shared__ __align__(16) float buf[2][kLnChunk][2 * kLnCols];
-	const int tid = threadIdx.x;
-	const int c0 = blockIdx.x * kLnCols;
-	const int64_t chunks = (R + kLnChunk - 1) / kLnChunk;
-	const bool producer = tid >= 64;
-	const bool consumer = !producer;
-	const int pt = tid - 64;
-	// scalar: column c of rows rr + 30 u; VEC: columns 4 q4 .. 4 q4 + 3 of row vr
-	const int c = pt % kLnCols, rr = pt / kLnCols;
-	const int q4 = pt % kLnVecPerRow, vr = pt / kLnVecPerRow;
-	constexpr int kVecRows = kLnProducers / kLnVecPerRow;  // 120: one row per producer thread and chunk
-	static_assert(kVecRows == kLnChunk, "a VEC producer owns one row of a chunk");
-	const int col = min(c0 + c, D - 1);
-	const int col4 = min(c0 + 4 * q4, D - 4);
-	float gv[kLnAhead][kLnPer], xv[kLnAhead][kLnPer], mv[kLnAhead][kLnPer], iv[kLnAhead][kLnPer];
-	auto load = [&](int64_t ch, int slot) {
-		if (VEC) {
-			const int64_t r = min(ch * kLnChunk + vr, R - 1);
-			const f32x4 g4 = *reinterpret_cast<const f32x4*>(g + r * D + col4);
-			const f32x4 x4 = *reinterpret_cast<const f32x4*>(x + r * D + col4);
-			const float m = mean[r], iv0 = inv[r];
+__device__ __forceinline__ void ln_columns_body(const LnColArgs& d, int block, float* lds) {
+	const int tid = threadIdx.x, lane = tid & 63;
+	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const int c0 = block * kLnCols, D = d.D;
+	const int64_t R = d.R, chunks = (R + kLnChunk - 1) / kLnChunk;
+	// a producer's slot u of a chunk: VEC row 16 u + lane / 4, columns 4 (lane % 4) ..; else row 4 u + lane / 16, column
+	// lane % 16 (columns past D read a clamped address: their chains are not stored)
+	constexpr int kSlots = VEC ? kLnWaveRows / 16 : kLnWaveRows / 4, kW = VEC ? 4 : 1;
+	constexpr int kRowStep = VEC ? 16 : 4;
+	const int cl = VEC ? 4 * (lane & 3) : lane & 15, rl = VEC ? lane >> 2 : lane >> 4;
+	const int col = min(c0 + cl, D - kW);
+	if (wave > 0) {
+		float gv[kLnAhead][kSlots][kW], xv[kLnAhead][kSlots][kW], mv[kLnAhead][kSlots], iv[kLnAhead][kSlots];
+		// a slot's offsets from its chunk's first row; the last chunk's rows past R read the last row
+		const int row0 = (wave - 1) * kLnWaveRows + rl, left = (int)(R - (chunks - 1) * kLnChunk) - 1;
+		unsigned off[kSlots], offl[kSlots];
 #pragma unroll
-			for (int u = 0; u < 4; ++u) {
-				gv[slot][u] = g4[u];
-				xv[slot][u] = x4[u];
-				mv[slot][u] = m;
-				iv[slot][u] = iv0;
-			}
-			return;
+		for (int u = 0; u < kSlots; ++u) {
+			off[u] = (unsigned)(row0 + kRowStep * u) * (unsigned)D + (unsigned)col;
+			offl[u] = (unsigned)min(row0 + kRowStep * u, left) * (unsigned)D + (unsigned)col;
 		}
+		auto load = [&](int64_t ch, int slot) {
+			const float* gp = d.g + ch * kLnChunk * D;
+			const float* xp = d.x + ch * kLnChunk * D;
+			const float* mp = d.mean + ch * kLnChunk;
+			const float* ip = d.inv + ch * kLnChunk;
+			const bool last = ch == chunks - 1;
 #pragma unroll
-		for (int u = 0; u < kLnPer; ++u) {
-			const int64_t r = min(ch * kLnChunk + rr + kLnRowStride * u, R - 1);
-			gv[slot][u] = g[r * D + col];
-			xv[slot][u] = x[r * D + col];
-			mv[slot][u] = mean[r];
-			iv[slot][u] = inv[r];
-		}
-	};
-	// the consumer's chain over n rows of buffer b: batches of eight rows in a ring of four, three batches' LDS reads
-	// in flight while one batch's eight dependent adds run
-	auto chain = [&](float& acc, int b, int n) {
-		const float* v = &buf[b][0][tid];
-		if (n == kLnChunk) {
-			constexpr int kB = kLnChunk / 8;
-			float t[4][8];
+			for (int u = 0; u < kSlots; ++u) {
+				const unsigned o = last ? offl[u] : off[u];
+				const unsigned r = last ? (unsigned)min(row0 + kRowStep * u, left) : (unsigned)(row0 + kRowStep * u);
+				if constexpr (VEC) {
+					const f32x4 g4 = *reinterpret_cast<const f32x4*>(gp + o);
+					const f32x4 x4 = *reinterpret_cast<const f32x4*>(xp + o);
 #pragma unroll
-			for (int q = 0; q < 3; ++q)
-#pragma unroll
-				for (int u = 0; u < 8; ++u) t[q][u] = v[(8 * q + u) * 2 * kLnCols];
-#pragma unroll
-			for (int q = 0; q < kB; ++q) {
-				if (q + 3 < kB) {
-#pragma unroll
-					for (int u = 0; u < 8; ++u) t[(q + 3) & 3][u] = v[(8 * (q + 3) + u) * 2 * kLnCols];
-				}
-#pragma unroll
-				for (int u = 0; u < 8; ++u) acc = acc + t[q & 3][u];
-			}
-		} else {
-			for (int i = 0; i < n; ++i) acc = acc + v[i * 2 * kLnCols];
-		}
-	};
-	static_assert(kLnChunk % 8 == 0 && kLnChunk >= 24, "the chain reads batches of eight rows, three ahead");
-	if (producer) {
-#pragma unroll
-		for (int k = 0; k < kLnAhead; ++k)
-			if (k < chunks) load(k, k);
-	}
-	float acc = 0.0f;
-	for (int64_t base = 0; base < chunks; base += kLnAhead) {
-#pragma unroll
-		for (int k = 0; k < kLnAhead; ++k) {
-			const int64_t ch = base + k;
-			if (ch >= chunks) break;
-			const int b = (int)(ch & 1);
-			if (producer) {
-				if (VEC) {
-					// columns past D read a clamped address: their values are never used
-					f32x4 pr, gg;
-#pragma unroll
-					for (int u = 0; u < 4; ++u) {
-						pr[u] = gv[k][u] * ((xv[k][u] - mv[k][u]) * iv[k][u]);
-						gg[u] = gv[k][u];
+					for (int i = 0; i < 4; ++i) {
+						gv[slot][u][i] = g4[i];
+						xv[slot][u][i] = x4[i];
 					}
-					*reinterpret_cast<f32x4*>(&buf[b][vr][4 * q4]) = pr;
-					*reinterpret_cast<f32x4*>(&buf[b][vr][kLnCols + 4 * q4]) = gg;
 				} else {
-#pragma unroll
-					for (int u = 0; u < kLnPer; ++u) {
-						const int row = rr + kLnRowStride * u;
-						buf[b][row][c] = gv[k][u] * ((xv[k][u] - mv[k][u]) * iv[k][u]);
-						buf[b][row][kLnCols + c] = gv[k][u];
-					}
+					gv[slot][u][0] = gp[o];
+					xv[slot][u][0] = xp[o];
 				}
-				if (ch + kLnAhead < chunks) load(ch + kLnAhead, k);
-			} else if (consumer && ch > 0) {
-				chain(acc, b ^ 1, kLnChunk);  // chunk ch - 1 is whole
+				mv[slot][u] = mp[r];
+				iv[slot][u] = ip[r];
+			}
+		};
+#pragma unroll
+		for (int k = 0; k < kLnAhead; ++k) load(min((int64_t)k, chunks - 1), k);
+		auto step = [&](int64_t ch, int k) {
+			float* pr = lds + (ch & 1) * kLnColBuf;
+			float* gg = pr + kLnCols * kLnColPitch;
+#pragma unroll
+			for (int u = 0; u < kSlots; ++u) {
+				const int row = (wave - 1) * kLnWaveRows + kRowStep * u + rl;
+#pragma unroll
+				for (int i = 0; i < kW; ++i) {
+					pr[(cl + i) * kLnColPitch + row] = gv[k][u][i] * ((xv[k][u][i] - mv[k][u]) * iv[k][u]);
+					gg[(cl + i) * kLnColPitch + row] = gv[k][u][i];
+				}
+			}
+			load(min(ch + kLnAhead, chunks - 1), k);
+			__syncthreads();
+		};
+		// whole rounds without a branch, so that the compiler waits for each slot's loads by count, then the rest
+		int64_t ch = 0;
+		for (; ch + kLnAhead <= chunks; ch += kLnAhead) {
+#pragma unroll
+			for (int k = 0; k < kLnAhead; ++k) step(ch + k, k);
+		}
+#pragma unroll
+		for (int k = 0; k < kLnAhead - 1; ++k)
+			if (ch + k < chunks) step(ch + k, k);
+		return;
+	}
+	// wave 0: at barrier ch chunk ch is whole; it is added before the producers, two barriers on, reuse its buffer
+	float acc = 0.0f;
+	const float* mine = lds + (lane & 31) * kLnColPitch;
+	__syncthreads();
+	for (int64_t ch = 0; ch < chunks; ++ch) {
+		const float* v = mine + (ch & 1) * kLnColBuf;
+		if (ch + 1 < chunks) {
+			const f32x4* q = reinterpret_cast<const f32x4*>(v);
+			constexpr int kB = kLnChunk / 16;
+			f32x4 t[3][4];
+#pragma unroll
+			for (int b = 0; b < 2; ++b)
+#pragma unroll
+				for (int e = 0; e < 4; ++e) t[b][e] = q[4 * b + e];
+#pragma unroll
+			for (int b = 0; b < kB; ++b) {
+				if (b + 2 < kB) {
+#pragma unroll
+					for (int e = 0; e < 4; ++e) t[(b + 2) % 3][e] = q[4 * (b + 2) + e];
+				}
+				__builtin_amdgcn_sched_barrier(0);  // keeps the reads ahead of the adds they run beside
+#pragma unroll
+				for (int e = 0; e < 4; ++e)
+#pragma unroll
+					for (int i = 0; i < 4; ++i) acc = acc + t[b % 3][e][i];
 			}
 			__syncthreads();
-		}
-	}
-	if (consumer && chunks > 0) {
-		const int64_t last = chunks - 1;
-		chain(acc, (int)(last & 1), (int)(R - last * kLnChunk));
-	}
-	if (consumer && c0 + (tid % kLnCols) < D) {
-		const int j = c0 + tid % kLnCols;
-		if (tid < kLnCols) {
-			if (dgamma) dgamma[j] = dg_first ? 0.0f + acc : dgamma[j] + acc;
 		} else {
-			if (dbeta) dbeta[j] = db_first ? 0.0f + acc : dbeta[j] + acc;
+			acc = lds_chain(v, (int)(R - ch * kLnChunk), acc);
 		}
+	}
+	const int j = c0 + (lane & 15);
+	if (lane >= 32 || j >= D) return;
+	if (lane < 16) {
+		if (d.dgamma) d.dgamma[j] = d.dg_first ? 0.0f + acc : d.dgamma[j] + acc;
+	} else {
+		if (d.dbeta) d.dbeta[j] = d.db_first ? 0.0f + acc : d.dbeta[j] + acc;
 	}
 }
 
@@ -907,26 +922,13 @@ constexpr int kLnMergedCols = 1;    // columns of a 256-thread workgroup beside 
 constexpr int kLnSmallPitch = kLnSmallRows + 4;  // a column's rows, padded against bank conflicts of the stores
 constexpr size_t kLnMergedLds = 2 * kLnMergedCols * kLnSmallPitch * sizeof(float);
 
-struct LnSmallArgs {
-	const float* g;
-	const float* x;
-	const float* mean;
-	const float* inv;
-	int R, D;
-	float* dgamma;
-	int dg_first;
-	float* dbeta;
-	int db_first;
-	int blocks;  // workgroups of the column chains
-};
-
 // block: the workgroup's index among the chains' workgroups; THREADS its size, COLS its columns; buf:
 // 2 COLS kLnSmallPitch floats of LDS.
 template <int THREADS, int COLS>
-__device__ __forceinline__ void ln_dgamma_small_body(const LnSmallArgs& d, int block, float* buf) {
+__device__ __forceinline__ void ln_dgamma_small_body(const LnColArgs& d, int block, float* buf) {
 	constexpr int kRowStep = THREADS / COLS;
 	constexpr int kPer = kLnSmallRows / kRowStep;
-	const int R = d.R, D = d.D;
+	const int R = (int)d.R, D = d.D;
 	const int tid = threadIdx.x;
 	const int c = tid % COLS, r0 = tid / COLS;  // rows r0 + kRowStep u
 	const int c0 = block * COLS;
@@ -988,17 +990,67 @@ __device__ __forceinline__ void ln_dgamma_small_body(const LnSmallArgs& d, int b
 	}
 }
 
-__global__ void __launch_bounds__(kLnSmallThreads) ln_dgamma_small_kernel(const LnSmallArgs d) {
+__global__ void __launch_bounds__(kLnSmallThreads) ln_dgamma_small_kernel(const LnColArgs d) {
 	__shared__ __align__(16) float buf[2 * kLnSmallCols * kLnSmallPitch];
 	ln_dgamma_small_body<kLnSmallThreads, kLnSmallCols>(d, (int)blockIdx.x, buf);
 }
 
-// dx and the column chains of one layernorm backward in one launch (up to 1024 rows): a workgroup per column for
-// the chains, first, so that the longest work starts first, then the dx row blocks beside them on the other CUs.
-__global__ void __launch_bounds__(256) ln_backward_small_kernel(const LnArgs a, const LnSmallArgs d) {
+// One layernorm backward in one launch: the workgroups of the column chains first, since theirs is the longest work,
+// then the dx row blocks beside them on the other CUs. COLS: no chains (0), those of at most 1024 rows, a column a
+// workgroup (1), or of any number of rows, 16 columns a workgroup (2).
+template <int PER, bool VEC, int COLS>
+__global__ void __launch_bounds__(256) ln_backward_rows_kernel(const LnArgs a, const LnColArgs d) {
 	extern __shared__ __align__(16) float lds[];
-	if ((int)blockIdx.x < d.blocks) ln_dgamma_small_body<256, kLnMergedCols>(d, (int)blockIdx.x, lds);
-	else ln_dx_body(a, (int)blockIdx.x - d.blocks, lds);
+	if (COLS != 0 && (int)blockIdx.x < d.blocks) {
+		if constexpr (COLS == 1) ln_dgamma_small_body<256, kLnMergedCols>(d, (int)blockIdx.x, lds);
+		if constexpr (COLS == 2) ln_columns_body<VEC>(d, (int)blockIdx.x, lds);
+		return;
+	}
+	ln_dx_body<PER, VEC>(a, (int)blockIdx.x - d.blocks, lds);
+}
+
+constexpr int kLnMaxPer = 16;
+constexpr int kLnMaxD = 1024 * kLnMaxPer;  // longest row a workgroup holds in registers
+
+using LnForwardFn = void (*)(const LnArgs);
+using LnBackwardFn = void (*)(const LnArgs, const LnColArgs);
+// [PER 16][VEC]
+const LnForwardFn kLnForward[2][2] = {{ln_forward_rows_kernel<8, false>, ln_forward_rows_kernel<8, true>},
+                                      {ln_forward_rows_kernel<16, false>, ln_forward_rows_kernel<16, true>}};
+// [PER 16][VEC][COLS]
+const LnBackwardFn kLnBackward[2][2][3] = {
+    {{ln_backward_rows_kernel<8, false, 0>, ln_backward_rows_kernel<8, false, 1>, ln_backward_rows_kernel<8, false, 2>},
+     {ln_backward_rows_kernel<8, true, 0>, ln_backward_rows_kernel<8, true, 1>, ln_backward_rows_kernel<8, true, 2>}},
+    {{ln_backward_rows_kernel<16, false, 0>, ln_backward_rows_kernel<16, false, 1>, ln_backward_rows_kernel<16, false, 2>},
+     {ln_backward_rows_kernel<16, true, 0>, ln_backward_rows_kernel<16, true, 1>, ln_backward_rows_kernel<16, true, 2>}}};
+
+// Raises the kernels' dynamic LDS limit once per device (a row of kLnMaxD floats and its product: 131 KB).
+hipError_t prepare_ln() {
+	static std::mutex mu;
+	static bool done[64] = {};
+	int dev = 0;
+	hipError_t e = hipGetDevice(&dev);
+	if (e != hipSuccess) return e;
+	if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
+	std::lock_guard<std::mutex> lock(mu);
+	if (done[dev]) return hipSuccess;
+	auto raise = [&](const void* fn) {
+		if (e == hipSuccess) e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+	};
+	for (int p = 0; p < 2; ++p)
+		for (int v = 0; v < 2; ++v) {
+			raise(reinterpret_cast<const void*>(kLnForward[p][v]));
+			for (int c = 0; c < 3; ++c) raise(reinterpret_cast<const void*>(kLnBackward[p][v][c]));
+		}
+	done[dev] = e == hipSuccess;
+	return e;
+}
+
+// Rows per workgroup: as many as its registers and chain lanes hold, but few enough for about `blocks` workgroups, and
+// enough that every thread has an element.
+int ln_rows(int64_t R, int D, int blocks) {
+	const int64_t most = std::max<int64_t>(1, std::min<int64_t>(kLnMaxRows, (D <= 8192 ? 8192 : kLnMaxD) / D));
+	return (int)std::max<int64_t>(1, std::min(std::min(most, R), std::max<int64_t>((R + blocks - 1) / blocks, (255 + D) / D)));
 }
 
 inline bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
@@ -1126,9 +1178,8 @@ hipError_t batchnorm_backward(const float* gy, const float* x, const unsigned ch
 hipError_t layernorm_forward(const float* x, const float* gamma, const float* beta, int64_t R, int D, float fd,
                              float eps, float* y, float* mean, float* inv_std, hipStream_t s) {
 	if (R == 0) return hipSuccess;
-	// as many rows per workgroup as LDS holds, but few enough for about 256 workgroups when the rows are few
-	const int rw = (int)std::min<int64_t>(std::min<int64_t>(std::min(64, kLnLdsFloats / (D + 1)), R), std::max<int64_t>(1, (R + 255) / 256));
-	if (rw >= 1 && R / rw < ((int64_t)1 << 31) && (int64_t)rw * D < ((int64_t)1 << 31)) {
+	const int rw = ln_rows(R, D, 1024);
+	if (D <= kLnMaxD && R / rw < ((int64_t)1 << 31) - 1) {
 		LnArgs a{};
 		a.x = x;
 		a.gm = gamma;
@@ -1141,10 +1192,12 @@ hipError_t layernorm_forward(const float* x, const float* gamma, const float* be
 		a.rw = rw;
 		a.fd = fd;
 		a.eps = eps;
-		a.vec = D % 4 == 0 && aligned16(x) && aligned16(y);
-		a.dq = make_fastdiv((unsigned)(a.vec ? D / 4 : D));
-		hipLaunchKernelGGL(ln_forward_lds_kernel, dim3((unsigned)((R + rw - 1) / rw)), dim3(256),
-		                   (size_t)rw * (D + 1) * sizeof(float), s, a);
+		const bool vec = D % 4 == 0 && aligned16(x) && aligned16(y);
+		a.dq = make_fastdiv((unsigned)(vec ? D / 4 : D));
+		const hipError_t e = prepare_ln();
+		if (e != hipSuccess) return e;
+		hipLaunchKernelGGL(kLnForward[D > 8192 ? 1 : 0][vec ? 1 : 0], dim3((unsigned)((R + rw - 1) / rw)), dim3(256),
+		                   (size_t)rw * (ln_pitch(D) + 2) * sizeof(float), s, a);
 		return hipGetLastError();
 	}
 	const int vec = D % 4 == 0 && aligned16(x) && aligned16(y) && aligned16(gamma) && aligned16(beta);
@@ -1157,10 +1210,9 @@ hipError_t layernorm_backward(const float* gy, const float* x, const float* gamm
                               const float* inv_std, int64_t R, int D, float fd, float* dx, int dx_first,
                               float* dgamma, int dgamma_first, float* dbeta, int dbeta_first, hipStream_t s) {
 	if (R == 0 && !dgamma && !dbeta) return hipSuccess;
-	const int rw = (int)std::min<int64_t>(std::min<int64_t>(std::min(64, (kLnLdsFloats - D) / (2 * (D + 1) + 4)),
-	                                                        std::max<int64_t>(R, 1)),
-	                                      std::max<int64_t>(1, (R + 255) / 256));
-	if (rw >= 1 && R / rw < ((int64_t)1 << 31) && (int64_t)rw * D < ((int64_t)1 << 31)) {
+	const int rw = ln_rows(std::max<int64_t>(R, 1), D, 512);
+	const bool cols = dgamma || dbeta;
+	if (D <= kLnMaxD && R / rw < ((int64_t)1 << 31) - D && R > 0) {
 		LnArgs a{};
 		a.g = gy;
 		a.x = x;
@@ -1173,33 +1225,23 @@ hipError_t layernorm_backward(const float* gy, const float* x, const float* gamm
 		a.rw = rw;
 		a.fd = fd;
 		a.first = dx_first;
-		a.vec = D % 4 == 0 && aligned16(x) && aligned16(gy) && aligned16(dx);
-		a.dq = make_fastdiv((unsigned)(a.vec ? D / 4 : D));
-		a.dd = make_fastdiv((unsigned)D);
-		const size_t dx_lds = ((size_t)2 * rw * (D + 1) + D + 4 * rw) * sizeof(float);
-		const int64_t dx_blocks = (R + rw - 1) / rw;
-		const bool small = (dgamma || dbeta) && R > 0 && R <= kLnSmallRows;
-		LnSmallArgs d{gy, x, mean, inv_std, (int)R, D, dgamma, dgamma_first, dbeta, dbeta_first,
-		              (D + kLnMergedCols - 1) / kLnMergedCols};
-		if (dx && R > 0 && small && dx_blocks + d.blocks < ((int64_t)1 << 31)) {
-			hipLaunchKernelGGL(ln_backward_small_kernel, dim3((unsigned)(d.blocks + dx_blocks)), dim3(256),
-			                   std::max(dx_lds, kLnMergedLds), s, a, d);
+		const bool vec = D % 4 == 0 && aligned16(x) && aligned16(gy) && (!dx || aligned16(dx));
+		a.dq = make_fastdiv((unsigned)(vec ? D / 4 : D));
+		LnColArgs d{gy, x, mean, inv_std, R, D, dgamma, dgamma_first, dbeta, dbeta_first, 0};
+		const bool small = cols && R <= kLnSmallRows;
+		hipError_t e = prepare_ln();
+		if (e != hipSuccess) return e;
+		if (small && !dx) {
+			d.blocks = (D + kLnSmallCols - 1) / kLnSmallCols;
+			hipLaunchKernelGGL(ln_dgamma_small_kernel, dim3((unsigned)d.blocks), dim3(kLnSmallThreads), 0, s, d);
 			return hipGetLastError();
 		}
-		d.blocks = (D + kLnSmallCols - 1) / kLnSmallCols;
-		if (dx && R > 0) {
-			hipLaunchKernelGGL(ln_dx_lds_kernel, dim3((unsigned)dx_blocks), dim3(256), dx_lds, s, a);
-			const hipError_t e = hipGetLastError();
-			if (e != hipSuccess) return e;
-		}
-		if (small)
-			hipLaunchKernelGGL(ln_dgamma_small_kernel, dim3((unsigned)d.blocks), dim3(kLnSmallThreads), 0, s, d);
-		else if ((dgamma || dbeta) && D % 4 == 0 && aligned16(gy) && aligned16(x))
-			hipLaunchKernelGGL(ln_dgamma_kernel<true>, dim3((unsigned)((D + kLnCols - 1) / kLnCols)), dim3(kLnThreads), 0, s,
-			                   gy, x, mean, inv_std, R, D, dgamma, dgamma_first, dbeta, dbeta_first);
-		else if (dgamma || dbeta)
-			hipLaunchKernelGGL(ln_dgamma_kernel<false>, dim3((unsigned)((D + kLnCols - 1) / kLnCols)), dim3(kLnThreads), 0, s,
-			                   gy, x, mean, inv_std, R, D, dgamma, dgamma_first, dbeta, dbeta_first);
+		if (cols) d.blocks = small ? (D + kLnMergedCols - 1) / kLnMergedCols : (D + kLnCols - 1) / kLnCols;
+		const int64_t blocks = d.blocks + (dx ? (R + rw - 1) / rw : 0);
+		const size_t lds_dx = dx ? (size_t)rw * (2 * ln_pitch(D) + 4) * sizeof(float) : 0;
+		const size_t lds_cols = !cols ? 0 : small ? kLnMergedLds : kLnColLds;
+		hipLaunchKernelGGL(kLnBackward[D > 8192 ? 1 : 0][vec ? 1 : 0][!cols ? 0 : small ? 1 : 2], dim3((unsigned)blocks), dim3(256),
+		                   std::max(lds_dx, lds_cols), s, a, d);
 		return hipGetLastError();
 	}
 	LnBwdArgs a{};
