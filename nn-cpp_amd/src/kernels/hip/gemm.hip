@@ -274,9 +274,9 @@ hipError_t gemm_launch(const GemmCall& g, hipStream_t s, int config, float* work
 	if (config == kNumConfigs + kValuShapes + 2 && chain4_ok(g)) return gemm_chain4_launch(g, s);
 	if (config >= kFirstRing && config < kFirstRing + kRingConfigs && ring_ok(g))
 		return gemm_ring_launch(g, s, config - kFirstRing);
+	if (config < 0 && ring_takes(g)) return gemm_ring_launch(g, s);
 	if (config < 0 && chain4_takes(g)) return gemm_chain4_launch(g, s);
 	if ((config < 0 || config >= kNumConfigs) && valu_ok && valu_takes(g)) return gemm_valu_launch(g, valu_shape(g), s);
-	if (config < 0 && ring_takes(g)) return gemm_ring_launch(g, s);
 	if (config < 0 || config >= kNumConfigs) config = pick_config(g);
 	const Config& cf = configs()[config];
 
@@ -346,7 +346,7 @@ hipError_t gemm_launch_pair(const GemmCall& g0, const GemmCall& g1, hipStream_t 
 	if (g0.batch_count != 1 || g1.batch_count != 1 || g0.batch.ndim != 0 || g1.batch.ndim != 0) return hipSuccess;
 	if (g0.m == 0 || g0.n == 0 || g1.m == 0 || g1.n == 0) return hipSuccess;
 	if (depth_cut(g0.m, g0.n, g0.k) || depth_cut(g1.m, g1.n, g1.k)) return hipSuccess;
-	if (ring_takes(g0) || ring_takes(g1)) return hipSuccess;
+	if (ring_takes_large(g0) || ring_takes_large(g1)) return hipSuccess;
 	const int c0 = pick_config(g0), c1 = pick_config(g1);
 	if (c0 != c1) return hipSuccess;
 	const Config& cf = configs()[c0];

@@ -96,7 +96,8 @@ hipError_t gemm_pieces4_launch(const GemmCall& g, hipStream_t s);
 // ordered sum) or the GELU epilogue (A B^T) allowed. config < 0 picks the tile by shape.
 constexpr int kRingConfigs = 4;
 bool ring_ok(const GemmCall& g);
-bool ring_takes(const GemmCall& g);  // the shapes it is routed for (measured)
+bool ring_takes(const GemmCall& g);        // the shapes it is routed for (measured)
+bool ring_takes_large(const GemmCall& g);  // those of them that take 64 x 64 tiles or larger
 hipError_t gemm_ring_launch(const GemmCall& g, hipStream_t s, int config = -1);
 const char* ring_config_name(int config);
 // A B on the chain kernel and A^T B (row sums allowed) on the pieces kernel in one launch (gemm_pieces.hip): single

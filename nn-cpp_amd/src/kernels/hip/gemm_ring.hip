@@ -10,11 +10,11 @@ namespace nnh {
 
 namespace {
 
-enum { kRing256x128 = 0, kRing128x128 = 1, kRing64x64 = 2, kRing64x64Deep = 3 };
+enum { kRing256x128 = 0, kRing128x128 = 1, kRing64x64 = 2, kRing32x32 = 3 };
 
 const RingConfig* ring_configs() {
 	static const RingConfig table[kRingConfigs] = {ring_config_256x128(), ring_config_128x128(), ring_config_64x64(),
-	                                               ring_config_64x64_deep()};
+	                                               ring_config_32x32()};
 	return table;
 }
 
@@ -52,21 +52,27 @@ bool ring_vec(const GemmCall& g) {
 	return ok;
 }
 
-// The time of `tiles` workgroups on a chip of 256 CUs, in cycles of a 32-deep step. Measured per step (4096 x 4096 x
-// 2048, every layout within 3%): 256 x 128 8790 cycles (8192 of them MFMAs), 128 x 128 4610 (4096), 64 x 64 2380 for
-// the two workgroups a CU holds (2048) and 1450 for one alone (1024; 64-deep stages 1350). A workgroup's start and
-// end (first loads, stores) cost about as much as 1 to 2 steps of its own.
-double ring_cost(double tiles, double steps, int config) {
+// The time of `tiles` workgroups on a chip of 256 CUs, in cycles, for `steps` 32-deep steps. Measured per step: 256 x 128
+// 8790 cycles (8192 of them MFMAs), 128 x 128 4610 (4096), 64 x 64 2380 for the two workgroups a CU holds (2048) and
+// 1450 for one alone (1024), 32 x 32 830 for two with A transposed and B not (512; 960 for the other layouts, whose
+// k-contiguous rows are a large stride apart and crowd a few L2 channels) and 490 (600) for one alone, whose waves have one
+// dependent MFMA chain each. A workgroup's start and end (first loads, stores) add the constants.
+double ring_cost(const GemmCall& g, double tiles, double steps, int config) {
 	const double rounds = tiles / 256;
+	auto pairs = [&](double two, double one, double ends) {  // two workgroups a CU
+		const double full = std::floor(rounds / 2), rest = std::ceil(rounds - 2 * full);
+		return full * (two * steps + ends) + (rest > 1 ? two * steps + ends : rest > 0 ? one * steps + ends : 0);
+	};
 	switch (config) {
 		case kRing256x128: return std::ceil(rounds) * (8790 * steps + 12000);
 		case kRing128x128: return std::ceil(rounds) * (4610 * steps + 9000);
-		case kRing64x64: {
-			const double pairs = std::floor(rounds / 2), rest = std::ceil(rounds - 2 * pairs);
-			return pairs * (2380 * steps + 6000) + (rest > 1 ? 2380 * steps + 6000 : rest > 0 ? 1450 * steps + 4500 : 0);
-		}
-		default: return std::ceil(rounds) * (1350 * steps + 4500);
+		case kRing64x64: return pairs(2380, 1450, 5000);
+		default: return g.ta && !g.tb ? pairs(830, 490, 4500) : pairs(960, 600, 4500);
 	}
+}
+
+bool narrow(const GemmCall& g) {
+	return g.m >= 128 && g.n < 128 && (double)g.m * (double)g.n * (double)g.batch_count >= 512.0 * 128 * 64;
 }
 
 int ring_pick(const GemmCall& g) {
@@ -78,7 +84,7 @@ int ring_pick(const GemmCall& g) {
 		if (i == kRing256x128 && !ring_vec(g)) continue;
 		const RingConfig& c = ring_configs()[i];
 		const double tiles = (double)((g.m + c.bm - 1) / c.bm) * (double)((g.n + c.bn - 1) / c.bn) * (double)g.batch_count;
-		const double t = ring_cost(tiles, steps, i);
+		const double t = ring_cost(g, tiles, steps, i);
 		if (i == 0 || cost == 0 || t < cost) {
 			cost = t;
 			best = i;
@@ -96,17 +102,32 @@ bool ring_ok(const GemmCall& g) {
 	return !g.rowsum || (g.ta && !g.tb && g.rowsum_outer == 0 && g.batch_count == 1 && g.batch.ndim == 0);
 }
 
-bool ring_takes(const GemmCall& g) {
-	// Products with a 64 x 64 tile for at least half the CUs and a depth of a few stages. Measured against the tile
-	// kernels (us): 4096^3 NN 1106 -> 995, 2048^3 157 -> 137, 1024^3 28.8 -> 23.4, 8192 x 512 x 2048 NT 152 -> 136,
-	// 2048 x 512 x 8192 TN 205 -> 157, 1021 x 771 x 1533 NN (one float a lane) 79 -> 42, 300 x 3000 x 500 24 -> 15.
-	// With fewer tiles the 32 x 32 tiles' shorter chains win (768^3, 144 tiles: 16.7 us against 18.4), and products
-	// narrower than 128 with 2^22 outputs or more (attention's 256 x 64 per head) keep their 128 x 64 tiles (256 of
-	// them, 256 deep: 26 to 31 us against 29 to 33).
+bool ring_takes_large(const GemmCall& g) {
+	// Products with a 64 x 64 tile for two thirds of the CUs or more, and a depth of a few stages. Measured against the
+	// tile kernels (us): 4096^3 NN 1106 -> 974, 2048^3 157 -> 137, 1024^3 28.8 -> 23.9, 8192 x 512 x 2048 NT 152 -> 136,
+	// 2048 x 512 x 8192 TN 205 -> 150, 1021 x 771 x 1533 NN (one float a lane) 79 -> 39, 300 x 3000 x 500 24 -> 14.
+	// With fewer tiles the tile kernels' three 32 x 32 workgroups a CU win (768^3, 144 tiles: 16.7 us against 18.4), and
+	// products narrower than 128 with 2^22 outputs or more (attention's 256 x 64 per head) keep their 128 x 64 tiles
+	// (256 of them, 256 deep: 26 to 31 us against 29 to 33).
 	if (!ring_ok(g) || g.k < 96) return false;
-	if (g.m >= 128 && g.n < 128 && (double)g.m * (double)g.n * (double)g.batch_count >= 512.0 * 128 * 64) return false;
+	if (narrow(g)) return false;
 	const double tiles = (double)((g.m + 63) / 64) * (double)((g.n + 63) / 64) * (double)g.batch_count;
 	return tiles >= 176;
+}
+
+bool ring_takes(const GemmCall& g) {
+	if (ring_takes_large(g)) return true;
+	// Smaller products, where the 32 x 32 tile's chains are the time. A^T B (a weight gradient) is faster here at every
+	// size: 512 x 512 x 8192 67 -> 52 us, 1024 x 512 x 4096 66 -> 46, 512 x 784 x 256 7.7 -> 5.9 (chain kernel), 256 x 256 x
+	// 300 7.0 -> 5.4 (VALU kernel). The other layouts where the tile kernel would check bounds (200 x 2000 x 1000 23 -> 17,
+	// 300 x 1000 x 512 NT 13.5 -> 10.4), and A B with a tile a CU at most (64 x 4096 x 4096 33.8 -> 32.4, 256 x 784 x 512 9.6 ->
+	// 7.1); whole aligned A B^T tiles stay where they are (512^3 7.3 us against 8.0, 64 x 4096 x 4096 33.6 against 38).
+	if (!ring_ok(g) || g.k < 128 || narrow(g)) return false;
+	const double tiles = (double)((g.m + 31) / 32) * (double)((g.n + 31) / 32) * (double)g.batch_count;
+	if (tiles < 64) return false;
+	if (g.ta && !g.tb) return true;
+	const bool whole = ring_vec(g) && g.m % 32 == 0 && g.n % 32 == 0 && g.k % 64 == 0 && g.ldc % 4 == 0 && aligned16(g.c);
+	return !whole || (!g.ta && !g.tb && tiles <= 256);
 }
 
 hipError_t gemm_ring_launch(const GemmCall& g, hipStream_t s, int config) {

@@ -32,21 +32,27 @@
 
 namespace nnh {
 
-template <int BM, int BN, int BK, int WM, int WN, int ST, int V>
+template <int BM, int BN, int BK, int WM, int WN, int ST, bool TA, bool TB, int V>
 struct RingShape {
 	static constexpr int kWavesN = BN / WN;
 	static constexpr int kWaves = (BM / WM) * (BN / WN);
 	static constexpr int kThreads = 64 * kWaves;
 	static constexpr int I = WM / 16, J = WN / 16;
 	static constexpr int kA = BM * BK, kB = BN * BK, kStage = kA + kB;
-	static constexpr int kPerLoad = 64 * V;  // floats one wave's load instruction moves
-	static constexpr int LA = kA / (kPerLoad * kWaves), LB = kB / (kPerLoad * kWaves);
+	// k-contiguous operands stored in fragment order (ring::kc_index), where one float a lane is loaded anyway. Loading
+	// single floats for its sake cost more than its quarter of the reads gave (512^3 A B on 32 x 32 tiles 7.1 -> 7.7 us).
+	static constexpr bool kFrag = V == 1;
+	static constexpr int VA = !TA && kFrag ? 1 : V, VB = TB && kFrag ? 1 : V;  // floats a lane loads
+	static constexpr int kPerA = 64 * VA, kPerB = 64 * VB;                     // floats a load instruction moves
+	static constexpr int LA = kA / (kPerA * kWaves), LB = kB / (kPerB * kWaves);
 	static constexpr int L = LA + LB;        // load instructions of a wave per stage
 	static constexpr int kLdsBytes = ST * kStage * 4;
-	static_assert(LA * kPerLoad * kWaves == kA && LB * kPerLoad * kWaves == kB, "a stage splits evenly over the waves");
+	static_assert(LA * kPerA * kWaves == kA && LB * kPerB * kWaves == kB, "a stage splits evenly over the waves");
 	static_assert(WM % 16 == 0 && WN % 16 == 0 && BM % WM == 0 && BN % WN == 0, "whole 16 x 16 blocks");
 	static_assert(BK % 32 == 0 && kAccAfter % BK == 0, "an even number of 16-deep groups; 256 on a stage boundary");
-	static_assert(ST >= 3 && ST <= 8 && (ST - 3) * L <= 63, "a wave can count at most 63 outstanding loads; the tail is written out for 8 stages");
+	static_assert(ST >= 3 && ST <= 8, "the tail is written out for 8 stages");
+	// the wait that leaves `stages` whole stages outstanding (a wave counts at most 63 loads: then it waits for more)
+	static constexpr int waits(int stages) { return stages * L < 63 ? stages * L : 63; }
 	static_assert(kLdsBytes <= 160 * 1024, "gfx950 has 160 KiB of LDS per CU");
 };
 
@@ -72,20 +78,29 @@ __device__ __forceinline__ int swz(int row) {
 // The same for an m/n-contiguous tile of R rows: the offset XORed onto the row index at depth k (a multiple of 16).
 template <int R>
 __device__ __forceinline__ int kswz(int k) {
-	return R >= 64 ? 16 * (k & 3) : 16 * ((k >> 1) & 1);
+	return R >= 64 ? 16 * (k & 3) : R == 32 ? 16 * ((k >> 1) & 1) : 0;
+}
+
+// Where row `row`, depth k of a k-contiguous tile lives. FRAG (fragment order): every 16 depths are stored lane group
+// by lane group, depth 4 t + g at position 4 g + t, so that a lane's operands of four MFMAs are one 16-byte read.
+template <int BK, bool FRAG>
+__device__ __forceinline__ int kc_index(int row, int k) {
+	const int c = FRAG ? (k / 16) * 4 + k % 4 : k / 4, e = FRAG ? (k / 4) % 4 : k % 4;
+	return row * BK + 4 * (c ^ swz<BK>(row)) + e;
 }
 
 // Float offset, from the tile's first element, of what lane `lane` loads with the load instruction that fills LDS
-// floats [64 V q, 64 V (q + 1)) of the tile. KC: k-contiguous (rows of BK), else depth rows of R. rows: valid rows of
-// the tile (>= 1; with V = 4 and !KC a multiple of 4), depth: valid depth of the stage (>= 1; with V = 4 and KC a
-// multiple of 4).
-template <bool KC, int R, int BK, int V>
+// floats [64 V q, 64 V (q + 1)) of the tile. KC: k-contiguous (rows of BK, FRAG as above), else depth rows of R. rows:
+// valid rows of the tile (>= 1; with V = 4 and !KC a multiple of 4), depth: valid depth of the stage (>= 1; with V = 4
+// and KC a multiple of 4).
+template <bool KC, bool FRAG, int R, int BK, int V>
 __device__ __forceinline__ unsigned src_offset(int q, int lane, int64_t ld, int rows, int depth) {
+	static_assert(V == 1 || !KC || !FRAG, "fragment order moves single floats");
 	const int pos = (q * 64 + lane) * V;
 	if (KC) {
 		const int row = pos / BK, e = pos % BK;
 		const int c = (e / 4) ^ swz<BK>(row);
-		const int k = 4 * c + (V == 1 ? e % 4 : 0);
+		const int k = FRAG ? 16 * (c / 4) + 4 * (e % 4) + c % 4 : 4 * c + (V == 1 ? e % 4 : 0);
 		return (unsigned)min(row, rows - 1) * (unsigned)ld + (unsigned)min(k, depth - V);
 	}
 	const int k = pos / R, e = pos % R;
@@ -100,7 +115,7 @@ enum RingExtra : int { kRingPlain = 0, kRingRowSums = 1, kRingGelu = 2 };
 
 template <int BM, int BN, int BK, int WM, int WN, int ST, bool TA, bool TB, int V, int EXTRA>
 __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
-	using S = RingShape<BM, BN, BK, WM, WN, ST, V>;
+	using S = RingShape<BM, BN, BK, WM, WN, ST, TA, TB, V>;
 	constexpr int I = S::I, J = S::J, NG = BK / 16;
 	constexpr bool RS = EXTRA == kRingRowSums;
 	static_assert(!RS || (TA && !TB && BM <= S::kThreads), "row sums: the weight-gradient layout, one thread a row");
@@ -133,22 +148,26 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 	unsigned offa[S::LA], offb[S::LB];
 #pragma unroll
 	for (int q = 0; q < S::LA; ++q)
-		offa[q] = ring::src_offset<!TA, BM, BK, V>(wave * S::LA + q, lane, p.lda, rows_a, BK);
+		offa[q] = ring::src_offset<!TA, S::kFrag, BM, BK, S::VA>(wave * S::LA + q, lane, p.lda, rows_a, BK);
 #pragma unroll
 	for (int q = 0; q < S::LB; ++q)
-		offb[q] = ring::src_offset<TB, BN, BK, V>(wave * S::LB + q, lane, p.ldb, rows_b, BK);
+		offb[q] = ring::src_offset<TB, S::kFrag, BN, BK, S::VB>(wave * S::LB + q, lane, p.ldb, rows_b, BK);
 
-	auto dma = [&](const float* src, unsigned off, float* dst) {
-		if constexpr (V == 4) __builtin_amdgcn_global_load_lds((ring::global_void*)(src + off), (ring::lds_void*)dst, 16, 0, 0);
-		else __builtin_amdgcn_global_load_lds((ring::global_void*)(src + off), (ring::lds_void*)dst, 4, 0, 0);
+	auto dma = [&](auto width, const float* src, unsigned off, float* dst) {
+		if constexpr (decltype(width)::value == 4)
+			__builtin_amdgcn_global_load_lds((ring::global_void*)(src + off), (ring::lds_void*)dst, 16, 0, 0);
+		else
+			__builtin_amdgcn_global_load_lds((ring::global_void*)(src + off), (ring::lds_void*)dst, 4, 0, 0);
 	};
+	constexpr std::integral_constant<int, S::VA> va{};
+	constexpr std::integral_constant<int, S::VB> vb{};
 	// The wave's load instruction q (0 .. L - 1) of the next stage, whole, into ring slot `slot`; advance() follows the
 	// last. Stages are issued in order.
 	auto issue_one = [&](int q, int slot) {
-		float* As = lds + slot * S::kStage + wave * S::LA * S::kPerLoad;
-		float* Bs = lds + slot * S::kStage + S::kA + wave * S::LB * S::kPerLoad;
-		if (q < S::LA) dma(a_next, offa[q < S::LA ? q : 0], As + q * S::kPerLoad);
-		else dma(b_next, offb[q >= S::LA ? q - S::LA : 0], Bs + (q - S::LA) * S::kPerLoad);
+		float* As = lds + slot * S::kStage + wave * S::LA * S::kPerA;
+		float* Bs = lds + slot * S::kStage + S::kA + wave * S::LB * S::kPerB;
+		if (q < S::LA) dma(va, a_next, offa[q < S::LA ? q : 0], As + q * S::kPerA);
+		else dma(vb, b_next, offb[q >= S::LA ? q - S::LA : 0], Bs + (q - S::LA) * S::kPerB);
 	};
 	auto advance = [&]() {
 		a_next += a_step;
@@ -157,14 +176,16 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 	// All of stage kt at once; a partial last stage loads nothing past the depth.
 	auto issue = [&](int kt, int slot) {
 		if (krem != BK && kt == nkt - 1) {
-			float* As = lds + slot * S::kStage + wave * S::LA * S::kPerLoad;
-			float* Bs = lds + slot * S::kStage + S::kA + wave * S::LB * S::kPerLoad;
+			float* As = lds + slot * S::kStage + wave * S::LA * S::kPerA;
+			float* Bs = lds + slot * S::kStage + S::kA + wave * S::LB * S::kPerB;
 #pragma unroll
 			for (int q = 0; q < S::LA; ++q)
-				dma(a_next, ring::src_offset<!TA, BM, BK, V>(wave * S::LA + q, lane, p.lda, rows_a, krem), As + q * S::kPerLoad);
+				dma(va, a_next, ring::src_offset<!TA, S::kFrag, BM, BK, S::VA>(wave * S::LA + q, lane, p.lda, rows_a, krem),
+				    As + q * S::kPerA);
 #pragma unroll
 			for (int q = 0; q < S::LB; ++q)
-				dma(b_next, ring::src_offset<TB, BN, BK, V>(wave * S::LB + q, lane, p.ldb, rows_b, krem), Bs + q * S::kPerLoad);
+				dma(vb, b_next, ring::src_offset<TB, S::kFrag, BN, BK, S::VB>(wave * S::LB + q, lane, p.ldb, rows_b, krem),
+				    Bs + q * S::kPerB);
 			return;
 		}
 #pragma unroll
@@ -178,32 +199,39 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 		float* Bs = As + S::kA;
 		for (int e = tid; e < BM * (BK - krem); e += S::kThreads) {
 			const int r = e % BM, k = krem + e / BM;
-			As[TA ? k * BM + (r ^ ring::kswz<BM>(k)) : r * BK + 4 * ((k / 4) ^ ring::swz<BK>(r)) + k % 4] = 0.0f;
+			As[TA ? k * BM + (r ^ ring::kswz<BM>(k)) : ring::kc_index<BK, S::kFrag>(r, k)] = 0.0f;
 		}
 		for (int e = tid; e < BN * (BK - krem); e += S::kThreads) {
 			const int r = e % BN, k = krem + e / BN;
-			Bs[TB ? r * BK + 4 * ((k / 4) ^ ring::swz<BK>(r)) + k % 4 : k * BN + (r ^ ring::kswz<BN>(k))] = -0.0f;
+			Bs[TB ? ring::kc_index<BK, S::kFrag>(r, k) : k * BN + (r ^ ring::kswz<BN>(k))] = -0.0f;
 		}
 		ring::wait_and_meet<63>();
 	};
 
 	// ---- fragments: element t of lane (g, lr) is depth kk + 4 t + g of row (column) lr of a 16-wide block ----
-	int koff = lr * BK + 4 * ring::swz<BK>(lr) + g;  // k-contiguous: chunk c is at koff ^ 4 c
+	// k-contiguous: chunk c is at koff ^ 4 c (fragment order: the lane's chunk of the 16 depths from kk is c = kk / 4 + g)
+	const int koff = lr * BK + 4 * ring::swz<BK>(lr) + (S::kFrag ? 0 : g);
 	int moffa[I], moffb[J];
 #pragma unroll
 	for (int i = 0; i < I; ++i) moffa[i] = g * BM + ((wm0 + 16 * i) ^ ring::kswz<BM>(g)) + lr;
 #pragma unroll
 	for (int j = 0; j < J; ++j) moffb[j] = g * BN + ((wn0 + 16 * j) ^ ring::kswz<BN>(g)) + lr;
-	// element t of the group of 16 depths from kk
+	// element t of the group of 16 depths from kk (fragment order: all four elements of every fourth block instead)
 	auto read_frags = [&](int slot, int kk, int t, f32x4* af, f32x4* bf) {
 		const float* As = lds + slot * S::kStage;
 		const float* Bs = As + S::kA;
 #pragma unroll
-		for (int i = 0; i < I; ++i)
-			af[i][t] = TA ? As[(kk + 4 * t) * BM + moffa[i]] : As[(wm0 + 16 * i) * BK + (koff ^ (kk + 4 * t))];
+		for (int i = 0; i < I; ++i) {
+			if (TA) af[i][t] = As[(kk + 4 * t) * BM + moffa[i]];
+			else if (!S::kFrag) af[i][t] = As[(wm0 + 16 * i) * BK + (koff ^ (kk + 4 * t))];
+			else if (i % 4 == t) af[i] = *reinterpret_cast<const f32x4*>(As + (wm0 + 16 * i) * BK + (koff ^ (kk + 4 * g)));
+		}
 #pragma unroll
-		for (int j = 0; j < J; ++j)
-			bf[j][t] = TB ? Bs[(wn0 + 16 * j) * BK + (koff ^ (kk + 4 * t))] : Bs[(kk + 4 * t) * BN + moffb[j]];
+		for (int j = 0; j < J; ++j) {
+			if (!TB) bf[j][t] = Bs[(kk + 4 * t) * BN + moffb[j]];
+			else if (!S::kFrag) bf[j][t] = Bs[(wn0 + 16 * j) * BK + (koff ^ (kk + 4 * t))];
+			else if (j % 4 == t) bf[j] = *reinterpret_cast<const f32x4*>(Bs + (wn0 + 16 * j) * BK + (koff ^ (kk + 4 * g)));
+		}
 	};
 
 	f32x4 acc[I][J];
@@ -239,8 +267,15 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 					for (int q = 0; q < S::L; ++q)
 						if (q * kSteps / S::L == step) issue_one(q, fill);
 				}
-				if (gi + 1 < NG) read_frags(slot, 16 * (gi + 1), t, af[cur ^ 1], bf[cur ^ 1]);
-				else if (decltype(has_next)::value) read_frags(after, 0, t, af[cur ^ 1], bf[cur ^ 1]);
+				// one chain a wave: the whole group's reads ahead of its first MFMA, so that the last of them does not
+				// meet the barrier half done
+				constexpr bool kBurst = I * J == 1;
+#pragma unroll
+				for (int tt = 0; tt < 4; ++tt) {
+					if (kBurst ? t != 0 : tt != t) continue;
+					if (gi + 1 < NG) read_frags(slot, 16 * (gi + 1), tt, af[cur ^ 1], bf[cur ^ 1]);
+					else if (decltype(has_next)::value) read_frags(after, 0, tt, af[cur ^ 1], bf[cur ^ 1]);
+				}
 #pragma unroll
 				for (int i = 0; i < I; ++i)
 #pragma unroll
@@ -280,7 +315,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 		int fill = 0, slot = 0;  // the slots the next issued and the next computed stage take
 		const int first = min(ST - 1, nkt);
 		for (; fill < first; ++fill) issue(fill, fill);
-		if (first == ST - 1) ring::wait_and_meet<((ST - 2) * S::L < 63 ? (ST - 2) * S::L : 63)>();
+		if (first == ST - 1) ring::wait_and_meet<S::waits(ST - 2)>();
 		else ring::wait_and_meet<0>();
 		ready(0, 0);
 #pragma unroll
@@ -290,7 +325,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 		auto run = [&](int end) {
 			for (; kt < end; ++kt) {
 				const int after = next(slot);
-				ring::wait_and_meet<(ST - 3) * S::L>();
+				ring::wait_and_meet<S::waits(ST - 3)>();
 				compute(slot, after, std::true_type{}, std::true_type{}, fill);
 				fill = next(fill);
 				slot = after;
@@ -311,7 +346,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 		run(last_whole);
 		if (kt < last_issue) {  // the partial stage's loads
 			const int after = next(slot);
-			ring::wait_and_meet<(ST - 3) * S::L>();
+			ring::wait_and_meet<S::waits(ST - 3)>();
 			issue(kt + ST - 1, fill);
 			compute(slot, after, std::true_type{}, std::false_type{}, 0);
 			slot = after;
@@ -322,7 +357,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 			constexpr int r = decltype(beyond)::value;
 			if (kt + 2 + r != nkt) return;
 			const int after = next(slot);
-			ring::wait_and_meet<r * S::L>();
+			ring::wait_and_meet<S::waits(r)>();
 			ready(kt + 1, after);
 			compute(slot, after, std::true_type{}, std::false_type{}, 0);
 			slot = after;
@@ -426,7 +461,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 }
 
 template <int BM, int BN, int BK, int WM, int WN, int ST, int WPE, bool TA, bool TB, int V, int EXTRA>
-__global__ void __launch_bounds__((RingShape<BM, BN, BK, WM, WN, ST, V>::kThreads))
+__global__ void __launch_bounds__((RingShape<BM, BN, BK, WM, WN, ST, TA, TB, V>::kThreads))
 __attribute__((amdgpu_waves_per_eu(WPE, WPE))) sgemm_ring_kernel(const GemmArgs p) {
 	ring_tile<BM, BN, BK, WM, WN, ST, TA, TB, V, EXTRA>(p, (int)blockIdx.x);
 }
@@ -442,7 +477,7 @@ struct RingConfig {
 
 template <int BM, int BN, int BK, int WM, int WN, int ST, int WPE>
 RingConfig make_ring_config(const char* name) {
-	using S = RingShape<BM, BN, BK, WM, WN, ST, 4>;
+	using S = RingShape<BM, BN, BK, WM, WN, ST, false, false, 4>;  // threads and LDS are the same for every layout
 	RingConfig c{};
 	c.name = name;
 	c.bm = BM;
@@ -469,6 +504,6 @@ RingConfig make_ring_config(const char* name) {
 RingConfig ring_config_256x128();
 RingConfig ring_config_128x128();
 RingConfig ring_config_64x64();
-RingConfig ring_config_64x64_deep();
+RingConfig ring_config_32x32();
 
 }  // namespace nnh
