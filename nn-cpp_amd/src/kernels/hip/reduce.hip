@@ -276,6 +276,60 @@ __global__ void __launch_bounds__(256) sum_rows2_kernel(const float* __restrict_
 	else dst[j] = dst[j] + s;
 }
 
+// The same two sums for 16-byte aligned rows of whole quads: a workgroup owns four columns, so a {32, 256, 512} gradient
+// gets 128 workgroups instead of 32. Thread b runs the four first sums of axis-1 index b (and b + 256, ...) from one
+// 16-byte load per axis-0 index, sixteen in flight; the second sums then read LDS four indices at a time. Neighbouring
+// workgroups share the rows' cache lines, so the block order gives each XCD a contiguous range of columns. Measured at
+// [32, 256, 512] 13.4 -> 8.6 us with the gradient in the caches, [32, 256, 2048] 26.9 -> 22.2 (bound by one CU's 16-byte accesses, 64 lines a load instruction).
+constexpr int kQ2Steps = 16, kQ2Pitch = kSum2MaxR1 + 4;
+
+__global__ void __launch_bounds__(256) sum_rows2_quad_kernel(const float* __restrict__ src, int r0, int r1, int inner,
+                                                             float* __restrict__ dst, int combine) {
+	__shared__ __align__(16) float part[4 * kQ2Pitch];
+	const int per = (int)gridDim.x / 8, bid = (int)blockIdx.x;
+	const int block = bid < per * 8 ? (bid % 8) * per + bid / 8 : bid;
+	const int j = 4 * block, tid = threadIdx.x;
+	const int64_t sa = (int64_t)r1 * inner;
+	for (int b = tid; b < r1; b += 256) {
+		const float* p = src + (int64_t)b * inner + j;
+		f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+		int a = 0;
+		for (; a + kQ2Steps <= r0; a += kQ2Steps) {
+			f32x4 v[kQ2Steps];
+#pragma unroll
+			for (int u = 0; u < kQ2Steps; ++u) v[u] = *reinterpret_cast<const f32x4*>(p + (a + u) * sa);
+#pragma unroll
+			for (int u = 0; u < kQ2Steps; ++u)
+#pragma unroll
+				for (int c = 0; c < 4; ++c) acc[c] = acc[c] + v[u][c];
+		}
+		for (; a < r0; ++a) {
+			const f32x4 v = *reinterpret_cast<const f32x4*>(p + a * sa);
+#pragma unroll
+			for (int c = 0; c < 4; ++c) acc[c] = acc[c] + v[c];
+		}
+#pragma unroll
+		for (int c = 0; c < 4; ++c) part[c * kQ2Pitch + b] = acc[c];
+	}
+	__syncthreads();
+	if (tid >= 4) return;
+	const float* v = part + tid * kQ2Pitch;
+	float s = 0.0f;
+	int b = 0;
+	for (; b + 32 <= r1; b += 32) {
+		f32x4 t[8];
+#pragma unroll
+		for (int e = 0; e < 8; ++e) t[e] = *reinterpret_cast<const f32x4*>(v + b + 4 * e);
+#pragma unroll
+		for (int e = 0; e < 8; ++e)
+#pragma unroll
+			for (int i = 0; i < 4; ++i) s = s + t[e][i];
+	}
+	for (; b < r1; ++b) s = s + v[b];
+	float* d = dst + j + tid;
+	*d = combine == 0 ? s : combine == 1 ? s + 0.0f : *d + s;
+}
+
 bool sum_rows2_fits(int64_t r0, int64_t r1, int64_t inner) {
 	return r0 > 0 && r1 > 0 && r1 <= kSum2MaxR1 && inner > 0 && r0 < (1 << 30) && inner < (1 << 30) &&
 	       r0 * r1 * inner < ((int64_t)1 << 62) / 4;
@@ -283,6 +337,11 @@ bool sum_rows2_fits(int64_t r0, int64_t r1, int64_t inner) {
 
 hipError_t sum_rows2(const float* src, int64_t r0, int64_t r1, int64_t inner, float* dst, int combine, hipStream_t s) {
 	if (!sum_rows2_fits(r0, r1, inner)) return hipErrorInvalidValue;
+	if (inner % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0) {
+		hipLaunchKernelGGL(sum_rows2_quad_kernel, dim3((unsigned)(inner / 4)), dim3(256), 0, s, src, (int)r0, (int)r1,
+		                   (int)inner, dst, combine);
+		return hipGetLastError();
+	}
 	hipLaunchKernelGGL(sum_rows2_kernel, dim3((unsigned)((inner + kS2Cols - 1) / kS2Cols)), dim3(256), 0, s, src, (int)r0,
 	                   (int)r1, (int)inner, dst, combine);
 	return hipGetLastError();
