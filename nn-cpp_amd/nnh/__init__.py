@@ -202,21 +202,46 @@ def header_functions():
 
 
 # ---- torch plumbing ----
+# A call's own work here is a few microseconds beside kernels of about the same, so the helpers below avoid what costs most
+# in Python: torch.cuda.current_stream() builds a Stream object and checks its device argument (3 us against 0.4 for the
+# raw handle), and an import statement and a dtype tuple per operand add up over a call's eight or so pointers.
+
+_torch = None
+_dtypes = ()
+
+
+def _load_torch():
+    global _torch, _dtypes
+    import torch
+    _dtypes = frozenset((torch.float32, torch.uint8, torch.int32))
+    _torch = torch
+    return torch
+
 
 def _stream(stream):
-    import torch
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return C.c_void_p(stream.cuda_stream)
+    if stream is not None:
+        return C.c_void_p(stream.cuda_stream)
+    torch = _torch or _load_torch()
+    # the current stream's handle; current_device() initialises the device context as current_stream() would
+    return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+
+
+def _p(t):
+    """The device address of a tensor's first element as an int (None for None), its dtype and device checked."""
+    if t is None:
+        return None
+    if t.dtype not in _dtypes:
+        _load_torch()
+        assert t.dtype in _dtypes, t.dtype
+    assert t.is_cuda, "nnh works on device tensors"
+    return t.data_ptr()
 
 
 def _ptr(t, offset=0):
+    """_p as a ctypes pointer, offset elements on."""
     if t is None:
         return None
-    import torch
-    assert t.dtype in (torch.float32, torch.uint8, torch.int32), t.dtype
-    assert t.is_cuda, "nnh works on device tensors"
-    return C.c_void_p(t.data_ptr() + offset * t.element_size())
+    return C.c_void_p(_p(t) + (offset * t.element_size() if offset else 0))
 
 
 def make_batch(shape=(), sa=(), sb=(), sc=()):
@@ -238,7 +263,7 @@ def make_epilogue(bias_mode=BIAS_NONE, bias=None, relu=False, alive=None):
 
 def sgemm(ta, tb, m, n, k, a, lda, b, ldb, c, ldc, accumulate=False, stream=None):
     """nn::kernels::sgemm on device tensors a, b, c (their first element is the matrix origin)."""
-    check(lib().nnh_sgemm(int(ta), int(tb), m, n, k, _ptr(a), lda, _ptr(b), ldb, _ptr(c), ldc, int(accumulate),
+    check(lib().nnh_sgemm(int(ta), int(tb), m, n, k, _p(a), lda, _p(b), ldb, _p(c), ldc, int(accumulate),
                           _stream(stream)))
 
 
@@ -246,7 +271,7 @@ def sgemm_batched(ta, tb, m, n, k, a, lda, b, ldb, c, ldc, accumulate=False, bat
                   config=-1, stream=None):
     bp = C.byref(batch) if batch is not None else None
     ep = C.byref(epilogue) if epilogue is not None else None
-    check(lib().nnh_sgemm_config(int(ta), int(tb), m, n, k, _ptr(a), lda, _ptr(b), ldb, _ptr(c), ldc,
+    check(lib().nnh_sgemm_config(int(ta), int(tb), m, n, k, _p(a), lda, _p(b), ldb, _p(c), ldc,
                                  int(accumulate), bp, ep, int(config), _stream(stream)))
 
 
@@ -266,13 +291,16 @@ def matmul_shape(a_shape, b_shape, ta=False, tb=False):
 
 def matmul(a, b, ta=False, tb=False, stream=None):
     """nn::matmul(a, b, ta, tb) on contiguous device tensors; returns a new tensor."""
-    import torch
+    torch = _torch or _load_torch()
     assert a.is_contiguous() and b.is_contiguous()
-    shape = matmul_shape(a.shape, b.shape, ta, tb)
+    if a.dim() == 2 and b.dim() == 2 and a.shape[0 if ta else 1] == b.shape[1 if tb else 0]:
+        shape = (a.shape[1 if ta else 0], b.shape[0 if tb else 1])  # two conforming matrices: no question to the library
+    else:
+        shape = matmul_shape(a.shape, b.shape, ta, tb)
     out = torch.empty(shape, dtype=torch.float32, device=a.device)
     ash = (C.c_size_t * a.dim())(*a.shape)
     bsh = (C.c_size_t * b.dim())(*b.shape)
-    check(lib().nnh_matmul(_ptr(a), ash, a.dim(), _ptr(b), bsh, b.dim(), int(ta), int(tb), _ptr(out),
+    check(lib().nnh_matmul(_p(a), ash, a.dim(), _p(b), bsh, b.dim(), int(ta), int(tb), _p(out),
                            _stream(stream)))
     return out
 
@@ -281,43 +309,43 @@ def matmul_backward(g, a, b, b_transposed=False, da=None, da_first=True, db=None
     """nn::matmul / nn::matmul_bt backward into the given gradient buffers (either may be None)."""
     ash = (C.c_size_t * a.dim())(*a.shape)
     bsh = (C.c_size_t * b.dim())(*b.shape)
-    check(lib().nnh_matmul_backward(_ptr(g), _ptr(a), ash, a.dim(), _ptr(b), bsh, b.dim(), int(b_transposed), _ptr(da),
-                                    int(da_first), _ptr(db), int(db_first), _stream(stream)))
+    check(lib().nnh_matmul_backward(_p(g), _p(a), ash, a.dim(), _p(b), bsh, b.dim(), int(b_transposed), _p(da),
+                                    int(da_first), _p(db), int(db_first), _stream(stream)))
 
 
 def linear_forward(x, w, bias, relu=False, stream=None):
     """nn::linear (optionally followed by nn::relu) on device tensors; returns y."""
-    import torch
+    torch = _torch or _load_torch()
     K = x.shape[-1]
     M = x.numel() // K if K else int(torch.tensor(x.shape[:-1]).prod())
     n = w.shape[0]
     y = torch.empty(tuple(x.shape[:-1]) + (n,), dtype=torch.float32, device=x.device)
-    check(lib().nnh_linear_forward(_ptr(x), M, K, _ptr(w), n, _ptr(bias), int(relu), _ptr(y), _stream(stream)))
+    check(lib().nnh_linear_forward(_p(x), M, K, _p(w), n, _p(bias), int(relu), _p(y), _stream(stream)))
     return y
 
 
 def linear_forward_multi(x, layers, stream=None):
     """Several nn::linear forwards over one input x; layers is [(w, bias), ...]; returns the outputs."""
-    import torch
+    torch = _torch or _load_torch()
     K = x.shape[-1]
     M = x.numel() // K if K else int(torch.tensor(x.shape[:-1]).prod())
     ys = [torch.empty(tuple(x.shape[:-1]) + (w.shape[0],), dtype=torch.float32, device=x.device) for w, _ in layers]
     cnt = len(layers)
     arr = lambda ts: (_vp * cnt)(*[t.data_ptr() for t in ts])
     ns = (C.c_size_t * cnt)(*[w.shape[0] for w, _ in layers])
-    check(lib().nnh_linear_forward_multi(_ptr(x), M, K, cnt, arr([w for w, _ in layers]), ns,
+    check(lib().nnh_linear_forward_multi(_p(x), M, K, cnt, arr([w for w, _ in layers]), ns,
                                          arr([b for _, b in layers]), arr(ys), _stream(stream)))
     return ys
 
 
 def linear_forward_add(x, w, bias, residual, out=None, stream=None):
     """nn::add(residual, nn::linear(x, w, bias)) in one kernel; returns y (out, which may be residual itself)."""
-    import torch
+    torch = _torch or _load_torch()
     K = x.shape[-1]
     M = x.numel() // K if K else int(torch.tensor(x.shape[:-1]).prod())
     n = w.shape[0]
     y = out if out is not None else torch.empty(tuple(x.shape[:-1]) + (n,), dtype=torch.float32, device=x.device)
-    check(lib().nnh_linear_forward_add(_ptr(x), M, K, _ptr(w), n, _ptr(bias), _ptr(residual), _ptr(y),
+    check(lib().nnh_linear_forward_add(_p(x), M, K, _p(w), n, _p(bias), _p(residual), _p(y),
                                        _stream(stream)))
     return y
 
@@ -325,31 +353,31 @@ def linear_forward_add(x, w, bias, residual, out=None, stream=None):
 def linear_backward(g, x, w, dx=None, dx_first=True, dw=None, dw_first=True, db=None, db_first=True, stream=None):
     """nn::linear's backward into the given gradient buffers (any may be None)."""
     lead = (C.c_size_t * (x.dim() - 1))(*x.shape[:-1])
-    check(lib().nnh_linear_backward(_ptr(g), _ptr(x), _ptr(w), lead, x.dim() - 1, x.shape[-1], w.shape[0],
-                                    _ptr(dx), int(dx_first), _ptr(dw), int(dw_first), _ptr(db), int(db_first),
+    check(lib().nnh_linear_backward(_p(g), _p(x), _p(w), lead, x.dim() - 1, x.shape[-1], w.shape[0],
+                                    _p(dx), int(dx_first), _p(dw), int(dw_first), _p(db), int(db_first),
                                     _stream(stream)))
 
 
 def relu_forward(x, stream=None):
-    import torch
+    torch = _torch or _load_torch()
     y = torch.empty_like(x)
-    check(lib().nnh_relu_forward(_ptr(x), _ptr(y), x.numel(), _stream(stream)))
+    check(lib().nnh_relu_forward(_p(x), _p(y), x.numel(), _stream(stream)))
     return y
 
 
 def relu_backward(x, g, dx, first=True, stream=None):
-    check(lib().nnh_relu_backward(_ptr(x), _ptr(g), _ptr(dx), int(first), x.numel(), _stream(stream)))
+    check(lib().nnh_relu_backward(_p(x), _p(g), _p(dx), int(first), x.numel(), _stream(stream)))
 
 
 def tensor_sum0(src, dst, combine=0, stream=None):
     rows = src.shape[0]
     inner = src.numel() // rows if rows else dst.numel()
-    check(lib().nnh_tensor_sum0(_ptr(src), rows, inner, _ptr(dst), int(combine), _stream(stream)))
+    check(lib().nnh_tensor_sum0(_p(src), rows, inner, _p(dst), int(combine), _stream(stream)))
 
 
 def zero_many(tensors, stream=None):
     """Every float32 device tensor in `tensors` filled with +0 in one launch per 32 (nnh_zero_many)."""
-    import torch
+    torch = _torch or _load_torch()
     for t in tensors:
         assert t.dtype == torch.float32 and t.is_cuda and t.is_contiguous(), "zero_many takes contiguous float32 device tensors"
     ptrs = (C.c_void_p * max(1, len(tensors)))(*[t.data_ptr() for t in tensors])
@@ -359,13 +387,13 @@ def zero_many(tensors, stream=None):
 
 def attention_forward(q, k, v, heads, mask=None, causal=False, stream=None):
     """nn::attention forward on device tensors; returns (out, probs)."""
-    import torch
+    torch = _torch or _load_torch()
     N, Tq, D = q.shape
     Tk = k.shape[1]
     out = torch.empty((N, Tq, D), dtype=torch.float32, device=q.device)
     probs = torch.empty((N, heads, Tq, Tk), dtype=torch.float32, device=q.device)
-    check(lib().nnh_attention_forward(_ptr(q), _ptr(k), _ptr(v), N, Tq, Tk, D, heads, _ptr(mask), int(causal),
-                                      _ptr(out), _ptr(probs), _stream(stream)))
+    check(lib().nnh_attention_forward(_p(q), _p(k), _p(v), N, Tq, Tk, D, heads, _p(mask), int(causal),
+                                      _p(out), _p(probs), _stream(stream)))
     return out, probs
 
 
@@ -373,24 +401,24 @@ def attention_backward(g, q, k, v, probs, heads, mask=None, causal=False, dq=Non
                        dk_first=True, dv=None, dv_first=True, stream=None):
     N, Tq, D = q.shape
     Tk = k.shape[1]
-    check(lib().nnh_attention_backward(_ptr(g), _ptr(q), _ptr(k), _ptr(v), _ptr(probs), N, Tq, Tk, D, heads,
-                                       _ptr(mask), int(causal), _ptr(dq), int(dq_first), _ptr(dk), int(dk_first),
-                                       _ptr(dv), int(dv_first), _stream(stream)))
+    check(lib().nnh_attention_backward(_p(g), _p(q), _p(k), _p(v), _p(probs), N, Tq, Tk, D, heads,
+                                       _p(mask), int(causal), _p(dq), int(dq_first), _p(dk), int(dk_first),
+                                       _p(dv), int(dv_first), _stream(stream)))
 
 
 def scaled_masked_softmax_forward(x, scale, mask=None, causal=False, stream=None):
-    import torch
+    torch = _torch or _load_torch()
     N, H, Tq, Tk = x.shape
     y = torch.empty_like(x)
-    check(lib().nnh_scaled_masked_softmax_forward(_ptr(x), N, H, Tq, Tk, float(scale), _ptr(mask), int(causal),
-                                                  _ptr(y), _stream(stream)))
+    check(lib().nnh_scaled_masked_softmax_forward(_p(x), N, H, Tq, Tk, float(scale), _p(mask), int(causal),
+                                                  _p(y), _stream(stream)))
     return y
 
 
 def scaled_masked_softmax_backward(y, g, dx, scale, mask=None, causal=False, first=True, stream=None):
     N, H, Tq, Tk = y.shape
-    check(lib().nnh_scaled_masked_softmax_backward(_ptr(y), _ptr(g), N, H, Tq, Tk, float(scale), _ptr(mask),
-                                                   int(causal), _ptr(dx), int(first), _stream(stream)))
+    check(lib().nnh_scaled_masked_softmax_backward(_p(y), _p(g), N, H, Tq, Tk, float(scale), _p(mask),
+                                                   int(causal), _p(dx), int(first), _stream(stream)))
 
 
 def conv_out(H, W, kh, kw, stride, pad):
@@ -402,26 +430,26 @@ def conv_out(H, W, kh, kw, stride, pad):
 
 def conv2d_forward(x, w, bias, stride, pad, fuse_relu, want_alive=True, stream=None):
     """nn::conv2d (fuse_relu=False) or nn::conv2d_relu; returns (y, alive or None)."""
-    import torch
+    torch = _torch or _load_torch()
     N, Cin, H, W = x.shape
     Cout, _, kh, kw = w.shape
     ho, wo = conv_out(H, W, kh, kw, stride, pad)
     y = torch.empty((N, Cout, max(ho, 0), max(wo, 0)), dtype=torch.float32, device=x.device)
     alive = torch.empty(y.shape, dtype=torch.uint8, device=x.device) if (fuse_relu and want_alive) else None
-    check(lib().nnh_conv2d_forward(_ptr(x), N, Cin, H, W, _ptr(w), Cout, kh, kw, _ptr(bias), int(stride), int(pad),
-                                   int(fuse_relu), _ptr(y), _ptr(alive), _stream(stream)))
+    check(lib().nnh_conv2d_forward(_p(x), N, Cin, H, W, _p(w), Cout, kh, kw, _p(bias), int(stride), int(pad),
+                                   int(fuse_relu), _p(y), _p(alive), _stream(stream)))
     return y, alive
 
 
 def maxpool2d_forward(x, kernel, stride, want_argmax=True, stream=None):
     """nn::maxpool2d on a device tensor {N, C, H, W}; returns (y, argmax or None), argmax as int32 holding the uint32
     offsets inside each (n, c) plane."""
-    import torch
+    torch = _torch or _load_torch()
     N, Cc, H, W = x.shape
     ho, wo = (H - kernel) // stride + 1, (W - kernel) // stride + 1
     y = torch.empty((N, Cc, ho, wo), dtype=torch.float32, device=x.device)
     argmax = torch.empty(y.shape, dtype=torch.int32, device=x.device) if want_argmax else None
-    check(lib().nnh_maxpool2d_forward(_ptr(x), N, Cc, H, W, kernel, stride, _ptr(y), _ptr(argmax), _stream(stream)))
+    check(lib().nnh_maxpool2d_forward(_p(x), N, Cc, H, W, kernel, stride, _p(y), _p(argmax), _stream(stream)))
     return y, argmax
 
 
@@ -429,7 +457,7 @@ def conv2d_relu_maxpool2d_forward(x, w, bias, stride, pad, pool_kernel, pool_str
                                   want_argmax=True, stream=None):
     """nn::conv2d_relu then nn::maxpool2d on its output in one call; returns (y, alive or None, pooled, argmax or
     None), argmax as int32 holding the uint32 offsets."""
-    import torch
+    torch = _torch or _load_torch()
     N, Cin, H, W = x.shape
     Cout, _, kh, kw = w.shape
     ho, wo = conv_out(H, W, kh, kw, stride, pad)
@@ -439,9 +467,9 @@ def conv2d_relu_maxpool2d_forward(x, w, bias, stride, pad, pool_kernel, pool_str
         if pool_kernel and pool_stride else (0, 0)
     pooled = torch.empty((N, Cout, max(po, 0), max(qo, 0)), dtype=torch.float32, device=x.device)
     argmax = torch.empty(pooled.shape, dtype=torch.int32, device=x.device) if want_argmax else None
-    check(lib().nnh_conv2d_relu_maxpool2d_forward(_ptr(x), N, Cin, H, W, _ptr(w), Cout, kh, kw, _ptr(bias), int(stride),
-                                                  int(pad), pool_kernel, pool_stride, _ptr(y), _ptr(alive),
-                                                  _ptr(pooled), _ptr(argmax), _stream(stream)))
+    check(lib().nnh_conv2d_relu_maxpool2d_forward(_p(x), N, Cin, H, W, _p(w), Cout, kh, kw, _p(bias), int(stride),
+                                                  int(pad), pool_kernel, pool_stride, _p(y), _p(alive),
+                                                  _p(pooled), _p(argmax), _stream(stream)))
     return y, alive, pooled, argmax
 
 
@@ -449,8 +477,8 @@ def conv2d_backward(g, x, w, alive, stride, pad, dx=None, dx_first=True, dw=None
                     db_first=True, stream=None):
     N, Cin, H, W = x.shape
     Cout, _, kh, kw = w.shape
-    check(lib().nnh_conv2d_backward(_ptr(g), _ptr(x), _ptr(w), _ptr(alive), N, Cin, H, W, Cout, kh, kw, int(stride),
-                                    int(pad), _ptr(dx), int(dx_first), _ptr(dw), int(dw_first), _ptr(db),
+    check(lib().nnh_conv2d_backward(_p(g), _p(x), _p(w), _p(alive), N, Cin, H, W, Cout, kh, kw, int(stride),
+                                    int(pad), _p(dx), int(dx_first), _p(dw), int(dw_first), _p(db),
                                     int(db_first), _stream(stream)))
 
 
@@ -463,21 +491,21 @@ def conv2d_packed_supported(x_shape, w_shape, stride, pad, with_pool=False):
 
 def conv2d_relu_forward_packed(x, w, bias, stride, pad, stream=None):
     """nn::conv2d_relu with its flags packed one bit per output; returns (y, alive_bits as uint8)."""
-    import torch
+    torch = _torch or _load_torch()
     N, Cin, H, W = x.shape
     Cout, _, kh, kw = w.shape
     ho, wo = conv_out(H, W, kh, kw, stride, pad)
     y = torch.empty((N, Cout, max(ho, 0), max(wo, 0)), dtype=torch.float32, device=x.device)
     bits = torch.empty(((y.numel() + 7) // 8,), dtype=torch.uint8, device=x.device)
-    check(lib().nnh_conv2d_relu_forward_packed(_ptr(x), N, Cin, H, W, _ptr(w), Cout, kh, kw, _ptr(bias), int(stride),
-                                               int(pad), _ptr(y), _ptr(bits), _stream(stream)))
+    check(lib().nnh_conv2d_relu_forward_packed(_p(x), N, Cin, H, W, _p(w), Cout, kh, kw, _p(bias), int(stride),
+                                               int(pad), _p(y), _p(bits), _stream(stream)))
     return y, bits
 
 
 def conv2d_relu_maxpool2d_forward_packed(x, w, bias, stride, pad, stream=None):
     """nn::conv2d_relu then a 2 x 2 stride-2 nn::maxpool2d, flags as bits and window maxima as 2-bit positions;
     returns (y, alive_bits, pooled, argmax2), both packed arrays uint8."""
-    import torch
+    torch = _torch or _load_torch()
     N, Cin, H, W = x.shape
     Cout, _, kh, kw = w.shape
     ho, wo = conv_out(H, W, kh, kw, stride, pad)
@@ -485,9 +513,9 @@ def conv2d_relu_maxpool2d_forward_packed(x, w, bias, stride, pad, stream=None):
     bits = torch.empty(((y.numel() + 7) // 8,), dtype=torch.uint8, device=x.device)
     pooled = torch.empty((N, Cout, max(ho, 0) // 2, max(wo, 0) // 2), dtype=torch.float32, device=x.device)
     amax2 = torch.empty((N * Cout * (max(ho, 0) // 2) * ((max(wo, 0) + 7) // 8),), dtype=torch.uint8, device=x.device)
-    check(lib().nnh_conv2d_relu_maxpool2d_forward_packed(_ptr(x), N, Cin, H, W, _ptr(w), Cout, kh, kw, _ptr(bias),
-                                                         int(stride), int(pad), _ptr(y), _ptr(bits), _ptr(pooled),
-                                                         _ptr(amax2), _stream(stream)))
+    check(lib().nnh_conv2d_relu_maxpool2d_forward_packed(_p(x), N, Cin, H, W, _p(w), Cout, kh, kw, _p(bias),
+                                                         int(stride), int(pad), _p(y), _p(bits), _p(pooled),
+                                                         _p(amax2), _stream(stream)))
     return y, bits, pooled, amax2
 
 
@@ -495,36 +523,36 @@ def conv2d_backward_packed(g, x, w, alive_bits, stride, pad, dx=None, dx_first=T
                            db_first=True, stream=None):
     N, Cin, H, W = x.shape
     Cout, _, kh, kw = w.shape
-    check(lib().nnh_conv2d_backward_packed(_ptr(g), _ptr(x), _ptr(w), _ptr(alive_bits), N, Cin, H, W, Cout, kh, kw,
-                                           int(stride), int(pad), _ptr(dx), int(dx_first), _ptr(dw), int(dw_first),
-                                           _ptr(db), int(db_first), _stream(stream)))
+    check(lib().nnh_conv2d_backward_packed(_p(g), _p(x), _p(w), _p(alive_bits), N, Cin, H, W, Cout, kh, kw,
+                                           int(stride), int(pad), _p(dx), int(dx_first), _p(dw), int(dw_first),
+                                           _p(db), int(db_first), _stream(stream)))
 
 
 def maxpool2d_backward_packed(g, argmax2, dx, first=True, stream=None):
     """nn::maxpool2d's backward (kernel 2, stride 2) from 2-bit window positions into dx {N, C, H, W}."""
     N, Cc, H, W = dx.shape
-    check(lib().nnh_maxpool2d_backward_packed(_ptr(g), _ptr(argmax2), N, Cc, H, W, _ptr(dx), int(first),
+    check(lib().nnh_maxpool2d_backward_packed(_p(g), _p(argmax2), N, Cc, H, W, _p(dx), int(first),
                                               _stream(stream)))
 
 
 def im2col(x, kh, kw, stride, pad, stream=None):
-    import torch
+    torch = _torch or _load_torch()
     N, Cin, H, W = x.shape
     ho, wo = conv_out(H, W, kh, kw, stride, pad)
     col = torch.empty((N, Cin * kh * kw, ho * wo), dtype=torch.float32, device=x.device)
-    check(lib().nnh_im2col(_ptr(x), N, Cin, H, W, kh, kw, int(stride), int(pad), _ptr(col), _stream(stream)))
+    check(lib().nnh_im2col(_p(x), N, Cin, H, W, kh, kw, int(stride), int(pad), _p(col), _stream(stream)))
     return col
 
 
 def col2im_add(col, dx, kh, kw, stride, pad, first=False, stream=None):
     N, Cin, H, W = dx.shape
-    check(lib().nnh_col2im_add(_ptr(col), N, Cin, H, W, kh, kw, int(stride), int(pad), _ptr(dx), int(first),
+    check(lib().nnh_col2im_add(_p(col), N, Cin, H, W, kh, kw, int(stride), int(pad), _p(dx), int(first),
                                _stream(stream)))
 
 
 def batchnorm_forward(x, weight, bias, eps, fuse_relu=False, want_alive=True, stream=None):
     """nn::batchnorm (training mode) on a device tensor {N, C, ...}; returns (y, alive or None, mean, var, inv_std)."""
-    import torch
+    torch = _torch or _load_torch()
     N, Cc = x.shape[0], x.shape[1]
     S = 1
     for d in x.shape[2:]:
@@ -532,8 +560,8 @@ def batchnorm_forward(x, weight, bias, eps, fuse_relu=False, want_alive=True, st
     y = torch.empty_like(x)
     alive = torch.empty(x.shape, dtype=torch.uint8, device=x.device) if (fuse_relu and want_alive) else None
     mean, var, inv = (torch.empty(Cc, dtype=torch.float32, device=x.device) for _ in range(3))
-    check(lib().nnh_batchnorm_forward(_ptr(x), N, Cc, S, _ptr(weight), _ptr(bias), float(eps), int(fuse_relu), _ptr(y),
-                                      _ptr(alive), _ptr(mean), _ptr(var), _ptr(inv), _stream(stream)))
+    check(lib().nnh_batchnorm_forward(_p(x), N, Cc, S, _p(weight), _p(bias), float(eps), int(fuse_relu), _p(y),
+                                      _p(alive), _p(mean), _p(var), _p(inv), _stream(stream)))
     return y, alive, mean, var, inv
 
 
@@ -543,21 +571,21 @@ def batchnorm_backward(g, x, alive, weight, mean, inv_std, dx=None, dx_first=Tru
     S = 1
     for d in x.shape[2:]:
         S *= d
-    check(lib().nnh_batchnorm_backward(_ptr(g), _ptr(x), _ptr(alive), _ptr(weight), _ptr(mean), _ptr(inv_std), N, Cc,
-                                       S, _ptr(dx), int(dx_first), _ptr(dw), int(dw_first), _ptr(db), int(db_first),
+    check(lib().nnh_batchnorm_backward(_p(g), _p(x), _p(alive), _p(weight), _p(mean), _p(inv_std), N, Cc,
+                                       S, _p(dx), int(dx_first), _p(dw), int(dw_first), _p(db), int(db_first),
                                        _stream(stream)))
 
 
 def layernorm_forward(x, gamma, beta, eps, stream=None):
     """nn::layernorm over the last axis of a device tensor; returns (y, mean, inv_std), one statistic per row."""
-    import torch
+    torch = _torch or _load_torch()
     D = x.shape[-1]
     R = x.numel() // D
     y = torch.empty_like(x)
     mean = torch.empty(R, dtype=torch.float32, device=x.device)
     inv = torch.empty(R, dtype=torch.float32, device=x.device)
-    check(lib().nnh_layernorm_forward(_ptr(x), R, D, _ptr(gamma), _ptr(beta), float(eps), _ptr(y), _ptr(mean),
-                                      _ptr(inv), _stream(stream)))
+    check(lib().nnh_layernorm_forward(_p(x), R, D, _p(gamma), _p(beta), float(eps), _p(y), _p(mean),
+                                      _p(inv), _stream(stream)))
     return y, mean, inv
 
 
@@ -565,8 +593,8 @@ def layernorm_backward(g, x, gamma, mean, inv_std, dx=None, dx_first=True, dgamm
                        dbeta=None, dbeta_first=True, stream=None):
     D = x.shape[-1]
     R = x.numel() // D
-    check(lib().nnh_layernorm_backward(_ptr(g), _ptr(x), _ptr(gamma), _ptr(mean), _ptr(inv_std), R, D, _ptr(dx),
-                                       int(dx_first), _ptr(dgamma), int(dgamma_first), _ptr(dbeta), int(dbeta_first),
+    check(lib().nnh_layernorm_backward(_p(g), _p(x), _p(gamma), _p(mean), _p(inv_std), R, D, _p(dx),
+                                       int(dx_first), _p(dgamma), int(dgamma_first), _p(dbeta), int(dbeta_first),
                                        _stream(stream)))
 
 
