@@ -5,9 +5,9 @@
 // lane_sum of row (n, c) (eight float partial sums over the row, combined as ((a0+a1)+(a2+a3))+((a4+a5)+(a6+a7)),
 // then the tail), divides by N*S, and does the same with lane_sq around the mean. Here:
 //   * bn_rows_kernel computes the per-row float sums (lane_sum, lane_sq, or the backward's masked lane_sum and
-//     lane_dot): a workgroup owns eight rows of one channel; all its threads stage row chunks in LDS with wide
-//     coalesced loads, and wave 0 runs the reference's eight lane chains per row over LDS (lane 8r + k is partial
-//     a[k] of row r), combines them and adds the tail in order.
+//     lane_dot): a workgroup owns four rows of one channel; all its threads form the terms from wide coalesced
+//     loads and put them in LDS, and wave 0 runs the reference's eight lane chains per row over LDS (lane 8r + k is
+//     partial a[k] of row r), combines them and adds the tail in order.
 //   * The channel-level double sums over n run in order in one thread of every workgroup that needs them (the
 //     rows' sums are staged in LDS first), so the channel's statistics come with each workgroup's own prologue
 //     instead of a launch of their own.
@@ -28,17 +28,45 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kRows = 8;  // rows per workgroup in bn_rows_kernel: one 8-lane group each, all in wave 0
+// acc + v[0] + v[1] + ... + v[n - 1] in order; v is 16-byte aligned LDS.
+__device__ __forceinline__ float lds_chain(const float* v, int n, float acc = 0.0f) {
+	const f32x4* q = reinterpret_cast<const f32x4*>(v);
+	const int nb = n / 16;
+	if (nb > 0) {
+		f32x4 t[3][4];
+#pragma unroll
+		for (int e = 0; e < 4; ++e) t[0][e] = q[e];
+#pragma unroll
+		for (int e = 0; e < 4; ++e) t[1][e] = q[4 * min(1, nb - 1) + e];
+		for (int b = 0; b < nb; b += 3) {
+#pragma unroll
+			for (int k = 0; k < 3; ++k) {
+				// past the end a redundant read of the last block: no branch around a read
+#pragma unroll
+				for (int e = 0; e < 4; ++e) t[(k + 2) % 3][e] = q[4 * min(b + k + 2, nb - 1) + e];
+				__builtin_amdgcn_sched_barrier(0);  // keeps the reads ahead of the adds they run beside
+				if (b + k < nb) {
+#pragma unroll
+					for (int e = 0; e < 4; ++e)
+#pragma unroll
+						for (int i = 0; i < 4; ++i) acc = acc + t[k][e][i];
+				}
+			}
+		}
+	}
+	for (int j = 16 * nb; j < n; ++j) acc = acc + v[j];
+	return acc;
+}
+
+// bn_rows_kernel: rows a workgroup owns, elements of each staged per step, and the LDS layout: partial k's elements
+// k, k + 8, k + 16, ... of a row lie back to back (kPart apart), so that its lane adds them from 16-byte reads. kPart is 8
+// mod 16: both the staging's four-byte stores (two partials, 32 positions) and the chains' reads (eight partials) then use
+// different banks.
+constexpr int kRows = 4, kChunk = 2304, kPart = kChunk / 8 + 8, kRowLds = 8 * kPart;
+constexpr int kRowTail = 8;  // a row's last S mod 8 terms, after the partials
+constexpr int kRowSet = kRows * (kRowLds + kRowTail);
 
 enum BnRowMode { kSum = 0, kSq = 1, kBwd = 2 };
-
-// Elements of each row staged per step. The LDS row pitch is the chunk plus 8 floats: lane 8r + k reads element
-// k + 8i of row r, bank (8r + k + 8i) mod 64 for a pitch of 8 mod 64, so the 64 lanes hit 64 banks.
-template <int MODE>
-struct RowChunk {
-	static constexpr int kChunk = MODE == kBwd ? 768 : 1024;
-	static constexpr int kPitch = kChunk + 8;
-};
 
 struct BnRowArgs {
 	const float* x;
@@ -50,9 +78,10 @@ struct BnRowArgs {
 	float* out1;                  // kBwd: lane_dot of masked g with x - mean
 	float* mean_out;              // kSq: the channel mean, written by the channel's first workgroup
 	int64_t N, C, S;
-	int groups;                   // workgroups per channel: ceil(N / kRows)
+	int64_t groups;               // workgroups per channel: ceil(N / kRows)
+	int64_t first_block;          // of this launch (a grid holds 2^31 - 1)
 	double dm;
-	int vec;                      // S % 4 == 0 and the row starts are 16-byte (flags 4-byte) aligned
+	FastDiv whole, last;          // units of a row in a whole chunk and in the last one
 };
 
 // Sums in double of v0[n * C + c] (and v1's) for n = 0..N-1 in order, as the reference adds a channel's row sums
@@ -72,7 +101,21 @@ __device__ void channel_dsums(const float* v0, const float* v1, int64_t N, int64
 		__syncthreads();
 		if (tid == 0) {
 			const int cnt = (int)(N - n0 < 256 ? N - n0 : 256);
-			for (int i = 0; i < cnt; ++i) {
+			int i = 0;
+			for (; i + 16 <= cnt; i += 16) {  // sixteen LDS reads ahead of the dependent adds
+				float t0[16], t1[16];
+#pragma unroll
+				for (int u = 0; u < 16; ++u) {
+					t0[u] = buf[0][i + u];
+					if (NSUM == 2) t1[u] = buf[1][i + u];
+				}
+#pragma unroll
+				for (int u = 0; u < 16; ++u) {
+					s0 += (double)t0[u];
+					if (NSUM == 2) s1 += (double)t1[u];
+				}
+			}
+			for (; i < cnt; ++i) {
 				s0 += (double)buf[0][i];
 				if (NSUM == 2) s1 += (double)buf[1][i];
 			}
@@ -88,91 +131,91 @@ __device__ void channel_dsums(const float* v0, const float* v1, int64_t N, int64
 	res[1] = out[1];
 }
 
-// Stages elements [s0, s0 + len) of rows n0 .. n0 + nrows - 1 of channel c from src into dst[r * PITCH + l].
-// Loads are clamped to valid addresses and all issued before the LDS stores.
-template <int CHUNK, int PITCH>
-__device__ __forceinline__ void stage_rows(const float* __restrict__ src, int64_t row0, int64_t row_step, int64_t S,
-                                           int64_t s0, int nrows, int len, int vec, float* dst) {
+// lane_sum (ops.cpp:804-812), lane_sq (824-834), and the backward's lane_sum / lane_sum_masked with lane_dot /
+// lane_dot_masked (848-897) of four rows (n0 .. n0 + 3) of channel c per workgroup. All threads load the rows (16-byte
+// loads with VEC: S % 4 == 0, aligned rows), form the terms the chains add (x, (x - mean)^2, or the masked g and g (x -
+// mean)) and put them in LDS; lane 8 r + k of wave 0 (the backward's second sum: lane 32 + 8 r + k) adds partial k of row
+// r, about 7 cycles a term, then the eight partials combine and the row's tail follows in order. Rows longer than kChunk
+// go chunk by chunk, the next chunk's loads in flight during the chains. Measured at [64, 16, 48, 48] (9.4 MB): sums 9.4 ->
+// 6.3 us, squares 10.4 -> 7.4, backward 27.3 -> 7.6, against eight rows a workgroup (128 of them), element-wise work in the
+// chain lanes and three exposed chunk loads.
+template <int MODE, bool VEC>
+__global__ void __launch_bounds__(256) bn_rows_kernel(const BnRowArgs a) {
+	extern __shared__ __align__(16) float lds[];  // a set of terms, and with kBwd a second one
+	__shared__ float buf[2][256];
+	__shared__ double bcast[2];
+	constexpr int kW = VEC ? 4 : 1;                        // floats of a unit
+	constexpr int kPer = kRows * kChunk / kW / 256;        // units a thread holds
+	constexpr int kBatch = VEC ? kPer : 18;                // of them in flight at once
 	const int tid = threadIdx.x;
-	if (vec) {
-		constexpr int kPer = kRows * CHUNK / 4 / 256;
-		const int q4 = len >> 2, tot = nrows * q4;
-		if (tot == 0) return;
-		f32x4 v[kPer];
+	const int64_t blk = a.first_block + blockIdx.x;
+	const int64_t c = blk / a.groups, j = blk - c * a.groups;
+	const int64_t n0 = j * kRows;
+	const int nrows = (int)(a.N - n0 < kRows ? (a.N > n0 ? a.N - n0 : 0) : kRows);
+	const int64_t row0 = n0 * a.C + c;  // row index of (n0, c); rows of one channel are C apart
+	const int64_t full = a.S & ~(int64_t)7;
+	const bool masked = MODE == kBwd && a.alive != nullptr;
+
+	float xv[kBatch][kW], gv[kBatch][kW];
+	unsigned fv[kBatch];
+	// units u0 .. u0 + kBatch - 1 (times 256 threads) of the chunk from s0: loads at clamped indices, then the terms
+	auto load = [&](int64_t s0, int u0, int tot, const FastDiv& dv) {
 #pragma unroll
-		for (int u = 0; u < kPer; ++u) {
-			const int ii = min(tid + 256 * u, tot - 1);
-			const int r = ii / q4, q = ii - r * q4;
-			v[u] = *reinterpret_cast<const f32x4*>(src + (row0 + r * row_step) * S + s0 + 4 * q);
-		}
+		for (int u = 0; u < kBatch; ++u) {
+			const int i = min(tid + 256 * (u0 + u), tot - 1);
+			const int r = (int)fdiv((unsigned)i, dv), q = i - r * (int)dv.d;
+			const int64_t at = (row0 + r * a.C) * a.S + s0 + kW * q;
+			if constexpr (VEC) {
+				const f32x4 x4 = *reinterpret_cast<const f32x4*>(a.x + at);
 #pragma unroll
-		for (int u = 0; u < kPer; ++u) {
-			const int idx = tid + 256 * u;
-			if (idx < tot) {
-				const int r = idx / q4, q = idx - r * q4;
-				*reinterpret_cast<f32x4*>(dst + r * PITCH + 4 * q) = v[u];
-			}
-		}
-	} else {
-		constexpr int kPer = kRows * CHUNK / 256;
-		const int tot = nrows * len;
-		if (tot == 0) return;
-		for (int b = 0; b < kPer; b += 16) {
-			float v[16];
+				for (int e = 0; e < 4; ++e) xv[u][e] = x4[e];
+				if (MODE == kBwd) {
+					const f32x4 g4 = *reinterpret_cast<const f32x4*>(a.g + at);
 #pragma unroll
-			for (int u = 0; u < 16; ++u) {
-				const int ii = min(tid + 256 * (b + u), tot - 1);
-				const int r = ii / len, l = ii - r * len;
-				v[u] = src[(row0 + r * row_step) * S + s0 + l];
-			}
-#pragma unroll
-			for (int u = 0; u < 16; ++u) {
-				const int idx = tid + 256 * (b + u);
-				if (idx < tot) {
-					const int r = idx / len, l = idx - r * len;
-					dst[r * PITCH + l] = v[u];
+					for (int e = 0; e < 4; ++e) gv[u][e] = g4[e];
+					if (masked) fv[u] = *reinterpret_cast<const unsigned*>(a.alive + at);
+				}
+			} else {
+				xv[u][0] = a.x[at];
+				if (MODE == kBwd) {
+					gv[u][0] = a.g[at];
+					if (masked) fv[u] = a.alive[at];
 				}
 			}
 		}
-	}
-}
-
-__device__ __forceinline__ void stage_flags(const unsigned char* __restrict__ src, int64_t row0, int64_t row_step,
-                                            int64_t S, int64_t s0, int nrows, int len, int vec, unsigned char* dst,
-                                            int pitch) {
-	const int tid = threadIdx.x;
-	if (vec) {
-		const int q4 = len >> 2, tot = nrows * q4;
-		for (int idx = tid; idx < tot; idx += 256) {
-			const int r = idx / q4, q = idx - r * q4;
-			*reinterpret_cast<unsigned*>(dst + r * pitch + 4 * q) =
-			    *reinterpret_cast<const unsigned*>(src + (row0 + r * row_step) * S + s0 + 4 * q);
-		}
-	} else {
-		const int tot = nrows * len;
-		for (int idx = tid; idx < tot; idx += 256) {
-			const int r = idx / len, l = idx - r * len;
-			dst[r * pitch + l] = src[(row0 + r * row_step) * S + s0 + l];
-		}
-	}
-}
-
-// lane_sum (ops.cpp:804-812), lane_sq (824-834), and the backward's lane_sum / lane_sum_masked with lane_dot /
-// lane_dot_masked (848-897) of eight rows (n0 .. n0 + 7) of channel c per workgroup.
-template <int MODE>
-__global__ void __launch_bounds__(256) bn_rows_kernel(const BnRowArgs a) {
-	constexpr int kChunk = RowChunk<MODE>::kChunk, kPitch = RowChunk<MODE>::kPitch;
-	__shared__ __align__(16) float xs[kRows * kPitch];
-	__shared__ __align__(16) float gs[MODE == kBwd ? kRows * kPitch : 1];
-	__shared__ __align__(16) unsigned char fs[MODE == kBwd ? kRows * kPitch : 4];
-	__shared__ float buf[2][256];
-	__shared__ double bcast[2];
-	const int tid = threadIdx.x;
-	const int64_t c = blockIdx.x / a.groups;
-	const int j = (int)(blockIdx.x - c * a.groups);
-	const int64_t n0 = (int64_t)j * kRows;
-	const int nrows = (int)(a.N - n0 < kRows ? a.N - n0 : kRows);
+	};
 	float mu = 0.0f;
+	auto put = [&](int64_t s0, int u0, int tot, const FastDiv& dv) {
+#pragma unroll
+		for (int u = 0; u < kBatch; ++u) {
+			const int i = tid + 256 * (u0 + u);
+			if (i >= tot) continue;
+			const int r = (int)fdiv((unsigned)i, dv), l = kW * (i - r * (int)dv.d);
+#pragma unroll
+			for (int e = 0; e < kW; ++e) {
+				float t0, t1 = 0.0f;
+				if (MODE == kSum) {
+					t0 = xv[u][e];
+				} else if (MODE == kSq) {
+					const float d = xv[u][e] - mu;
+					t0 = d * d;
+				} else {
+					t0 = masked && !((fv[u] >> (8 * e)) & 0xffu) ? 0.0f : gv[u][e];
+					t1 = t0 * (xv[u][e] - mu);
+				}
+				const int at = s0 + l + e < full ? r * kRowLds + ((l + e) & 7) * kPart + ((l + e) >> 3)
+				                                 : kRows * kRowLds + r * kRowTail + (int)(s0 + l + e - full);
+				lds[at] = t0;
+				if (MODE == kBwd) lds[kRowSet + at] = t1;
+			}
+		}
+	};
+	auto chunk_len = [&](int64_t s0) { return (int)(a.S - s0 < kChunk ? a.S - s0 : kChunk); };
+	auto units = [&](int64_t s0) { return nrows * (chunk_len(s0) / kW); };
+	auto div_of = [&](int64_t s0) -> const FastDiv& { return s0 + kChunk < a.S ? a.whole : a.last; };
+	// With VEC a whole chunk is one batch, loaded before the channel's mean is known
+	const bool any = nrows > 0 && a.S > 0;
+	if (VEC && any) load(0, 0, units(0), div_of(0));
 	if (MODE == kSq) {
 		double s[2];
 		channel_dsums<1>(a.rowsum, nullptr, a.N, a.C, c, buf, bcast, s);
@@ -181,101 +224,40 @@ __global__ void __launch_bounds__(256) bn_rows_kernel(const BnRowArgs a) {
 	} else if (MODE == kBwd) {
 		mu = a.mean[c];
 	}
-	const bool masked = MODE == kBwd && a.alive != nullptr;
-	const int r = tid >> 3, k = tid & 7;
-	const int64_t full = a.S & ~(int64_t)7;
-	const int64_t row0 = n0 * a.C + c;  // row index of (n0, c); rows of one channel are C apart
-	float acc0 = 0.0f, acc1 = 0.0f;
-	int64_t s0 = 0;
-	do {
-		const int len = (int)(a.S - s0 < kChunk ? a.S - s0 : kChunk);
-		stage_rows<kChunk, kPitch>(MODE == kBwd ? a.g : a.x, row0, a.C, a.S, s0, nrows, len, a.vec,
-		                           MODE == kBwd ? gs : xs);
-		if (MODE == kBwd) {
-			stage_rows<kChunk, kPitch>(a.x, row0, a.C, a.S, s0, nrows, len, a.vec, xs);
-			if (masked) stage_flags(a.alive, row0, a.C, a.S, s0, nrows, len, a.vec, fs, kPitch);
-		}
-		__syncthreads();
-		if (tid < 64) {
-			const int lfull = (int)(full - s0 < len ? (full - s0 > 0 ? full - s0 : 0) : len);
-			if (r < nrows) {
-				const float* xr = xs + r * kPitch;
-				const float* gr = gs + r * kPitch;
-				const unsigned char* fr = fs + r * kPitch;
-				// 16 steps of the lane's chain per batch: the batch's LDS reads are all issued before its adds
-				int l = k;
-				for (; l + 8 * 15 < lfull; l += 8 * 16) {
-					float xv[16], gv[16];
-					unsigned char fv[16];
-#pragma unroll
-					for (int u = 0; u < 16; ++u) {
-						xv[u] = xr[l + 8 * u];
-						if (MODE == kBwd) {
-							gv[u] = gr[l + 8 * u];
-							if (masked) fv[u] = fr[l + 8 * u];
-						}
-					}
-#pragma unroll
-					for (int u = 0; u < 16; ++u) {
-						if (MODE == kSum) {
-							acc0 = acc0 + xv[u];
-						} else if (MODE == kSq) {
-							const float d = xv[u] - mu;
-							acc0 = acc0 + d * d;
-						} else {
-							const float gm = masked ? (fv[u] ? gv[u] : 0.0f) : gv[u];
-							acc0 = acc0 + gm;
-							acc1 = acc1 + gm * (xv[u] - mu);
-						}
-					}
-				}
-				for (; l < lfull; l += 8) {
-					if (MODE == kSum) {
-						acc0 = acc0 + xr[l];
-					} else if (MODE == kSq) {
-						const float d = xr[l] - mu;
-						acc0 = acc0 + d * d;
-					} else {
-						const float gm = masked ? (fr[l] ? gr[l] : 0.0f) : gr[l];
-						acc0 = acc0 + gm;
-						acc1 = acc1 + gm * (xr[l] - mu);
-					}
-				}
-			}
-			if (s0 + len >= a.S) {  // last chunk: combine the eight partials of each row, then the tail in order
-				const int base = (tid & 63) & ~7;
-				float p0[8], p1[8];
-#pragma unroll
-				for (int u = 0; u < 8; ++u) {
-					p0[u] = __shfl(acc0, base + u);
-					if (MODE == kBwd) p1[u] = __shfl(acc1, base + u);
-				}
-				if (k == 0 && r < nrows) {
-					float t0 = ((p0[0] + p0[1]) + (p0[2] + p0[3])) + ((p0[4] + p0[5]) + (p0[6] + p0[7]));
-					float t1 = 0.0f;
-					if (MODE == kBwd) t1 = ((p1[0] + p1[1]) + (p1[2] + p1[3])) + ((p1[4] + p1[5]) + (p1[6] + p1[7]));
-					const float* xr = xs + r * kPitch;
-					for (int l = lfull; l < len; ++l) {
-						if (MODE == kSum) {
-							t0 = t0 + xr[l];
-						} else if (MODE == kSq) {
-							t0 = t0 + (xr[l] - mu) * (xr[l] - mu);
-						} else {
-							const float gv =
-							    masked ? (fs[r * kPitch + l] ? gs[r * kPitch + l] : 0.0f) : gs[r * kPitch + l];
-							t0 = t0 + gv;
-							t1 = t1 + gv * (xr[l] - mu);
-						}
-					}
-					const int64_t row = row0 + r * a.C;
-					a.out0[row] = t0;
-					if (MODE == kBwd) a.out1[row] = t1;
-				}
+	if (nrows <= 0) return;
+	const int which = (tid >> 5) & 1, r = (tid >> 3) & 3, k = tid & 7;
+	const bool adds = tid < 64 && r < nrows && (which == 0 || MODE == kBwd);
+	const float* set = lds + which * kRowSet;
+	float acc = 0.0f;
+	for (int64_t s0 = 0; s0 < a.S; s0 += kChunk) {
+		const int tot = units(s0);
+		if constexpr (VEC) {
+			put(s0, 0, tot, div_of(s0));
+		} else {
+			for (int u0 = 0; u0 < kPer; u0 += kBatch) {
+				load(s0, u0, tot, div_of(s0));
+				put(s0, u0, tot, div_of(s0));
 			}
 		}
 		__syncthreads();
-		s0 += kChunk;
-	} while (s0 < a.S);
+		if (VEC && s0 + kChunk < a.S) load(s0 + kChunk, 0, units(s0 + kChunk), div_of(s0 + kChunk));
+		if (adds) {
+			const int64_t left = full - s0;
+			const int n = (int)(left < kChunk ? (left > 0 ? left : 0) : kChunk) / 8;
+			acc = lds_chain(set + r * kRowLds + k * kPart, n, acc);
+		}
+		__syncthreads();
+	}
+	if (tid >= 64) return;
+	// the partials combine as ((a0 + a1) + (a2 + a3)) + ((a4 + a5) + (a6 + a7)), then the tail in order
+	float p[8];
+#pragma unroll
+	for (int u = 0; u < 8; ++u) p[u] = __shfl(acc, (tid & ~7) + u);
+	if (!adds || k != 0) return;
+	float t = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+	const float* tail = set + kRows * kRowLds + r * kRowTail;
+	for (int l = 0; l < (int)(a.S - full); ++l) t = t + tail[l];
+	(which == 0 ? a.out0 : a.out1)[row0 + r * a.C] = t;
 }
 
 constexpr int kElemChunk = 4096;  // channel elements per workgroup in the elementwise kernels (16 per thread)
@@ -322,6 +304,19 @@ __global__ void __launch_bounds__(256) bn_norm_kernel(const BnElemArgs a) {
 	const int tid = threadIdx.x;
 	const int64_t c = blockIdx.x / a.chunks;
 	const int64_t j = blockIdx.x - c * a.chunks;
+	const int64_t total = a.N * a.S;
+	const int64_t e0 = j * kElemChunk;
+	// the chunk's elements are loaded ahead of the channel's sums (clamped: past the end the last group again)
+	f32x4 xs[kElemChunk / 1024];
+	int64_t offs[kElemChunk / 1024];
+	if (a.vec && total > 0) {
+#pragma unroll
+		for (int u = 0; u < kElemChunk / 1024; ++u) {
+			const int64_t e = e0 + 4 * (tid + 256 * u);
+			offs[u] = channel_offset<FAST>(e < total ? e : total - 4, a, c);
+			xs[u] = *reinterpret_cast<const f32x4*>(a.x + offs[u]);
+		}
+	}
 	double s[2];
 	channel_dsums<1>(a.rowv0, nullptr, a.N, a.C, c, buf, bcast, s);
 	const float mu = a.mean[c];
@@ -332,15 +327,12 @@ __global__ void __launch_bounds__(256) bn_norm_kernel(const BnElemArgs a) {
 		a.inv_out[c] = inv;
 	}
 	const float scale = a.w[c] * inv, bc = a.b[c];
-	const int64_t total = a.N * a.S;
-	const int64_t e0 = j * kElemChunk;
 	if (a.vec) {
 #pragma unroll
 		for (int u = 0; u < kElemChunk / 1024; ++u) {
-			const int64_t e = e0 + 4 * (tid + 256 * u);
-			if (e >= total) break;
-			const int64_t off = channel_offset<FAST>(e, a, c);
-			const f32x4 xv = *reinterpret_cast<const f32x4*>(a.x + off);
+			if (e0 + 4 * (tid + 256 * u) >= total) continue;
+			const int64_t off = offs[u];
+			const f32x4 xv = xs[u];
 			f32x4 o;
 			unsigned fl = 0;
 #pragma unroll
@@ -382,6 +374,23 @@ __global__ void __launch_bounds__(256) bn_dx_kernel(const BnElemArgs a) {
 	const int tid = threadIdx.x;
 	const int64_t c = blockIdx.x / a.chunks;
 	const int64_t j = blockIdx.x - c * a.chunks;
+	const int64_t total = a.N * a.S;
+	const int64_t e0 = j * kElemChunk;
+	const bool masked = a.alive_in != nullptr;
+	// loaded ahead of the channel's sums, as in bn_norm_kernel
+	f32x4 gs[kElemChunk / 1024], xs[kElemChunk / 1024];
+	unsigned fls[kElemChunk / 1024];
+	int64_t offs[kElemChunk / 1024];
+	if (a.y && a.vec && total > 0) {
+#pragma unroll
+		for (int u = 0; u < kElemChunk / 1024; ++u) {
+			const int64_t e = e0 + 4 * (tid + 256 * u);
+			offs[u] = channel_offset<FAST>(e < total ? e : total - 4, a, c);
+			gs[u] = *reinterpret_cast<const f32x4*>(a.g + offs[u]);
+			xs[u] = *reinterpret_cast<const f32x4*>(a.x + offs[u]);
+			fls[u] = masked ? *reinterpret_cast<const unsigned*>(a.alive_in + offs[u]) : 0x01010101u;
+		}
+	}
 	double s[2];
 	channel_dsums<2>(a.rowv0, a.rowv1, a.N, a.C, c, buf, bcast, s);
 	const float mu = a.mean[c], inv = a.inv_in[c];
@@ -392,18 +401,13 @@ __global__ void __launch_bounds__(256) bn_dx_kernel(const BnElemArgs a) {
 	}
 	if (!a.y) return;
 	const float kk = a.w[c] * inv / a.fm, fm = a.fm, av = (float)sdy, bb = (float)sdyx;
-	const int64_t total = a.N * a.S;
-	const int64_t e0 = j * kElemChunk;
-	const bool masked = a.alive_in != nullptr;
 	if (a.vec) {
 #pragma unroll
 		for (int u = 0; u < kElemChunk / 1024; ++u) {
-			const int64_t e = e0 + 4 * (tid + 256 * u);
-			if (e >= total) break;
-			const int64_t off = channel_offset<FAST>(e, a, c);
-			const f32x4 gv = *reinterpret_cast<const f32x4*>(a.g + off);
-			const f32x4 xv = *reinterpret_cast<const f32x4*>(a.x + off);
-			const unsigned fl = masked ? *reinterpret_cast<const unsigned*>(a.alive_in + off) : 0x01010101u;
+			if (e0 + 4 * (tid + 256 * u) >= total) continue;
+			const int64_t off = offs[u];
+			const f32x4 gv = gs[u], xv = xs[u];
+			const unsigned fl = fls[u];
 			f32x4 old = a.first ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : *reinterpret_cast<const f32x4*>(a.y + off);
 			f32x4 o;
 #pragma unroll
@@ -560,36 +564,6 @@ __global__ void __launch_bounds__(256) ln_backward_kernel(const LnBwdArgs a) {
 constexpr int kLnMaxRows = 32;  // chains of one kind in a wave: lanes 0 .. 31, the backward's second kind lanes 32 .. 63
 
 __device__ __host__ __forceinline__ int ln_pitch(int D) { return ((D + 3) & ~3) + 4; }
-
-// acc + v[0] + v[1] + ... + v[n - 1] in order; v is 16-byte aligned LDS.
-__device__ __forceinline__ float lds_chain(const float* v, int n, float acc = 0.0f) {
-	const f32x4* q = reinterpret_cast<const f32x4*>(v);
-	const int nb = n / 16;
-	if (nb > 0) {
-		f32x4 t[3][4];
-#pragma unroll
-		for (int e = 0; e < 4; ++e) t[0][e] = q[e];
-#pragma unroll
-		for (int e = 0; e < 4; ++e) t[1][e] = q[4 * min(1, nb - 1) + e];
-		for (int b = 0; b < nb; b += 3) {
-#pragma unroll
-			for (int k = 0; k < 3; ++k) {
-				// past the end a redundant read of the last block: no branch around a read
-#pragma unroll
-				for (int e = 0; e < 4; ++e) t[(k + 2) % 3][e] = q[4 * min(b + k + 2, nb - 1) + e];
-				__builtin_amdgcn_sched_barrier(0);  // keeps the reads ahead of the adds they run beside
-				if (b + k < nb) {
-#pragma unroll
-					for (int e = 0; e < 4; ++e)
-#pragma unroll
-						for (int i = 0; i < 4; ++i) acc = acc + t[k][e][i];
-				}
-			}
-		}
-	}
-	for (int j = 16 * nb; j < n; ++j) acc = acc + v[j];
-	return acc;
-}
 
 struct LnArgs {
 	const float* x;
@@ -1025,7 +999,7 @@ const LnBackwardFn kLnBackward[2][2][3] = {
      {ln_backward_rows_kernel<16, true, 0>, ln_backward_rows_kernel<16, true, 1>, ln_backward_rows_kernel<16, true, 2>}}};
 
 // Raises the kernels' dynamic LDS limit once per device (a row of kLnMaxD floats and its product: 131 KB).
-hipError_t prepare_ln() {
+hipError_t prepare_norm() {
 	static std::mutex mu;
 	static bool done[64] = {};
 	int dev = 0;
@@ -1037,6 +1011,8 @@ hipError_t prepare_ln() {
 	auto raise = [&](const void* fn) {
 		if (e == hipSuccess) e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
 	};
+	raise(reinterpret_cast<const void*>(bn_rows_kernel<kBwd, false>));  // two sets of terms: 76 KB
+	raise(reinterpret_cast<const void*>(bn_rows_kernel<kBwd, true>));
 	for (int p = 0; p < 2; ++p)
 		for (int v = 0; v < 2; ++v) {
 			raise(reinterpret_cast<const void*>(kLnForward[p][v]));
@@ -1056,12 +1032,23 @@ int ln_rows(int64_t R, int D, int blocks) {
 inline bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 template <int MODE>
-hipError_t launch_rows(BnRowArgs& a, hipStream_t s) {
-	a.groups = (int)((a.N + kRows - 1) / kRows);
-	const int64_t blocks = a.C * (a.groups > 0 ? a.groups : 1);
-	if (a.groups == 0) a.groups = 1;
-	hipLaunchKernelGGL(bn_rows_kernel<MODE>, dim3((unsigned)blocks), dim3(256), 0, s, a);
-	return hipGetLastError();
+hipError_t launch_rows(BnRowArgs& a, bool vec, hipStream_t s) {
+	const hipError_t e = prepare_norm();
+	if (e != hipSuccess) return e;
+	a.groups = std::max<int64_t>(1, (a.N + kRows - 1) / kRows);
+	const int per = vec ? 4 : 1;
+	const int64_t last = a.S > 0 ? (a.S - 1) % kChunk + 1 : per;
+	a.whole = make_fastdiv((unsigned)(kChunk / per));
+	a.last = make_fastdiv((unsigned)(last / per));
+	const int64_t blocks = a.C * a.groups, most = ((int64_t)1 << 31) - 1;
+	for (a.first_block = 0; a.first_block < blocks; a.first_block += most) {
+		hipLaunchKernelGGL((vec ? bn_rows_kernel<MODE, true> : bn_rows_kernel<MODE, false>),
+		                   dim3((unsigned)std::min(most, blocks - a.first_block)), dim3(256),
+		                   (MODE == kBwd ? 2 : 1) * kRowSet * sizeof(float), s, a);
+		const hipError_t err = hipGetLastError();
+		if (err != hipSuccess) return err;
+	}
+	return hipSuccess;
 }
 
 hipError_t launch_elem(bool fwd, BnElemArgs& a, hipStream_t s) {
@@ -1096,16 +1083,16 @@ hipError_t batchnorm_forward(const float* x, const float* w, const float* b, con
 	r.C = g.C;
 	r.S = g.S;
 	r.dm = g.dm;
-	r.vec = g.S % 4 == 0 && aligned16(x);
+	const bool row_vec = g.S % 4 == 0 && aligned16(x);
 	hipError_t e = hipSuccess;
 	if (g.N > 0) {
-		e = launch_rows<kSum>(r, s);
+		e = launch_rows<kSum>(r, row_vec, s);
 		if (e != hipSuccess) return e;
 	}
 	r.rowsum = rowsum;
 	r.out0 = rowsq;
 	r.mean_out = mean;
-	e = launch_rows<kSq>(r, s);  // also writes the channel means (a workgroup per channel when N is 0)
+	e = launch_rows<kSq>(r, row_vec, s);  // also writes the channel means (a workgroup per channel when N is 0)
 	if (e != hipSuccess) return e;
 	BnElemArgs a{};
 	a.x = x;
@@ -1146,8 +1133,9 @@ hipError_t batchnorm_backward(const float* gy, const float* x, const unsigned ch
 		r.C = g.C;
 		r.S = g.S;
 		r.dm = g.dm;
-		r.vec = g.S % 4 == 0 && aligned16(x) && aligned16(gy) && (!alive || reinterpret_cast<uintptr_t>(alive) % 4 == 0);
-		const hipError_t e = launch_rows<kBwd>(r, s);
+		const bool row_vec =
+		    g.S % 4 == 0 && aligned16(x) && aligned16(gy) && (!alive || reinterpret_cast<uintptr_t>(alive) % 4 == 0);
+		const hipError_t e = launch_rows<kBwd>(r, row_vec, s);
 		if (e != hipSuccess) return e;
 	}
 	BnElemArgs a{};
@@ -1194,7 +1182,7 @@ hipError_t layernorm_forward(const float* x, const float* gamma, const float* be
 		a.eps = eps;
 		const bool vec = D % 4 == 0 && aligned16(x) && aligned16(y);
 		a.dq = make_fastdiv((unsigned)(vec ? D / 4 : D));
-		const hipError_t e = prepare_ln();
+		const hipError_t e = prepare_norm();
 		if (e != hipSuccess) return e;
 		hipLaunchKernelGGL(kLnForward[D > 8192 ? 1 : 0][vec ? 1 : 0], dim3((unsigned)((R + rw - 1) / rw)), dim3(256),
 		                   (size_t)rw * (ln_pitch(D) + 2) * sizeof(float), s, a);
@@ -1229,7 +1217,7 @@ hipError_t layernorm_backward(const float* gy, const float* x, const float* gamm
 		a.dq = make_fastdiv((unsigned)(vec ? D / 4 : D));
 		LnColArgs d{gy, x, mean, inv_std, R, D, dgamma, dgamma_first, dbeta, dbeta_first, 0};
 		const bool small = cols && R <= kLnSmallRows;
-		hipError_t e = prepare_ln();
+		hipError_t e = prepare_norm();
 		if (e != hipSuccess) return e;
 		if (small && !dx) {
 			d.blocks = (D + kLnSmallCols - 1) / kLnSmallCols;
