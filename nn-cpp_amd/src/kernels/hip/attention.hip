@@ -1,22 +1,22 @@
 // attention.hip - nn::attention's forward (src/autograd/ops.cpp:1226-1261) as one kernel for head width 64.
 //
-// A workgroup owns 64 query rows of one (sample, head) pair and runs the reference's three steps for them
+// A workgroup owns 32 query rows of one (sample, head) pair and runs the reference's three steps for them
 // with the score rows resident in LDS:
-//   1. S = Q_h K_h^T: each element the fma chain over d = 0..63 from +0 (sgemm F,T, ops.cpp:1256). Wave w
-//      takes keys 64w..64w+63 against the 64 queries as two 32x32x1 MFMA chains computing S^T (the product
-//      fma(k, q, acc) is the reference's fma(q, k, acc)); lane l holds key row 64w + l in registers (the
-//      MFMA's A operand), the queries come from LDS.
-//   2. masked_softmax_row (ops.cpp:1183-1204) over the 64 rows: scale and mask, std::max's scan, glibc's
+//   1. S = Q_h K_h^T: each element the fma chain over d = 0..63 from +0 (sgemm F,T, ops.cpp:1256). A wave takes 64
+//      keys against the 32 queries, computing S^T (the product fma(k, q, acc) is the reference's fma(q, k, acc)).
+//   2. masked_softmax_row (ops.cpp:1183-1204) over the 32 rows: scale and mask, std::max's scan, glibc's
 //      expf, the sum over live keys in key order, the division; the probabilities go to `probs` (kept for the
 //      backward pass) and stay in LDS.
 //   3. O_h = P V_h: each element the fma chain over the keys j = 0..Tk-1 from +0 (sgemm F,F, ops.cpp:1259),
-//      every key included (a zero probability still meets its V entry). Wave w takes output columns
-//      16w..16w+15 as one 16x16x1 MFMA chain over the 64 rows; P comes from LDS, V from global memory a
-//      chunk of keys ahead.
+//      every key included (a zero probability still meets its V entry). Wave w takes output columns 16w..16w+15;
+//      P comes from LDS, V from global memory 16 steps of four keys ahead.
 // Same bits as the three-launch path (batched GEMM, row softmax, batched GEMM): both sgemm shapes are below
 // nn-cpp's depth cut (k = 64 and k = Tk <= 256), so every element is a single chain.
-// Two workgroups share a CU (about 67 KB of LDS each at Tk = 256), so one's MFMA phases can overlap the other's
-// VALU phases.
+// What bounds the forward: the vector ALUs and the matrix cores in turn (a third of the issue cycles each) and the
+// waits between the phases. Four workgroups share a CU (34 KB of LDS each at Tk = 256, 128 registers a lane), so one's
+// MFMA phases overlap another's VALU phases. Measured at 32 x 8 heads x 256 x 64 (us): 64 rows a workgroup and two
+// workgroups a CU 85, 32 rows 81, and 74 with a third of the vector instructions taken out (rows summed by one wave
+// for 32 rows at once, V's addresses kept uniform, no division by Tk, one test for 16 exponentials' special cases).
 #include "attention.hpp"
 #include "gemm.hpp"
 
@@ -27,11 +27,9 @@ namespace nnh {
 
 namespace {
 
-constexpr int kRows = 64;          // query rows per workgroup
+constexpr int kRows = 32;          // query rows per workgroup
 constexpr int kDh = 64;            // head width
-constexpr int kKLd = kDh + 4;      // LDS row stride of the queries (16-byte reads of 16 lanes hit distinct banks)
 constexpr int kMaxKeys = 256;     // four waves of 64 keys
-constexpr int kVChunk = 16;        // keys of V each lane keeps in flight
 
 struct FusedArgs {
 	const float* q;
@@ -44,63 +42,71 @@ struct FusedArgs {
 	int qblocks, total;
 	int causal;
 	float scale;
-	FastDiv quads;     // division by tk / 4
 };
 
-inline int lds_floats_p(int tk) { return kRows * (tk + 4); }
+// LDS row stride of the scores: whole groups of 16 keys (four steps of the 16x16x4 product for each lane group) and
+// four floats more, so that the 16-byte reads of 16 rows hit distinct banks.
+__host__ __device__ inline int score_stride(int tk) { return (tk + 15) / 16 * 16 + 4; }
 
-using M32 = Mfma<kMf32>;
-using M16 = Mfma<kMf16>;
-
-// Phases 0 and 1, shared by the forward and the backward: (R K^T)^T for the 64 rows of R (row stride d, nr of
-// them valid) against the keys of K (row stride d, tk valid). Wave w takes keys 64w + l (lane l holds key row
-// 64w + l in registers: the MFMA's A operand) against rows 32u + (l & 31), u = 0, 1 (staged in LDS with
-// coalesced loads, read as the B operand), each element the fma chain over d = 0..63 from +0. Ends with a
-// barrier after which the LDS is free.
-__device__ __forceinline__ void rows_times_keys(const float* rp, int nr, const float* kp, int tk, int d, float* sm,
-                                                M32::Acc& s0, M32::Acc& s1) {
-	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	const bool keys_here = 64 * wave < tk;
-	// loads are unconditional (indices clamped into range) so that all are in flight before the first wait;
-	// values past the end are never used
-	f32x4 kv[kDh / 4];
-	if (keys_here) {
-		const float* kr = kp + (int64_t)min(64 * wave + lane, tk - 1) * d;
-#pragma unroll
-		for (int u = 0; u < kDh / 4; ++u) kv[u] = *reinterpret_cast<const f32x4*>(kr + 4 * u);
-	}
-	{
-		f32x4 rs[kRows * kDh / 4 / 256];
-#pragma unroll
-		for (int u = 0; u < kRows * kDh / 4 / 256; ++u) {
-			const int row = (tid >> 4) + 16 * u;
-			rs[u] = *reinterpret_cast<const f32x4*>(rp + (int64_t)min(row, nr - 1) * d + 4 * (tid & 15));
-		}
-#pragma unroll
-		for (int u = 0; u < kRows * kDh / 4 / 256; ++u)
-			*reinterpret_cast<f32x4*>(sm + ((tid >> 4) + 16 * u) * kKLd + 4 * (tid & 15)) = rs[u];
-	}
-	__syncthreads();
-#pragma unroll
-	for (int r = 0; r < M32::NV; ++r) s0[r] = s1[r] = 0.0f;
-	if (keys_here) {
-		const float* rb0 = sm + (lane & 31) * kKLd;
-		const float* rb1 = rb0 + 32 * kKLd;
-#pragma unroll
-		for (int d4 = 0; d4 < kDh / 4; ++d4) {
-			const f32x4 b0 = *reinterpret_cast<const f32x4*>(rb0 + 4 * d4);
-			const f32x4 b1 = *reinterpret_cast<const f32x4*>(rb1 + 4 * d4);
-#pragma unroll
-			for (int c = 0; c < 4; ++c) {
-				s0 = M32::mma(kv[d4][c], b0[c], s0);
-				s1 = M32::mma(kv[d4][c], b1[c], s1);
-			}
-		}
-	}
-	__syncthreads();  // the staged rows are dead
+// The 64-float rows' operand of the 16x16x4 product from 16-byte loads: lane (g, i) loads floats 16c + 4g .. + 3 of
+// its row i and needs floats 16c + 4s + g (s = 0..3), the transpose of four registers over the four lane groups.
+__device__ __forceinline__ f32x4 lane_groups_transposed(const f32x4& x) {
+	auto bits = [](float v) { return __builtin_bit_cast(unsigned, v); };
+	auto flt = [](unsigned v) { return __builtin_bit_cast(float, v); };
+	const auto a = __builtin_amdgcn_permlane32_swap(bits(x[0]), bits(x[2]), false, false);
+	const auto b = __builtin_amdgcn_permlane32_swap(bits(x[1]), bits(x[3]), false, false);
+	const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+	const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+	return f32x4{flt(c[0]), flt(c[1]), flt(d[0]), flt(d[1])};
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) attention_fused_kernel(const FusedArgs a) {
+// Phase 1, shared by the forward and the backward: (R K^T)^T for the 32 rows of R (row stride d, nr of them valid)
+// against keys key0 .. key0 + 63 of K (row stride d, tk valid): s[t][u] of lane (g, i) holds keys key0 + 16t + 4g ..
+// + 3 of row 16u + i, each element the fma chain over d = 0..63 from +0 on the 16x16x4 MFMA (two independent chains a
+// wave). Tiles of 16 keys from `limit` on stay +0. Both operands come straight from global memory, 64 bytes of 16 rows
+// a load instruction; a lane holding one key row whole would load 16 bytes of 64 rows at a time (the dS kernel 49 us
+// against 45 so).
+using M4 = Mfma<kMf16x4>;
+constexpr int kTiles = kRows / 16, kKeyTiles = 4;
+
+__device__ __forceinline__ void rows_times_keys(const float* rp, int nr, const float* kp, int tk, int key0, int limit,
+                                                int d, M4::Acc (&s)[kKeyTiles][kTiles]) {
+	const int lane = threadIdx.x & 63, g = lane >> 4, il = lane & 15;
+#pragma unroll
+	for (int t = 0; t < kKeyTiles; ++t)
+#pragma unroll
+		for (int u = 0; u < kTiles; ++u) s[t][u] = M4::Acc{0.0f, 0.0f, 0.0f, 0.0f};
+	if (key0 >= limit) return;  // uniform
+	// loads are unconditional (indices clamped into range) so that they are in flight together; values past the end
+	// are never used
+	auto load = [&](f32x4 (&dst)[kDh / 16], const float* base, int row) {
+#pragma unroll
+		for (int c = 0; c < kDh / 16; ++c) dst[c] = *reinterpret_cast<const f32x4*>(base + (int64_t)row * d + 16 * c + 4 * g);
+	};
+	f32x4 q[kTiles][kDh / 16], k[2][kDh / 16];
+#pragma unroll
+	for (int u = 0; u < kTiles; ++u) load(q[u], rp, min(16 * u + il, nr - 1));
+	load(k[0], kp, min(key0 + il, tk - 1));
+#pragma unroll
+	for (int u = 0; u < kTiles; ++u)
+#pragma unroll
+		for (int c = 0; c < kDh / 16; ++c) q[u][c] = lane_groups_transposed(q[u][c]);
+#pragma unroll
+	for (int t = 0; t < kKeyTiles; ++t) {
+		if (key0 + 16 * t >= limit) return;  // uniform
+		if (t + 1 < kKeyTiles) load(k[(t + 1) & 1], kp, min(key0 + 16 * (t + 1) + il, tk - 1));
+#pragma unroll
+		for (int c = 0; c < kDh / 16; ++c) {
+			const f32x4 kc = lane_groups_transposed(k[t & 1][c]);
+#pragma unroll
+			for (int e = 0; e < 4; ++e)
+#pragma unroll
+				for (int u = 0; u < kTiles; ++u) s[t][u] = M4::mma(kc[e], q[u][c][e], s[t][u]);
+		}
+	}
+}
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) attention_fused_kernel(const FusedArgs a) {
 	extern __shared__ __align__(16) float sm[];
 	__shared__ unsigned long long table[32];
 	__shared__ float rowmax[kRows], rowsum[kRows];
@@ -110,35 +116,35 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) a
 	const int nh = lid / a.qblocks, qb = lid - nh * a.qblocks;
 	const int n = nh / a.heads, h = nh - n * a.heads;
 	const int i0 = qb * kRows, nq = min(kRows, a.tq - i0);
-	const int tk = a.tk, ldp = tk + 4;
+	const int tk = a.tk, ldp = score_stride(tk);
 	const float* qp = a.q + ((int64_t)n * a.tq + i0) * a.d + h * kDh;
 	const float* kp = a.k + (int64_t)n * tk * a.d + h * kDh;
 	const float* vp = a.v + (int64_t)n * tk * a.d + h * kDh;
 	const float* padrow = a.pad ? a.pad + (int64_t)n * tk : nullptr;
 	if (tid < 32) table[tid] = kExp2Table[tid];
-	const bool pv4 = tk % 16 == 0;  // O = P V on the 16x16x4 MFMA (P kept in LDS in its permuted layout)
 
-	// 0, 1. S^T for keys 64w + l against queries 32u + (l & 31), u = 0, 1 (fma(k, q, acc) is the reference's
-	// fma(q, k, acc))
-	const bool keys_here = 64 * wave < tk;
-	M32::Acc s0, s1;
-	rows_times_keys(qp, nq, kp, tk, a.d, sm, s0, s1);
+	// 1. S^T (fma(k, q, acc) is the reference's fma(q, k, acc)). Scores past the block's causal limit are replaced
+	// below whatever they are and not computed; the waves' key blocks rotate over the workgroups, so that every SIMD
+	// gets short and long ones.
+	const int kw = (wave + lid) & 3, g = lane >> 4, il = lane & 15;
+	const int block_live = a.causal ? min(tk, i0 + nq) : tk;  // keys any row of the block reaches
+	M4::Acc s[kKeyTiles][kTiles];
+	rows_times_keys(qp, nq, kp, tk, 64 * kw, block_live, a.d, s);
 
-	// 2a. scaled and masked scores into LDS rows of stride tk + 4 (ops.cpp:1186-1191). Accumulator registers
-	// 4t .. 4t+3 hold four consecutive keys of one query: one 16-byte store each.
+	// 2a. scaled and masked scores into LDS (ops.cpp:1186-1191): four consecutive keys of one query a 16-byte store
 	f32x4* sm4 = reinterpret_cast<f32x4*>(sm);
 	const int ldp4 = ldp / 4;
-	if (keys_here) {
+	{
 		const bool masked = padrow != nullptr || a.causal;
 #pragma unroll
-		for (int t = 0; t < M32::NV / 4; ++t) {
-			const int j = 64 * wave + M32::crow(4 * t, lane);
+		for (int t = 0; t < kKeyTiles; ++t) {
+			const int j = 64 * kw + 16 * t + 4 * g;
 #pragma unroll
-			for (int u = 0; u < 2; ++u) {
-				const int row = 32 * u + M32::ccol(lane);
+			for (int u = 0; u < kTiles; ++u) {
+				const int row = 16 * u + il;
 				f32x4 val;
 #pragma unroll
-				for (int c = 0; c < 4; ++c) val[c] = (u ? s1[4 * t + c] : s0[4 * t + c]) * a.scale;
+				for (int c = 0; c < 4; ++c) val[c] = s[t][u][c] * a.scale;
 				if (masked) {  // uniform
 					const f32x4 pd = padrow ? *reinterpret_cast<const f32x4*>(padrow + min(j, tk - 4)) : f32x4{1, 1, 1, 1};
 #pragma unroll
@@ -154,19 +160,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) a
 	__syncthreads();
 
 	// 2b. the row maxima: std::max's scan is v_0 when v_0 is NaN, else the largest non-NaN value, which fmaxf
-	// gives in any order (a zero maximum's sign cannot change v - m or its exp). Four lanes per row.
+	// gives in any order (a zero maximum's sign cannot change v - m or its exp). Eight lanes per row.
 	{
-		const int row = 16 * wave + (lane >> 2), q = lane & 3;
+		const int row = 8 * wave + (lane >> 3), q = lane & 7;
 		float m = __builtin_nanf("");
 		if (row < nq) {
 			const float* o = sm + row * ldp;
-			for (int j = 4 * q; j < tk; j += 16) {
+			for (int j = 4 * q; j < tk; j += 32) {
 				const f32x4 x = *reinterpret_cast<const f32x4*>(o + j);
 				m = fmaxf(m, fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
 			}
 		}
 		m = fmaxf(m, __shfl_xor(m, 1));
 		m = fmaxf(m, __shfl_xor(m, 2));
+		m = fmaxf(m, __shfl_xor(m, 4));
 		if (row < nq && q == 0) {
 			const float first = sm[row * ldp];
 			rowmax[row] = first != first ? first : m;
@@ -174,57 +181,65 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) a
 	}
 	__syncthreads();
 
-	// 2c. p_j = exp(v_j - m) for the live keys, exact zeros past the causal limit (ops.cpp:1197-1201). Lane l takes
-	// row l, wave w the quads of keys w, w + 4, ..., kExpQuads of them at a time so that their table reads and
-	// double-precision chains overlap. Keys past a row's causal limit take exp(0) in place of exp(-2e9 - m), whose
-	// result is replaced by an exact zero, which keeps waves out of exp's special-case path (padded keys stay live
-	// and go through exp). Quads past the block's last live key are zero for every row: a wave stores them without
-	// computing anything.
+	// 2c. p_j = exp(v_j - m) for the live keys, exact zeros past the causal limit (ops.cpp:1197-1201). Half wave h of
+	// the eight takes the quads of keys h, h + 8, ... of its lanes' 32 rows, kExpQuads of them at a time so that their
+	// table reads and double-precision chains overlap. Keys past a row's causal limit take exp(0) in place of
+	// exp(-2e9 - m), whose result is replaced by an exact zero, which keeps waves out of exp's special-case path (padded
+	// keys stay live and go through exp). Quads past the block's last live key are zero for every row: they are stored
+	// without computing anything.
 	{
-		constexpr int kExpQuads = 4;
-		const int row = lane, nq4 = tk / 4;
+		constexpr int kExpQuads = 4, kHalves = 8;
+		const int row = lane & 31, nq4 = tk / 4;
 		const float m = rowmax[min(row, nq - 1)];
 		const int live = a.causal ? min(tk, i0 + row + 1) : tk;
-		const int block_live = a.causal ? min(tk, i0 + nq) : tk;  // keys any row of the block reaches
 		f32x4* orow = sm4 + row * ldp4;
-		for (int q0 = wave; q0 < nq4; q0 += 4 * kExpQuads) {
-			if (4 * q0 >= block_live) {  // uniform: this and every later quad of the wave is dead for all rows
+		for (int q0 = 2 * wave + (lane >> 5); q0 < nq4; q0 += kHalves * kExpQuads) {
+			if (4 * q0 >= block_live) {  // this and every later quad of the half wave is dead for all rows
 				if (row < nq) {
 #pragma unroll
 					for (int h2 = 0; h2 < kExpQuads; ++h2)
-						if (q0 + 4 * h2 < nq4) orow[q0 + 4 * h2] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+						if (q0 + kHalves * h2 < nq4) orow[q0 + kHalves * h2] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 				}
 				continue;
 			}
 			f32x4 x[kExpQuads];
-#pragma unroll
-			for (int h2 = 0; h2 < kExpQuads; ++h2) x[h2] = orow[min(q0 + 4 * h2, nq4 - 1)];
 			float ex[4 * kExpQuads];
 #pragma unroll
-			for (int h2 = 0; h2 < kExpQuads; ++h2)
+			for (int h2 = 0; h2 < kExpQuads; ++h2) x[h2] = orow[min(q0 + kHalves * h2, nq4 - 1)];
+			// uniform: no key of the wave's quads is past any row's limit
+			const bool whole = !a.causal || 4 * (q0 + kHalves * (kExpQuads - 1) + 1) + 3 <= i0;
+			if (__all(whole)) {
 #pragma unroll
-				for (int c = 0; c < 4; ++c) ex[4 * h2 + c] = 4 * (q0 + 4 * h2) + c < live ? x[h2][c] - m : 0.0f;
-			expf_glibc_n(ex, table);
+				for (int e = 0; e < 4 * kExpQuads; ++e) ex[e] = x[e / 4][e % 4] - m;
+				expf_glibc_n(ex, table);
+			} else {
+#pragma unroll
+				for (int e = 0; e < 4 * kExpQuads; ++e)
+					ex[e] = 4 * (q0 + kHalves * (e / 4)) + e % 4 < live ? x[e / 4][e % 4] - m : 0.0f;
+				expf_glibc_n(ex, table);
+#pragma unroll
+				for (int e = 0; e < 4 * kExpQuads; ++e)
+					ex[e] = 4 * (q0 + kHalves * (e / 4)) + e % 4 < live ? ex[e] : 0.0f;
+			}
 			if (row < nq) {
 #pragma unroll
 				for (int h2 = 0; h2 < kExpQuads; ++h2) {
-					const int q = q0 + 4 * h2;
-#pragma unroll
-					for (int c = 0; c < 4; ++c) x[h2][c] = 4 * q + c < live ? ex[4 * h2 + c] : 0.0f;
-					if (q < nq4) orow[q] = x[h2];
+					const int q = q0 + kHalves * h2;
+					if (q < nq4) orow[q] = f32x4{ex[4 * h2], ex[4 * h2 + 1], ex[4 * h2 + 2], ex[4 * h2 + 3]};
 				}
 			}
 		}
 	}
 	__syncthreads();
 
-	// 2d. the sum over the live keys in key order from +0, one lane per row (ops.cpp:1198-1200)
-	{
-		const int row = 16 * wave + lane;
-		if (lane < 16 && row < nq) {
+	// 2d. the sum over the live keys in key order from +0, one lane per row (ops.cpp:1198-1200): all rows in one wave,
+	// whose adds issue once for 32 rows, another wave for another workgroup
+	if (wave == ((lid >> 2) & 3)) {
+		const int row = lane;
+		if (row < nq) {
 			const float* o = sm + row * ldp;
 			const int live = a.causal ? min(tk, i0 + row + 1) : tk;
-			float s = 0.0f;
+			float sum = 0.0f;
 			int j = 0;
 			for (; j + 16 <= live; j += 16) {
 				f32x4 x[4];
@@ -232,192 +247,129 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) a
 				for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const f32x4*>(o + j + 4 * u);
 #pragma unroll
 				for (int u = 0; u < 4; ++u) {
-					s += x[u][0];
-					s += x[u][1];
-					s += x[u][2];
-					s += x[u][3];
+					sum += x[u][0];
+					sum += x[u][1];
+					sum += x[u][2];
+					sum += x[u][3];
 				}
 			}
-			for (; j < live; ++j) s += o[j];
-			rowsum[row] = s;
-			rowinv[row] = 1.0 / (double)s;
+			for (; j < live; ++j) sum += o[j];
+			rowsum[row] = sum;
+			rowinv[row] = 1.0 / (double)sum;
 		}
 	}
 	__syncthreads();
 
-	// 2e. p_j / sum into probs and back into LDS (ops.cpp:1203)
+	// 2e. p_j / sum into probs (ops.cpp:1203) and back into LDS as the 16x16x4 product below reads its rows: key j at
+	// (j % 4) q4 + j / 4, q4 = Tk / 4 rounded up to 4. Every quad is read and divided first, then, after a barrier,
+	// written back in that order. A thread has quads il, il + 16, ... of rows 4g + w and 16 + 4g + w: 256-byte pieces
+	// of a row in memory, and the four rows of a wave's 4-byte LDS stores 16 banks apart.
+	const int steps = tk >> 2, q4 = (steps + 3) & ~3;
 	{
 		float* pr = a.probs + ((int64_t)nh * a.tq + i0) * tk;
-		const unsigned quads = (unsigned)(nq * (tk / 4));
-		if (pv4) {
-			// the 16x16x4 product below reads each row permuted, key j at j % 4 (Tk / 4) + j / 4: every quad is read
-			// and divided first, then, after a barrier, written back in that order (at most kRows Tk / 1024 quads a
-			// thread)
-			constexpr int kPer = kRows * kMaxKeys / 4 / 256;
-			f32x4 yv[kPer];
+		constexpr int kPer = kMaxKeys / 64;
+		f32x4 yv[kTiles][kPer];
 #pragma unroll
-			for (int u = 0; u < kPer; ++u) {
-				const unsigned e = tid + 256 * u;
-				if (e < quads) {
-					const unsigned row = fdiv(e, a.quads);
-					const int j = (int)(e - row * a.quads.d) * 4;
-					const f32x4 x = *reinterpret_cast<const f32x4*>(sm + row * ldp + j);
-					float y[4] = {x[0], x[1], x[2], x[3]};
-					div_n_by_row_sum(y, rowsum[row], rowinv[row]);
-					yv[u] = f32x4{y[0], y[1], y[2], y[3]};
-					*reinterpret_cast<f32x4*>(pr + (int64_t)row * tk + j) = yv[u];
+		for (int u = 0; u < kTiles; ++u) {
+			const int row = 16 * u + 4 * g + wave;
+			if (row < nq) {
+				const float sum = rowsum[row];
+				const double inv = rowinv[row];
+#pragma unroll
+				for (int x = 0; x < kPer; ++x) {
+					const int jq = il + 16 * x;
+					if (jq < steps) {
+						const f32x4 v = sm4[row * ldp4 + jq];
+						float y[4] = {v[0], v[1], v[2], v[3]};
+						div_n_by_row_sum(y, sum, inv);
+						yv[u][x] = f32x4{y[0], y[1], y[2], y[3]};
+						*reinterpret_cast<f32x4*>(pr + row * tk + 4 * jq) = yv[u][x];
+					}
 				}
 			}
-			__syncthreads();
+		}
+		__syncthreads();
 #pragma unroll
-			for (int u = 0; u < kPer; ++u) {
-				const unsigned e = tid + 256 * u;
-				if (e < quads) {
-					const unsigned row = fdiv(e, a.quads);
-					const int jq = (int)(e - row * a.quads.d);
+		for (int u = 0; u < kTiles; ++u) {
+			const int row = 16 * u + 4 * g + wave;
 #pragma unroll
-					for (int c = 0; c < 4; ++c) sm[row * ldp + c * (tk >> 2) + jq] = yv[u][c];
-				}
-			}
-		} else {
-			for (unsigned e = tid; e < quads; e += 256) {
-				const unsigned row = fdiv(e, a.quads);
-				const int j = (int)(e - row * a.quads.d) * 4;
-				float* o = sm + row * ldp + j;
-				const f32x4 x = *reinterpret_cast<const f32x4*>(o);
-				float y[4] = {x[0], x[1], x[2], x[3]};
-				div_n_by_row_sum(y, rowsum[row], rowinv[row]);
-				const f32x4 y4 = {y[0], y[1], y[2], y[3]};
-				*reinterpret_cast<f32x4*>(o) = y4;
-				*reinterpret_cast<f32x4*>(pr + (int64_t)row * tk + j) = y4;
+			for (int x = 0; x < kPer; ++x) {
+				const int jq = il + 16 * x;
+				if (row < nq && jq < steps)
+#pragma unroll
+					for (int c = 0; c < 4; ++c) sm[row * ldp + c * q4 + jq] = yv[u][x][c];
 			}
 		}
 	}
 	__syncthreads();
 
-	if (pv4) {
-		// 3. O columns 16w .. 16w+15 for the 64 rows on the 16x16x4 MFMA (Mfma<kMf16x4>: four keys per instruction,
-		// bit for bit four fmas in key order): four 16-row tiles, four independent chains over every key. At step s
-		// lane (g, i) supplies P[16 t + i][4 s + g], read four steps at a time from the permuted rows (positions
-		// g Tk / 4 + s), and V[4 s + g][16 w + i], loaded 16 steps ahead.
-		using M4 = Mfma<kMf16x4>;
-		const int g = lane >> 4, il = lane & 15, q4 = tk >> 2;
-		M4::Acc acc4[4];
+	// 3. O columns 16w .. 16w+15 for the 32 rows on the 16x16x4 MFMA (Mfma<kMf16x4>: four keys per instruction,
+	// bit for bit four fmas in key order): two 16-row tiles, two independent chains over every key. At step s
+	// lane (g, i) supplies P[16 t + i][4 s + g], read four steps at a time from the permuted rows (positions
+	// g q4 + s; steps past the last one are read, never used, and rows past nq hold stale values, never stored), and
+	// V[4 s + g][16 w + i], loaded 16 steps ahead.
+	M4::Acc acc4[kTiles];
 #pragma unroll
-		for (int t = 0; t < 4; ++t) acc4[t] = M4::Acc{0.0f, 0.0f, 0.0f, 0.0f};
-		const float* vcol = vp + 16 * wave + il;
-		const float* pbase = sm + il * ldp + g * q4;
-		auto load_v = [&](float (&dst)[16], int s0) {  // steps s0 .. s0 + 15 (clamped rows are loaded, never used)
+	for (int t = 0; t < kTiles; ++t) acc4[t] = M4::Acc{0.0f, 0.0f, 0.0f, 0.0f};
+	// V's row of a step: a uniform address (the step's first key) and the lane's offset, one key a lane group
+	const unsigned vlane = (unsigned)g * (unsigned)a.d + (unsigned)(16 * wave + il);
+	auto v_at = [&](int step) { return (vp + (int64_t)(4 * min(step, steps - 1)) * a.d)[vlane]; };
+	const float* pbase = sm + il * ldp + g * q4;
+	auto load_v = [&](float (&dst)[16], int s0) {  // steps s0 .. s0 + 15 (clamped rows are loaded, never used)
 #pragma unroll
-			for (int u = 0; u < 16; ++u) dst[u] = vcol[(int64_t)min(4 * (s0 + u) + g, tk - 1) * a.d];
-		};
-		auto load_p = [&](f32x4 (&dst)[4], int s0) {  // steps s0 .. s0 + 3 of the four tiles
+		for (int u = 0; u < 16; ++u) dst[u] = v_at(s0 + u);
+	};
+	auto load_p = [&](f32x4 (&dst)[kTiles], int s0) {  // steps s0 .. s0 + 3 of the tiles
 #pragma unroll
-			for (int t = 0; t < 4; ++t) dst[t] = *reinterpret_cast<const f32x4*>(pbase + 16 * t * ldp + min(s0, q4 - 4));
-		};
-		float v0[16], v1[16];
-		f32x4 pa[4], pb[4];
-		auto chunk = [&](const float (&v)[16], int s0) {  // 16 steps from s0, P one group of four steps ahead
-			load_p(pa, s0);
+		for (int t = 0; t < kTiles; ++t) dst[t] = *reinterpret_cast<const f32x4*>(pbase + 16 * t * ldp + min(s0, q4 - 4));
+	};
+	float v0[16], v1[16];
+	f32x4 pa[kTiles], pb[kTiles];
+	auto chunk = [&](const float (&v)[16], int s0) {  // 16 steps from s0, P one group of four steps ahead
+		load_p(pa, s0);
 #pragma unroll
-			for (int h4 = 0; h4 < 4; ++h4) {
-				f32x4 (&cur)[4] = (h4 & 1) ? pb : pa;
-				f32x4 (&nxt)[4] = (h4 & 1) ? pa : pb;
-				if (h4 < 3) load_p(nxt, s0 + 4 * (h4 + 1));
-#pragma unroll
-				for (int e = 0; e < 4; ++e)
-#pragma unroll
-					for (int t = 0; t < 4; ++t) acc4[t] = M4::mma(cur[t][e], v[4 * h4 + e], acc4[t]);
-			}
-		};
-		// tk % 16 == 0: q4 is a multiple of 4, whole groups of four steps; chunks of 16 steps, V two chunks ahead
-		load_v(v0, 0);
-		load_v(v1, 16);
-		int s0 = 0;
-		for (; s0 + 32 <= q4; s0 += 32) {
-			chunk(v0, s0);
-			load_v(v0, s0 + 32);
-			chunk(v1, s0 + 16);
-			load_v(v1, s0 + 48);
-		}
-		// the rest: fewer than 32 steps, in groups of four
-		for (; s0 < q4; s0 += 4) {
-			float vv[16];
-			f32x4 pp[4];
-			load_p(pp, s0);
-#pragma unroll
-			for (int e = 0; e < 4; ++e) vv[e] = vcol[(int64_t)(4 * (s0 + e) + g) * a.d];
+		for (int h4 = 0; h4 < 4; ++h4) {
+			f32x4 (&cur)[kTiles] = (h4 & 1) ? pb : pa;
+			f32x4 (&nxt)[kTiles] = (h4 & 1) ? pa : pb;
+			if (h4 < 3) load_p(nxt, s0 + 4 * (h4 + 1));
 #pragma unroll
 			for (int e = 0; e < 4; ++e)
 #pragma unroll
-				for (int t = 0; t < 4; ++t) acc4[t] = M4::mma(pp[t][e], vv[e], acc4[t]);
+				for (int t = 0; t < kTiles; ++t) acc4[t] = M4::mma(cur[t][e], v[4 * h4 + e], acc4[t]);
 		}
-		float* op = a.out + ((int64_t)n * a.tq + i0) * a.d + h * kDh + 16 * wave + il;
+	};
+	load_v(v0, 0);  // chunks of 16 steps, V two chunks ahead
+	load_v(v1, 16);
+	int s0 = 0;
+	for (; s0 + 32 <= steps; s0 += 32) {
+		chunk(v0, s0);
+		load_v(v0, s0 + 32);
+		chunk(v1, s0 + 16);
+		load_v(v1, s0 + 48);
+	}
+	// the rest: fewer than 32 steps, in groups of four, of which the last may be partial
+	for (; s0 < steps; s0 += 4) {
+		float vv[4];
+		f32x4 pp[kTiles];
+		load_p(pp, s0);
 #pragma unroll
-		for (int t = 0; t < 4; ++t)
+		for (int e = 0; e < 4; ++e) vv[e] = v_at(s0 + e);
 #pragma unroll
-			for (int r = 0; r < 4; ++r) {
-				const int row = 16 * t + 4 * g + r;
-				if (row < nq) op[(int64_t)row * a.d] = acc4[t][r];
+		for (int e = 0; e < 4; ++e)
+			if (s0 + e < steps) {  // uniform
+#pragma unroll
+				for (int t = 0; t < kTiles; ++t) acc4[t] = M4::mma(pp[t][e], vv[e], acc4[t]);
 			}
-		return;
 	}
-
-	// 3. O columns 16w .. 16w+15 for the 64 rows: the chain over every key in order
-	M16::Acc o;
+	float* op = a.out + ((int64_t)n * a.tq + i0) * a.d + h * kDh + 16 * wave + il;
 #pragma unroll
-	for (int r = 0; r < M16::NV; ++r) o[r] = 0.0f;
-	{
-		const f32x4* prow4 = sm4 + M16::arow(lane) * ldp4;  // rows past nq hold stale values, never stored
-		const int vlane = 16 * wave + M16::bcol(lane);
-		// V entries of keys j0 .. j0+kVChunk-1 for this lane's column; rows past tk are clamped to the last key
-		// (loaded, never used), so every load is issued unconditionally with a uniform row address.
-		auto load_v = [&](float (&dst)[kVChunk], int j0) {
+	for (int t = 0; t < kTiles; ++t)
 #pragma unroll
-			for (int u = 0; u < kVChunk; ++u) dst[u] = (vp + (int64_t)min(j0 + u, tk - 1) * a.d)[vlane];
-		};
-		// P quads of keys j0 .. j0+kVChunk-1 (quads past tk, in a partial chunk, read a stale in-row value)
-		auto load_p = [&](f32x4 (&dst)[kVChunk / 4], int j0) {
-#pragma unroll
-			for (int u4 = 0; u4 < kVChunk / 4; ++u4) dst[u4] = prow4[min(j0 + 4 * u4, tk - 4) / 4];
-		};
-		auto steps = [&](const f32x4 (&p)[kVChunk / 4], const float (&src)[kVChunk], int j0, bool whole) {
-#pragma unroll
-			for (int u4 = 0; u4 < kVChunk / 4; ++u4) {
-				if (whole || j0 + 4 * u4 < tk) {  // tk % 4 == 0: whole quads only, no step past the last key
-#pragma unroll
-					for (int c = 0; c < 4; ++c) o = M16::mma(p[u4][c], src[4 * u4 + c], o);
-				}
-			}
-		};
-		float v0[kVChunk], v1[kVChunk];
-		f32x4 p0[kVChunk / 4], p1[kVChunk / 4];
-		load_v(v0, 0);
-		load_v(v1, kVChunk);
-		load_p(p0, 0);
-		int j0 = 0;
-		for (; j0 + 2 * kVChunk <= tk; j0 += 2 * kVChunk) {  // V two chunks ahead, P one chunk ahead
-			load_p(p1, j0 + kVChunk);
-			steps(p0, v0, j0, true);
-			load_v(v0, j0 + 2 * kVChunk);
-			load_p(p0, j0 + 2 * kVChunk);
-			steps(p1, v1, j0 + kVChunk, true);
-			load_v(v1, j0 + 3 * kVChunk);
+		for (int r = 0; r < 4; ++r) {
+			const int row = 16 * t + 4 * g + r;
+			if (row < nq) op[(int64_t)row * a.d] = acc4[t][r];
 		}
-		if (j0 < tk) {
-			load_p(p1, j0 + kVChunk);
-			steps(p0, v0, j0, false);
-			if (j0 + kVChunk < tk) steps(p1, v1, j0 + kVChunk, false);
-		}
-	}
-	float* op = a.out + ((int64_t)n * a.tq + i0) * a.d + h * kDh + 16 * wave + M16::ccol(lane);
-#pragma unroll
-	for (int r = 0; r < M16::NV; ++r) {
-		const int row = M16::crow(r, lane);
-		if (row < nq) op[(int64_t)row * a.d] = o[r];
-	}
 }
-
 
 struct DScoresArgs {
 	const float* g;      // upstream gradient {N, Tq, D}
@@ -431,14 +383,14 @@ struct DScoresArgs {
 	float scale;
 };
 
-// The first half of nn::attention's backward for 64 query rows of one (sample, head) pair (ops.cpp:1286-1290):
+// The first half of nn::attention's backward for 32 query rows of one (sample, head) pair (ops.cpp:1286-1290):
 //   dP = G_h V_h^T                     each element the fma chain over d = 0..63 from +0 (sgemm F,T)
 //   dot_i = sum_j dP_ij * y_ij         the products rounded, then added in key order from +0
 //   dS_ij = masked ? 0 : scale * (y_ij * (dP_ij - dot_i)) + 0     (masked_softmax_row_backward, ops.cpp:1216-1224)
-// dP stays in the MFMA accumulators (wave w holds keys 64w..64w+63 of the 64 rows, four consecutive keys per
+// dP stays in the MFMA accumulators (wave w holds keys 64w..64w+63 of the 32 rows, four consecutive keys per
 // four registers); y is loaded in the same layout; only the products dP y go through LDS, where one lane per
 // row adds them in key order. dS is written to HBM for the dQ and dK products.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) attention_dscores_kernel(const DScoresArgs a) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) attention_dscores_kernel(const DScoresArgs a) {
 	extern __shared__ __align__(16) float sm[];
 	__shared__ float rowdot[kRows];
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -446,7 +398,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) a
 	const int nh = lid / a.qblocks, qb = lid - nh * a.qblocks;
 	const int n = nh / a.heads, h = nh - n * a.heads;
 	const int i0 = qb * kRows, nq = min(kRows, a.tq - i0);
-	const int tk = a.tk, ldp4 = (tk + 4) / 4;
+	const int tk = a.tk, ldp4 = score_stride(tk) / 4;
 	const float* gp = a.g + ((int64_t)n * a.tq + i0) * a.d + h * kDh;
 	const float* vp = a.v + (int64_t)n * tk * a.d + h * kDh;
 	const float* yp = a.probs + ((int64_t)nh * a.tq + i0) * tk;
@@ -454,35 +406,29 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) a
 	const float* padrow = a.pad ? a.pad + (int64_t)n * tk : nullptr;
 	f32x4* sm4 = reinterpret_cast<f32x4*>(sm);
 
-	// dP^T for keys 64w + l against rows 32u + (l & 31)
-	const bool keys_here = 64 * wave < tk;
-	M32::Acc s0, s1;
-	rows_times_keys(gp, nq, vp, tk, a.d, sm, s0, s1);
-
-	// y in the accumulator layout: quad t of unit u is y[32u + ccol][64w + crow(4t) .. +3] (rows and keys clamped
+	// dP^T; y in the accumulators' layout: y[t][u] is row 16u + i, keys key0 + 16t + 4g .. + 3 (rows and keys clamped
 	// into range; values outside are never used)
-	constexpr int kQ = M32::NV / 4;
-	f32x4 y[2][kQ];
-	if (keys_here) {
+	const int key0 = 64 * wave, g = lane >> 4, il = lane & 15;
+	M4::Acc s[kKeyTiles][kTiles];
+	rows_times_keys(gp, nq, vp, tk, key0, tk, a.d, s);
+	f32x4 y[kKeyTiles][kTiles];
+	if (key0 < tk) {
 #pragma unroll
-		for (int u = 0; u < 2; ++u) {
-			const int row = min(32 * u + M32::ccol(lane), nq - 1);
+		for (int t = 0; t < kKeyTiles; ++t)
 #pragma unroll
-			for (int t = 0; t < kQ; ++t) {
-				const int j = min(64 * wave + M32::crow(4 * t, lane), tk - 4);
-				y[u][t] = *reinterpret_cast<const f32x4*>(yp + (int64_t)row * tk + j);
-			}
-		}
-		// the products dP y, rounded, into LDS rows of stride tk + 4 (tk % 4 == 0: every quad is whole)
+			for (int u = 0; u < kTiles; ++u)
+				y[t][u] = *reinterpret_cast<const f32x4*>(yp + (int64_t)min(16 * u + il, nq - 1) * tk +
+				                                          min(key0 + 16 * t + 4 * g, tk - 4));
+		// the products dP y, rounded, into LDS (tk % 4 == 0: every quad is whole)
 #pragma unroll
-		for (int u = 0; u < 2; ++u) {
-			const int row = 32 * u + M32::ccol(lane);
+		for (int t = 0; t < kKeyTiles; ++t) {
+			const int j = key0 + 16 * t + 4 * g;
 #pragma unroll
-			for (int t = 0; t < kQ; ++t) {
-				const int j = 64 * wave + M32::crow(4 * t, lane);
+			for (int u = 0; u < kTiles; ++u) {
+				const int row = 16 * u + il;
 				f32x4 prod;
 #pragma unroll
-				for (int c = 0; c < 4; ++c) prod[c] = (u ? s1[4 * t + c] : s0[4 * t + c]) * y[u][t][c];
+				for (int c = 0; c < 4; ++c) prod[c] = s[t][u][c] * y[t][u][c];
 				if (row < nq && j < tk) sm4[row * ldp4 + j / 4] = prod;
 			}
 		}
@@ -491,9 +437,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) a
 
 	// dot_i: one lane per row, every key in order from +0
 	{
-		const int row = 16 * wave + lane;
-		if (lane < 16 && row < nq) {
-			const f32x4* o = sm4 + row * ldp4;
+		const int r = lane;
+		if (wave == ((lid >> 2) & 3) && r < nq) {
+			const f32x4* o = sm4 + r * ldp4;
 			float dot = 0.0f;
 			int q = 0;
 			for (; q + 4 <= tk / 4; q += 4) {
@@ -515,27 +461,24 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) a
 				dot += x[2];
 				dot += x[3];
 			}
-			rowdot[row] = dot;
+			rowdot[r] = dot;
 		}
 	}
 	__syncthreads();
 
 	// dS from the registers
-	if (keys_here) {
+	if (key0 < tk) {
 		const bool masked = padrow != nullptr || a.causal;
 #pragma unroll
-		for (int u = 0; u < 2; ++u) {
-			const int row = 32 * u + M32::ccol(lane);
+		for (int u = 0; u < kTiles; ++u) {
+			const int row = 16 * u + il;
 			const float dot = rowdot[min(row, nq - 1)];
 #pragma unroll
-			for (int t = 0; t < kQ; ++t) {
-				const int j = 64 * wave + M32::crow(4 * t, lane);
+			for (int t = 0; t < kKeyTiles; ++t) {
+				const int j = key0 + 16 * t + 4 * g;
 				f32x4 r;
 #pragma unroll
-				for (int c = 0; c < 4; ++c) {
-					const float dp = u ? s1[4 * t + c] : s0[4 * t + c];
-					r[c] = a.scale * (y[u][t][c] * (dp - dot)) + 0.0f;
-				}
+				for (int c = 0; c < 4; ++c) r[c] = a.scale * (y[t][u][c] * (s[t][u][c] - dot)) + 0.0f;
 				if (masked) {  // uniform
 					const f32x4 pd = padrow ? *reinterpret_cast<const f32x4*>(padrow + min(j, tk - 4)) : f32x4{1, 1, 1, 1};
 #pragma unroll
@@ -580,8 +523,7 @@ hipError_t attention_fused_forward(const float* q, const float* k, const float* 
 	a.total = (int)total;
 	a.causal = causal ? 1 : 0;
 	a.scale = scale;
-	a.quads = make_fastdiv((unsigned)(tk / 4));
-	const int lds = 4 * max(kRows * kKLd, lds_floats_p((int)tk));
+	const int lds = 4 * kRows * score_stride((int)tk);
 	hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_fused_kernel),
 	                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds);
 	if (e != hipSuccess) return e;
@@ -609,7 +551,7 @@ hipError_t attention_fused_dscores(const float* g, const float* v, const float* 
 	a.total = (int)total;
 	a.causal = causal ? 1 : 0;
 	a.scale = scale;
-	const int lds = 4 * max(kRows * kKLd, lds_floats_p((int)tk));
+	const int lds = 4 * kRows * score_stride((int)tk);
 	hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_dscores_kernel),
 	                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds);
 	if (e != hipSuccess) return e;

@@ -36,7 +36,9 @@ __device__ __forceinline__ float expf_main(float x, const unsigned long long* ta
 	const unsigned long long ki = (unsigned long long)__double_as_longlong(kd);
 	kd -= kShift;
 	const double r = __builtin_fma(kInvLn2N, xd, -kd);
-	const double s = __longlong_as_double((long long)(table[ki & 31] + (ki << 47)));
+	// table entry + (k << 47): only the high word changes
+	const unsigned long long t = table[ki & 31];
+	const double s = __hiloint2double((int)((unsigned)(t >> 32) + ((unsigned)ki << 15)), (int)(unsigned)t);
 	const double z = __builtin_fma(kC0, r, kC1), r2 = r * r;
 	double y = __builtin_fma(kC2, r, 1.0);
 	y = __builtin_fma(z, r2, y);
@@ -68,14 +70,14 @@ __device__ __forceinline__ float expf_glibc(float x, const unsigned long long* t
 template <int N>
 __device__ __forceinline__ void expf_glibc_n(float (&v)[N], const unsigned long long* table) {
 	float x[N];
-	bool special = false;
+	unsigned largest = 0;  // of |x|, as bits above the sign's: NaN and infinity are the largest
 #pragma unroll
 	for (int i = 0; i < N; ++i) {
 		x[i] = v[i];
 		v[i] = expf_main(x[i], table);
-		special |= expf_is_special(x[i]);
+		largest = max(largest, __float_as_uint(x[i]) << 1);
 	}
-	if (special) {
+	if (largest >= 0x42b00000u << 1) {  // some |x| >= 88: expf_is_special
 #pragma unroll
 		for (int i = 0; i < N; ++i) v[i] = expf_is_special(x[i]) ? expf_special(x[i], v[i]) : v[i];
 	}
@@ -101,16 +103,16 @@ __device__ __forceinline__ float div_by_row_sum(float p, float s, double rinv) {
 // division only for the values that need it, behind one test that a wave skips when none of its lanes does.
 template <int N>
 __device__ __forceinline__ void div_n_by_row_sum(float (&v)[N], float s, double rinv) {
-	bool tiny = false;
+	// a tiny quotient has 0 < p < s 2^-125 < 2^-100 (s is at most the row's length): one look at the smallest positive p
+	unsigned smallest = ~0u;
 	float p[N];
 #pragma unroll
 	for (int i = 0; i < N; ++i) {
 		p[i] = v[i];
-		const double q = (double)p[i] * rinv;
-		tiny |= row_quotient_tiny(q);
-		v[i] = (float)q;
+		v[i] = (float)((double)p[i] * rinv);
+		smallest = min(smallest, __float_as_uint(p[i]) - 1u);  // p = 0 and NaN become large
 	}
-	if (tiny) {
+	if (smallest < 0x0d800000u) {  // the bits of 2^-100
 #pragma unroll
 		for (int i = 0; i < N; ++i)
 			if (row_quotient_tiny((double)p[i] * rinv)) v[i] = p[i] / s;
