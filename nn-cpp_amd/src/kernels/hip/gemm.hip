@@ -340,6 +340,12 @@ hipError_t gemm_launch_pair(const GemmCall& g0, const GemmCall& g1, hipStream_t 
 		launched = e == hipSuccess;
 		return e;
 	}
+	// two products of some hundred 32 x 32 tiles on the ring kernel
+	if (ring_pair_takes(g0, g1)) {
+		hipError_t e = gemm_ring_pair_launch(g0, g1, s);
+		launched = e == hipSuccess;
+		return e;
+	}
 	// g0 = A B and g1 = A^T B (row sums allowed), single matrices, no depth cut, both on one configuration that
 	// has the pair kernels
 	if (g0.ta || g0.tb || g0.gather || g0.rowsum || !g1.ta || g1.tb || g1.gather || g1.rowsum_outer > 0) return hipSuccess;

@@ -99,6 +99,8 @@ bool ring_ok(const GemmCall& g);
 bool ring_takes(const GemmCall& g);        // the shapes it is routed for (measured)
 bool ring_takes_large(const GemmCall& g);  // those of them that take 64 x 64 tiles or larger
 hipError_t gemm_ring_launch(const GemmCall& g, hipStream_t s, int config = -1);
+bool ring_pair_takes(const GemmCall& g0, const GemmCall& g1);  // an A B or A B^T and an A^T B in one grid
+hipError_t gemm_ring_pair_launch(const GemmCall& g0, const GemmCall& g1, hipStream_t s);
 const char* ring_config_name(int config);
 // A B on the chain kernel and A^T B (row sums allowed) on the pieces kernel in one launch (gemm_pieces.hip): single
 // matrices, each taken by its own kernel's route (chain4_takes, a depth cut and pieces4_takes) and at most

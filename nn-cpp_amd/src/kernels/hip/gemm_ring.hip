@@ -38,6 +38,11 @@ hipError_t prepare_ring() {
 				if (e != hipSuccess) return e;
 			}
 	}
+	for (int i = 0; i < 12; ++i) {
+		e = hipFuncSetAttribute(reinterpret_cast<const void*>(ring_pair_32x32(i / 4, (i / 2) & 1, i & 1)),
+		                        hipFuncAttributeMaxDynamicSharedMemorySize, ring_configs()[kRing32x32].lds_bytes);
+		if (e != hipSuccess) return e;
+	}
 	done[dev] = true;
 	return hipSuccess;
 }
@@ -124,17 +129,17 @@ bool ring_takes(const GemmCall& g) {
 	// 7.1); whole aligned A B^T tiles stay where they are (512^3 7.3 us against 8.0, 64 x 4096 x 4096 33.6 against 38).
 	if (!ring_ok(g) || g.k < 128 || narrow(g)) return false;
 	const double tiles = (double)((g.m + 31) / 32) * (double)((g.n + 31) / 32) * (double)g.batch_count;
-	if (tiles < 64) return false;
+	// few outputs with row sums have no other pipelined kernel (the backward of a 256 -> 10 layer at 256 rows, its dX 4 us of
+	// it: 13.2 us with dW on the tile kernel, 11.1 here)
+	if (tiles < 64) return g.rowsum != nullptr;
 	if (g.ta && !g.tb) return true;
 	const bool whole = ring_vec(g) && g.m % 32 == 0 && g.n % 32 == 0 && g.k % 64 == 0 && g.ldc % 4 == 0 && aligned16(g.c);
 	return !whole || (!g.ta && !g.tb && tiles <= 256);
 }
 
-hipError_t gemm_ring_launch(const GemmCall& g, hipStream_t s, int config) {
-	if (!ring_ok(g)) return hipErrorInvalidValue;
-	hipError_t e = prepare_ring();
-	if (e != hipSuccess) return e;
-	const RingConfig& c = ring_configs()[config >= 0 ? config : ring_pick(g)];
+namespace {
+
+GemmArgs ring_args(const GemmCall& g, const RingConfig& c) {
 	GemmArgs p{};
 	p.a = g.a;
 	p.b = g.b;
@@ -158,12 +163,49 @@ hipError_t gemm_ring_launch(const GemmCall& g, hipStream_t s, int config) {
 	bool c_vec = g.ldc % 4 == 0 && aligned16(g.c) && (!g.ep.gelu_y || (aligned16(g.ep.gelu_y) && aligned16(g.ep.gelu_t)));
 	for (int d = 0; d < g.batch.ndim; ++d) c_vec = c_vec && g.batch.sc[d] % 4 == 0;
 	p.c_vec = c_vec ? 1 : 0;
+	return p;
+}
+
+}  // namespace
+
+hipError_t gemm_ring_launch(const GemmCall& g, hipStream_t s, int config) {
+	if (!ring_ok(g)) return hipErrorInvalidValue;
+	hipError_t e = prepare_ring();
+	if (e != hipSuccess) return e;
+	const RingConfig& c = ring_configs()[config >= 0 ? config : ring_pick(g)];
+	const GemmArgs p = ring_args(g, c);
 	const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * p.batch_count;
 	if (blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
 	if (g.ep.gelu_y && (g.ta || !g.tb || g.rowsum)) return hipErrorInvalidValue;
 	const int v = ring_vec(g) ? 1 : 0;
 	const auto fn = g.ep.gelu_y ? c.gelu_fn[v] : g.rowsum ? c.rowsum_fn[v] : c.fn[(g.ta ? 2 : 0) + (g.tb ? 1 : 0)][v];
 	hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3((unsigned)c.threads), (size_t)c.lds_bytes, s, p);
+	return hipGetLastError();
+}
+
+bool ring_pair_takes(const GemmCall& g0, const GemmCall& g1) {
+	// A product's dX (or dA) and dW (or dB), each with fewer 64 x 64 tiles than the chip takes: on 32 x 32 tiles side by
+	// side, one's workgroups fill the CUs that the other leaves idle. Backward passes over M rows of a K -> N layer (us, two
+	// launches or the tile kernel's pair before): matmul 512, 512, 512 14.1 -> 10.6, 256, 512, 256 9.9 -> 6.4, 300, 900, 130 15.4 ->
+	// 9.3, 640, 640, 256 13.9 -> 12.9; linear with its bias 512, 512, 512 18.6 -> 13.6, 256, 784, 512 13.4 -> 11.3, 200, 300, 500
+	// 11.6 -> 8.1. Below 64 tiles of a product or 128 deep the chain kernels' pairs and the tile pair stay.
+	if (g0.ta || !g1.ta || g1.tb || !ring_ok(g0) || !ring_ok(g1) || g0.rowsum || g0.ep.gelu_y || g1.ep.gelu_y) return false;
+	if (g0.tb && g1.rowsum) return false;  // not compiled: a linear layer's dX is an A B
+	if (g0.batch_count != 1 || g1.batch_count != 1 || g0.batch.ndim != 0 || g1.batch.ndim != 0) return false;
+	if (g0.k < 128 || g1.k < 128 || ring_takes_large(g0) || ring_takes_large(g1)) return false;
+	auto tiles = [](const GemmCall& g) { return (double)((g.m + 31) / 32) * (double)((g.n + 31) / 32); };
+	return tiles(g0) >= 64 && tiles(g1) >= 64;
+}
+
+hipError_t gemm_ring_pair_launch(const GemmCall& g0, const GemmCall& g1, hipStream_t s) {
+	if (!ring_pair_takes(g0, g1)) return hipErrorInvalidValue;
+	hipError_t e = prepare_ring();
+	if (e != hipSuccess) return e;
+	const RingConfig& c = ring_configs()[kRing32x32];
+	const GemmArgs p0 = ring_args(g0, c), p1 = ring_args(g1, c);
+	const int b0 = p0.tiles_m * p0.tiles_n, b1 = p1.tiles_m * p1.tiles_n;  // below 176 x 4 each
+	const auto fn = ring_pair_32x32(g0.tb ? 2 : g1.rowsum ? 1 : 0, ring_vec(g0) ? 1 : 0, ring_vec(g1) ? 1 : 0);
+	hipLaunchKernelGGL(fn, dim3((unsigned)(b0 + b1)), dim3((unsigned)c.threads), (size_t)c.lds_bytes, s, p0, p1, b0);
 	return hipGetLastError();
 }
 

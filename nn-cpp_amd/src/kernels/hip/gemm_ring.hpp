@@ -466,6 +466,16 @@ __attribute__((amdgpu_waves_per_eu(WPE, WPE))) sgemm_ring_kernel(const GemmArgs 
 	ring_tile<BM, BN, BK, WM, WN, ST, TA, TB, V, EXTRA>(p, (int)blockIdx.x);
 }
 
+// Two products in one grid on the same tile: A B or A B^T (workgroups 0 .. blocks0 - 1) and an A^T B, with or without
+// row sums.
+template <int BM, int BN, int BK, int WM, int WN, int ST, int WPE, bool TB0, int V0, int V1, int EXTRA1>
+__global__ void __launch_bounds__((RingShape<BM, BN, BK, WM, WN, ST, false, TB0, V0>::kThreads))
+__attribute__((amdgpu_waves_per_eu(WPE, WPE))) sgemm_ring_pair_kernel(const GemmArgs p0, const GemmArgs p1, int blocks0) {
+	const int block = (int)blockIdx.x;
+	if (block < blocks0) ring_tile<BM, BN, BK, WM, WN, ST, false, TB0, V0, kRingPlain>(p0, block);
+	else ring_tile<BM, BN, BK, WM, WN, ST, true, false, V1, EXTRA1>(p1, block - blocks0);
+}
+
 // One compiled tile shape of the ring kernel: its kernels by layout (ta * 2 + tb) and by the load width.
 struct RingConfig {
 	const char* name;
@@ -500,6 +510,9 @@ RingConfig make_ring_config(const char* name) {
 #undef NNH_RING
 	return c;
 }
+
+using RingPairFn = void (*)(const GemmArgs, const GemmArgs, int);
+RingPairFn ring_pair_32x32(int kind, int v0, int v1);  // kind 0: A B, 1: A B with row sums of the other, 2: A B^T
 
 RingConfig ring_config_256x128();
 RingConfig ring_config_128x128();

@@ -82,3 +82,29 @@ def test_ring_batches(gpu, oracle, shape):
     for i in range(nb):
         want = oracle.sgemm(0, 0, m, n, k, a[i], k, b[i], n, np.zeros((m, n), np.float32), n, 0)
         assert_same(got[i], want, (shape, i))
+
+
+@pytest.mark.parametrize("M,K,n", [(256, 256, 256), (255, 260, 253), (128, 517, 130), (300, 900, 131), (640, 324, 256),
+                                   (250, 33, 7), (129, 96, 10)])
+@pytest.mark.parametrize("first", [True, False])
+def test_ring_pairs(gpu, oracle, M, K, n, first):
+    """Both gradients of a layer in one grid (the smallest sizes: dW with its row sums on a few tiles), 16-byte and 4-byte
+    loads, fresh and added, with and without the bias."""
+    import torch
+
+    import nnh
+    x, w, g = synth.normal(31, (M, K)), synth.normal(32, (n, K)), synth.normal(33, (M, n))
+    dx0, dw0, db0 = synth.normal(34, (M, K)), synth.normal(35, (n, K)), synth.normal(36, (n,))
+    xd, wd, gd = (torch.from_numpy(a).cuda() for a in (x, w, g))
+    want = oracle.linear_backward(g, x, w, dx=dx0, dx_first=first, dw=dw0, dw_first=first, db=db0, db_first=first)
+    for bias in (True, False):
+        dx, dw, db = (torch.from_numpy(a).cuda() for a in (dx0, dw0, db0))
+        nnh.linear_backward(gd, xd, wd, dx=dx, dx_first=first, dw=dw, dw_first=first, db=db if bias else None, db_first=first)
+        for got, ref, what in ((dx, want[0], "dx"), (dw, want[1], "dw"), (db, want[2] if bias else db0, "db")):
+            assert_same(host(got), ref, (what, M, K, n, first, bias))
+    b = np.ascontiguousarray(w.T)  # the same product as a matmul: dA = G B^T, dB = A^T G
+    da, dbm = (torch.from_numpy(a).cuda() for a in (dx0, np.ascontiguousarray(dw0.T)))
+    nnh.matmul_backward(gd, xd, torch.from_numpy(b).cuda(), da=da, da_first=first, db=dbm, db_first=first)
+    want = oracle.linear_backward(g, x, w, dx=dx0, dx_first=first, dw=dw0, dw_first=first)
+    assert_same(host(da), want[0], ("da", M, K, n, first))
+    assert_same(host(dbm), want[1].T, ("db matmul", M, K, n, first))
