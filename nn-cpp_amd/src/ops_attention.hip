@@ -1,6 +1,6 @@
 // ops_attention.hip - extern "C" entry points of nn::attention and nn::scaled_masked_softmax (include/nnh.h).
 //
-// Forward (src/autograd/ops.cpp:1226-1261): for heads of width 64 and Tk <= 256, one fused kernel per 64 query
+// Forward (src/autograd/ops.cpp:1226-1261): for heads of width 64 and Tk <= 256, one fused kernel per 32 query
 // rows (kernels/hip/attention.hip). Otherwise three launches over all (sample, head) pairs at once:
 //   probs = Q_h K_h^T   (batched sgemm F,T with two-level batch addressing n*T*D + h*Dh, row stride D)
 //   probs = masked_softmax_row(probs) per row
