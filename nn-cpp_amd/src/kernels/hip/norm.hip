@@ -5,9 +5,9 @@
 // lane_sum of row (n, c) (eight float partial sums over the row, combined as ((a0+a1)+(a2+a3))+((a4+a5)+(a6+a7)),
 // then the tail), divides by N*S, and does the same with lane_sq around the mean. Here:
 //   * bn_rows_kernel computes the per-row float sums (lane_sum, lane_sq, or the backward's masked lane_sum and
-//     lane_dot): a workgroup owns four rows of one channel; all its threads form the terms from wide coalesced
-//     loads and put them in LDS, and wave 0 runs the reference's eight lane chains per row over LDS (lane 8r + k is
-//     partial a[k] of row r), combines them and adds the tail in order.
+//     lane_dot): a workgroup owns 4, 8 or 32 rows of one channel; all its threads form the terms from wide coalesced
+//     loads and put them in LDS, and the reference's eight lane chains per row run over LDS (thread 8r + k is
+//     partial a[k] of row r), combine and add the tail in order.
 //   * The channel-level double sums over n run in order in one thread of every workgroup that needs them (the
 //     rows' sums are staged in LDS first), so the channel's statistics come with each workgroup's own prologue
 //     instead of a launch of their own.
@@ -27,6 +27,9 @@ namespace nnh {
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Workgroups of 256 threads in one launch: HIP takes fewer than 2^32 work-items a dimension.
+constexpr int64_t kMaxGrid = ((int64_t)1 << 24) - 1;
 
 // acc + v[0] + v[1] + ... + v[n - 1] in order; v is 16-byte aligned LDS.
 __device__ __forceinline__ float lds_chain(const float* v, int n, float acc = 0.0f) {
@@ -62,9 +65,17 @@ __device__ __forceinline__ float lds_chain(const float* v, int n, float acc = 0.
 // k, k + 8, k + 16, ... of a row lie back to back (kPart apart), so that its lane adds them from 16-byte reads. kPart is 8
 // mod 16: both the staging's four-byte stores (two partials, 32 positions) and the chains' reads (eight partials) then use
 // different banks.
-constexpr int kRows = 4, kChunk = 2304, kPart = kChunk / 8 + 8, kRowLds = 8 * kPart;
-constexpr int kRowTail = 8;  // a row's last S mod 8 terms, after the partials
-constexpr int kRowSet = kRows * (kRowLds + kRowTail);
+template <int ROWS, int CHUNK>
+struct BnRowShape {
+	static constexpr int kRows = ROWS, kChunk = CHUNK;
+	static constexpr int kPart = (CHUNK / 8 + 7) / 16 * 16 + 8, kRowLds = 8 * kPart;
+	static constexpr int kRowTail = 8;  // a row's last S mod 8 terms, after the partials
+	static constexpr int kRowSet = ROWS * (kRowLds + kRowTail);
+	static_assert(CHUNK % 8 == 0 && kPart >= CHUNK / 8 && 8 * ROWS <= 256, "eight partials a row, a thread each");
+};
+using BnLong = BnRowShape<4, 2304>;
+using BnMedium = BnRowShape<8, 1024>;
+using BnShort = BnRowShape<32, 128>;
 
 enum BnRowMode { kSum = 0, kSq = 1, kBwd = 2 };
 
@@ -78,8 +89,8 @@ struct BnRowArgs {
 	float* out1;                  // kBwd: lane_dot of masked g with x - mean
 	float* mean_out;              // kSq: the channel mean, written by the channel's first workgroup
 	int64_t N, C, S;
-	int64_t groups;               // workgroups per channel: ceil(N / kRows)
-	int64_t first_block;          // of this launch (a grid holds 2^31 - 1)
+	int64_t groups;               // workgroups per channel: ceil(N / rows)
+	int64_t first_block;          // of this launch
 	double dm;
 	FastDiv whole, last;          // units of a row in a whole chunk and in the last one
 };
@@ -132,21 +143,26 @@ __device__ void channel_dsums(const float* v0, const float* v1, int64_t N, int64
 }
 
 // lane_sum (ops.cpp:804-812), lane_sq (824-834), and the backward's lane_sum / lane_sum_masked with lane_dot /
-// lane_dot_masked (848-897) of four rows (n0 .. n0 + 3) of channel c per workgroup. All threads load the rows (16-byte
+// lane_dot_masked (848-897) of SH::kRows rows of channel c per workgroup. All threads load the rows (16-byte
 // loads with VEC: S % 4 == 0, aligned rows), form the terms the chains add (x, (x - mean)^2, or the masked g and g (x -
-// mean)) and put them in LDS; lane 8 r + k of wave 0 (the backward's second sum: lane 32 + 8 r + k) adds partial k of row
-// r, about 7 cycles a term, then the eight partials combine and the row's tail follows in order. Rows longer than kChunk
-// go chunk by chunk, the next chunk's loads in flight during the chains. Measured at [64, 16, 48, 48] (9.4 MB): sums 9.4 ->
-// 6.3 us, squares 10.4 -> 7.4, backward 27.3 -> 7.6, against eight rows a workgroup (128 of them), element-wise work in the
-// chain lanes and three exposed chunk loads.
-template <int MODE, bool VEC>
+// mean)) and put them in LDS; thread 8 r + k (the backward's second sum: those after the first sum's, or the same one where
+// they fill the workgroup) adds partial k of row r, about 7 cycles a term, then the eight partials combine and the row's
+// tail follows in order. Rows longer than kChunk go chunk by chunk, the next chunk's loads in flight during the chains.
+// Measured at [64, 16, 48, 48] (9.4 MB): sums 9.4 -> 6.3 us, squares 10.4 -> 7.4, backward 27.3 -> 7.6, against eight rows
+// a workgroup (128 of them), element-wise work in the chain lanes and three exposed chunk loads.
+template <int MODE, bool VEC, class SH>
 __global__ void __launch_bounds__(256) bn_rows_kernel(const BnRowArgs a) {
+	constexpr int kRows = SH::kRows, kChunk = SH::kChunk, kPart = SH::kPart, kRowLds = SH::kRowLds;
+	constexpr int kRowTail = SH::kRowTail, kRowSet = SH::kRowSet;
 	extern __shared__ __align__(16) float lds[];  // a set of terms, and with kBwd a second one
 	__shared__ float buf[2][256];
 	__shared__ double bcast[2];
 	constexpr int kW = VEC ? 4 : 1;                        // floats of a unit
 	constexpr int kPer = kRows * kChunk / kW / 256;        // units a thread holds
-	constexpr int kBatch = VEC ? kPer : 18;                // of them in flight at once
+	constexpr int kBatch = VEC ? kPer : kPer % 18 == 0 ? 18 : 16;  // of them in flight at once
+	static_assert(kPer * 256 * kW == kRows * kChunk && kPer % kBatch == 0, "a chunk splits evenly over the threads");
+	constexpr int kSets = MODE == kBwd ? 2 : 1, kSetThreads = 8 * kRows;
+	constexpr int kMine = kSets * kSetThreads <= 256 ? 1 : kSets;  // chains of a thread
 	const int tid = threadIdx.x;
 	const int64_t blk = a.first_block + blockIdx.x;
 	const int64_t c = blk / a.groups, j = blk - c * a.groups;
@@ -225,10 +241,10 @@ __global__ void __launch_bounds__(256) bn_rows_kernel(const BnRowArgs a) {
 		mu = a.mean[c];
 	}
 	if (nrows <= 0) return;
-	const int which = (tid >> 5) & 1, r = (tid >> 3) & 3, k = tid & 7;
-	const bool adds = tid < 64 && r < nrows && (which == 0 || MODE == kBwd);
+	const int which = kMine == 1 ? tid / kSetThreads : 0, r = (tid % kSetThreads) >> 3, k = tid & 7;
+	const bool adds = which < kSets && r < nrows;
 	const float* set = lds + which * kRowSet;
-	float acc = 0.0f;
+	float acc[kMine] = {};
 	for (int64_t s0 = 0; s0 < a.S; s0 += kChunk) {
 		const int tot = units(s0);
 		if constexpr (VEC) {
@@ -244,20 +260,23 @@ __global__ void __launch_bounds__(256) bn_rows_kernel(const BnRowArgs a) {
 		if (adds) {
 			const int64_t left = full - s0;
 			const int n = (int)(left < kChunk ? (left > 0 ? left : 0) : kChunk) / 8;
-			acc = lds_chain(set + r * kRowLds + k * kPart, n, acc);
+#pragma unroll
+			for (int i = 0; i < kMine; ++i) acc[i] = lds_chain(set + i * kRowSet + r * kRowLds + k * kPart, n, acc[i]);
 		}
 		__syncthreads();
 	}
-	if (tid >= 64) return;
 	// the partials combine as ((a0 + a1) + (a2 + a3)) + ((a4 + a5) + (a6 + a7)), then the tail in order
-	float p[8];
 #pragma unroll
-	for (int u = 0; u < 8; ++u) p[u] = __shfl(acc, (tid & ~7) + u);
-	if (!adds || k != 0) return;
-	float t = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
-	const float* tail = set + kRows * kRowLds + r * kRowTail;
-	for (int l = 0; l < (int)(a.S - full); ++l) t = t + tail[l];
-	(which == 0 ? a.out0 : a.out1)[row0 + r * a.C] = t;
+	for (int i = 0; i < kMine; ++i) {
+		float p[8];
+#pragma unroll
+		for (int u = 0; u < 8; ++u) p[u] = __shfl(acc[i], (tid & 56) + u);
+		if (!adds || k != 0) continue;
+		float t = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+		const float* tail = set + i * kRowSet + kRows * kRowLds + r * kRowTail;
+		for (int l = 0; l < (int)(a.S - full); ++l) t = t + tail[l];
+		(which + i == 0 ? a.out0 : a.out1)[row0 + r * a.C] = t;
+	}
 }
 
 constexpr int kElemChunk = 4096;  // channel elements per workgroup in the elementwise kernels (16 per thread)
@@ -1011,8 +1030,10 @@ hipError_t prepare_norm() {
 	auto raise = [&](const void* fn) {
 		if (e == hipSuccess) e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
 	};
-	raise(reinterpret_cast<const void*>(bn_rows_kernel<kBwd, false>));  // two sets of terms: 76 KB
-	raise(reinterpret_cast<const void*>(bn_rows_kernel<kBwd, true>));
+	raise(reinterpret_cast<const void*>(bn_rows_kernel<kBwd, false, BnLong>));  // two sets of terms: 76 KB
+	raise(reinterpret_cast<const void*>(bn_rows_kernel<kBwd, true, BnLong>));
+	raise(reinterpret_cast<const void*>(bn_rows_kernel<kBwd, false, BnMedium>));
+	raise(reinterpret_cast<const void*>(bn_rows_kernel<kBwd, true, BnMedium>));
 	for (int p = 0; p < 2; ++p)
 		for (int v = 0; v < 2; ++v) {
 			raise(reinterpret_cast<const void*>(kLnForward[p][v]));
@@ -1031,24 +1052,41 @@ int ln_rows(int64_t R, int D, int blocks) {
 
 inline bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
-template <int MODE>
-hipError_t launch_rows(BnRowArgs& a, bool vec, hipStream_t s) {
+template <int MODE, class SH>
+hipError_t launch_rows_as(BnRowArgs& a, bool vec, hipStream_t s) {
 	const hipError_t e = prepare_norm();
 	if (e != hipSuccess) return e;
-	a.groups = std::max<int64_t>(1, (a.N + kRows - 1) / kRows);
+	a.groups = std::max<int64_t>(1, (a.N + SH::kRows - 1) / SH::kRows);
 	const int per = vec ? 4 : 1;
-	const int64_t last = a.S > 0 ? (a.S - 1) % kChunk + 1 : per;
-	a.whole = make_fastdiv((unsigned)(kChunk / per));
+	const int64_t last = a.S > 0 ? (a.S - 1) % SH::kChunk + 1 : per;
+	a.whole = make_fastdiv((unsigned)(SH::kChunk / per));
 	a.last = make_fastdiv((unsigned)(last / per));
-	const int64_t blocks = a.C * a.groups, most = ((int64_t)1 << 31) - 1;
-	for (a.first_block = 0; a.first_block < blocks; a.first_block += most) {
-		hipLaunchKernelGGL((vec ? bn_rows_kernel<MODE, true> : bn_rows_kernel<MODE, false>),
-		                   dim3((unsigned)std::min(most, blocks - a.first_block)), dim3(256),
-		                   (MODE == kBwd ? 2 : 1) * kRowSet * sizeof(float), s, a);
+	const int64_t blocks = a.C * a.groups;
+	for (a.first_block = 0; a.first_block < blocks; a.first_block += kMaxGrid) {
+		hipLaunchKernelGGL((vec ? bn_rows_kernel<MODE, true, SH> : bn_rows_kernel<MODE, false, SH>),
+		                   dim3((unsigned)std::min(kMaxGrid, blocks - a.first_block)), dim3(256),
+		                   (MODE == kBwd ? 2 : 1) * SH::kRowSet * sizeof(float), s, a);
 		const hipError_t err = hipGetLastError();
 		if (err != hipSuccess) return err;
 	}
 	return hipSuccess;
+}
+
+// Rows a workgroup. Every workgroup of the squares repeats the channel's double sum over N rows (about 8 cycles a row), and
+// issues its loads for a whole chunk, so short rows go 32 to a workgroup, and rows of up to 1024 go 8 as long as 256
+// workgroups are left. Forward and backward with four rows a workgroup against this (us): [256, 256] 243 -> 30 and 171 ->
+// 21, [4096, 128] 5707 -> 644 and 1339 -> 146, [64, 576, 7 x 7] 141 -> 29 and 115 -> 28, [27, 60] 19.9 -> 15.5, [64, 128, 14 x
+// 14] 25.8 -> 22.5 and 22.5 -> 18.0, [128, 64, 28 x 28] 32 -> 30 and 35 -> 32. The backward's two sets of terms fill LDS with
+// 1024 long rows: from 900 on four rows are faster ([32, 64, 32 x 32] 13.5 against 16.9), as for a few aligned rows from 64
+// ([32, 8, 10 x 10] 10.7 against 11.6).
+template <int MODE>
+hipError_t launch_rows(BnRowArgs& a, bool vec, hipStream_t s) {
+	auto fills = [&](int rows) { return a.C * ((a.N + rows - 1) / rows) >= 256; };
+	if (a.S <= BnShort::kChunk && (MODE != kBwd || !vec || a.S <= 64 || fills(BnShort::kRows)))
+		return launch_rows_as<MODE, BnShort>(a, vec, s);
+	if (a.S <= (MODE == kBwd ? 768 : BnMedium::kChunk) && fills(BnMedium::kRows))
+		return launch_rows_as<MODE, BnMedium>(a, vec, s);
+	return launch_rows_as<MODE, BnLong>(a, vec, s);
 }
 
 hipError_t launch_elem(bool fwd, BnElemArgs& a, hipStream_t s) {

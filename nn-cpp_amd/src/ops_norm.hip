@@ -15,7 +15,8 @@ namespace {
 constexpr uint64_t kGridMax = ((uint64_t)1 << 31) - 1;
 
 // ops.cpp:901-907: x needs a channel axis (the caller folds the axes after it into S); N, C and S describe it.
-// Also the limits of the kernels' grids: C * ceil(N / 8) and C * ceil(N * S / 4096) workgroups.
+// Sizes above C * ceil(N / 8) or C * ceil(N * S / 4096) = 2^31 - 1 are refused (the second is the element-wise
+// kernels' workgroups; the row sums take at most the first, 2^24 - 1 a launch).
 int bn_geom(size_t N, size_t C, size_t S, BnGeom& g) {
 	uint64_t count = 0;
 	if (!count_ok({N, C, S}, count)) return fail(NNH_ERR_INVALID, "batchnorm: size out of range (above 2^60 elements)");

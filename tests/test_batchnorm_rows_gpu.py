@@ -40,3 +40,45 @@ def test_row_sums(gpu, oracle, N, C, S, relu):
         nnh.batchnorm_backward(gd, xd, alive, wd, mean, inv, dx=dx, dw=dw, db=db)
         for got, want, what in ((dx, dx0, "dx"), (dw, dw0, "dw"), (db, db0, "db")):
             assert_same(got.cpu().numpy(), want.reshape(got.shape), (what, N, C, S, off))
+
+
+@pytest.mark.parametrize("N,C,S", [(1, 256, 1), (31, 256, 8), (32, 257, 5), (33, 128, 7), (65, 90, 127), (32, 256, 128),
+                                   (40, 52, 129), (9, 128, 256), (8, 256, 768), (7, 256, 769), (17, 90, 1000), (9, 130, 1024),
+                                   (9, 130, 1025)])
+@pytest.mark.parametrize("relu", [False, True])
+def test_short_row_sums(gpu, oracle, N, C, S, relu):
+    """Enough short rows to go 32 or 8 to a workgroup: lengths and counts around both."""
+    test_row_sums(gpu, oracle, N, C, S, relu)
+
+
+def test_more_rows_than_one_launch_takes(gpu):
+    """40 x 2^23 rows of one element: the row sums take 2^24 workgroups, more than the 2^32 - 1 work-items of a launch. The
+    reference is the same sums in order, channel-wise."""
+    import torch
+
+    import nnh
+    N, C = 40, 1 << 23
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.empty(N, C, device="cuda").normal_(generator=gen)
+    w, b = (torch.empty(C, device="cuda").normal_(generator=gen) for _ in range(2))
+    y, _, mean, var, inv = nnh.batchnorm_forward(x, w, b, EPS)
+    s, q = (torch.zeros(C, dtype=torch.float64, device="cuda") for _ in range(2))
+    for n in range(N):
+        s += x[n].double()
+    assert torch.equal(mean, (s / N).float())
+    for n in range(N):
+        d = x[n] - mean
+        q += (d * d).double()
+    assert torch.equal(var, (q / N).float())
+    assert torch.equal(y, (x - mean) * (w * inv) + b)
+    del y, d
+    g = torch.empty(N, C, device="cuda").normal_(generator=gen)
+    dw, db = torch.empty_like(w), torch.empty_like(b)
+    nnh.batchnorm_backward(g, x, None, w, mean, inv, dw=dw, db=db)
+    s.zero_()
+    q.zero_()
+    for n in range(N):
+        s += g[n].double()
+        q += (g[n] * (x[n] - mean)).double()
+    assert torch.equal(db, s.float() + 0.0)
+    assert torch.equal(dw, (q * inv.double()).float() + 0.0)
