@@ -386,7 +386,11 @@ __global__ void __launch_bounds__(256) bn_norm_kernel(const BnElemArgs a) {
 // The backward rule's per-channel part (ops.cpp:970-999): the prologue adds the rows' sums in double, the
 // channel's first workgroup adds sdy into db and sdg * inv_std into dw, and every workgroup writes its chunk of
 // dx = k * (M * g' - a - ((x - mean) * inv_std) * b) with k = weight * inv_std / M, g' masked by alive.
-template <bool FAST>
+// AHEAD: the chunk's elements are loaded ahead of the channel's sums, which takes 88 registers (5 waves a SIMD) against 44
+// (8): a few percent faster while the sums are short, but with thousands of samples the sums are the time and all of a
+// channel's workgroups have to be resident at once ([4096, 8, 16 x 16] 164 us with it, 118 without; [512, 16, 14 x 14] 24.5
+// and 25.2; [1024, 8, 28 x 28] 55 and 46).
+template <bool FAST, bool AHEAD>
 __global__ void __launch_bounds__(256) bn_dx_kernel(const BnElemArgs a) {
 	__shared__ float buf[2][256];
 	__shared__ double bcast[2];
@@ -396,19 +400,19 @@ __global__ void __launch_bounds__(256) bn_dx_kernel(const BnElemArgs a) {
 	const int64_t total = a.N * a.S;
 	const int64_t e0 = j * kElemChunk;
 	const bool masked = a.alive_in != nullptr;
-	// loaded ahead of the channel's sums, as in bn_norm_kernel
 	f32x4 gs[kElemChunk / 1024], xs[kElemChunk / 1024];
 	unsigned fls[kElemChunk / 1024];
 	int64_t offs[kElemChunk / 1024];
-	if (a.y && a.vec && total > 0) {
+	auto load = [&](int u) {  // past the end the last group again
+		const int64_t e = e0 + 4 * (tid + 256 * u);
+		offs[u] = channel_offset<FAST>(e < total ? e : total - 4, a, c);
+		gs[u] = *reinterpret_cast<const f32x4*>(a.g + offs[u]);
+		xs[u] = *reinterpret_cast<const f32x4*>(a.x + offs[u]);
+		fls[u] = masked ? *reinterpret_cast<const unsigned*>(a.alive_in + offs[u]) : 0x01010101u;
+	};
+	if (AHEAD && a.y && a.vec && total > 0) {
 #pragma unroll
-		for (int u = 0; u < kElemChunk / 1024; ++u) {
-			const int64_t e = e0 + 4 * (tid + 256 * u);
-			offs[u] = channel_offset<FAST>(e < total ? e : total - 4, a, c);
-			gs[u] = *reinterpret_cast<const f32x4*>(a.g + offs[u]);
-			xs[u] = *reinterpret_cast<const f32x4*>(a.x + offs[u]);
-			fls[u] = masked ? *reinterpret_cast<const unsigned*>(a.alive_in + offs[u]) : 0x01010101u;
-		}
+		for (int u = 0; u < kElemChunk / 1024; ++u) load(u);
 	}
 	double s[2];
 	channel_dsums<2>(a.rowv0, a.rowv1, a.N, a.C, c, buf, bcast, s);
@@ -424,6 +428,7 @@ __global__ void __launch_bounds__(256) bn_dx_kernel(const BnElemArgs a) {
 #pragma unroll
 		for (int u = 0; u < kElemChunk / 1024; ++u) {
 			if (e0 + 4 * (tid + 256 * u) >= total) continue;
+			if (!AHEAD) load(u);
 			const int64_t off = offs[u];
 			const f32x4 gv = gs[u], xv = xs[u];
 			const unsigned fl = fls[u];
@@ -1099,8 +1104,10 @@ hipError_t launch_elem(bool fwd, BnElemArgs& a, hipStream_t s) {
 		if (fast) hipLaunchKernelGGL(bn_norm_kernel<true>, grid, dim3(256), 0, s, a);
 		else hipLaunchKernelGGL(bn_norm_kernel<false>, grid, dim3(256), 0, s, a);
 	} else {
-		if (fast) hipLaunchKernelGGL(bn_dx_kernel<true>, grid, dim3(256), 0, s, a);
-		else hipLaunchKernelGGL(bn_dx_kernel<false>, grid, dim3(256), 0, s, a);
+		const bool ahead = a.N <= 512;
+		const auto fn = fast ? (ahead ? bn_dx_kernel<true, true> : bn_dx_kernel<true, false>)
+		                     : (ahead ? bn_dx_kernel<false, true> : bn_dx_kernel<false, false>);
+		hipLaunchKernelGGL(fn, grid, dim3(256), 0, s, a);
 	}
 	return hipGetLastError();
 }

@@ -51,6 +51,13 @@ def test_short_row_sums(gpu, oracle, N, C, S, relu):
     test_row_sums(gpu, oracle, N, C, S, relu)
 
 
+@pytest.mark.parametrize("N,C,S", [(512, 2, 16), (513, 3, 8), (513, 2, 7), (600, 1, 20), (2049, 2, 4)])
+@pytest.mark.parametrize("relu", [False, True])
+def test_many_samples(gpu, oracle, N, C, S, relu):
+    """Sample counts on both sides of where dx loads its elements after the channel's sums, whole chunks and remainders."""
+    test_row_sums(gpu, oracle, N, C, S, relu)
+
+
 def test_more_rows_than_one_launch_takes(gpu):
     """40 x 2^23 rows of one element: the row sums take 2^24 workgroups, more than the 2^32 - 1 work-items of a launch. The
     reference is the same sums in order, channel-wise."""
