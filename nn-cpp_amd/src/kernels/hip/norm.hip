@@ -13,8 +13,10 @@
 //     instead of a launch of their own.
 //   * bn_norm_kernel (forward) and bn_dx_kernel (backward) are elementwise over a channel's N*S elements in 4096-
 //     element chunks, 16-byte loads and stores where the rows allow.
-// Layer norm. Each row's sums are single float chains (ops.cpp:1017-1026), so one thread owns a row; the
-// gamma/beta gradient sums run down columns in row order, one thread per column (ops.cpp:1063-1075).
+// Layer norm. Each row's sums are single float chains (ops.cpp:1017-1026): a workgroup holds some rows in registers, all
+// its threads form the chains' terms and put them in LDS, and one thread a chain adds them there. The gamma/beta
+// gradient sums run down columns in row order (ops.cpp:1063-1075): chains over LDS again, beside dx in the same launch.
+// Longer rows than a workgroup's registers hold take one thread a row and one a column.
 #include "norm.hpp"
 
 #include <algorithm>
@@ -578,16 +580,17 @@ __global__ void __launch_bounds__(256) ln_backward_kernel(const LnBwdArgs a) {
 // registers from the load to the store. Only the row chains (one dependent add per element, the reference's order) run
 // over LDS: all threads put the terms there, element-wise, and one lane per chain adds them in order, sixteen at a time
 // from 16-byte reads two blocks ahead, about 7 cycles an add (4.3 from registers; the reads take the rest). The rows of
-// LDS are padded to a multiple of four floats plus four, so that the lanes of a read (one row each) use different banks.
-// What bounds it: the two (forward) or one (backward) chain of D adds, 1.3 us at D = 512, between the load and the store;
+// LDS are an odd number of 16-byte words apart, so that the lanes of a read (one row each) use different banks.
+// What bounds it: the two (forward) or one (backward) chain of D adds, 1.5 us at D = 512, between the load and the store;
 // rw is chosen so that 2 to 4 workgroups share a CU and one's chain runs beside another's memory traffic. Measured
 // over [8192, 512]: forward 22.8 -> 12.4 us, dx alone 37.2 -> 12.0, against a version that also ran the element-wise
 // passes in the chain lanes.
 // PER: 16-byte groups (VEC) or quadruples of floats a thread holds: rw * D <= 1024 PER.
 
-constexpr int kLnMaxRows = 32;  // chains of one kind in a wave: lanes 0 .. 31, the backward's second kind lanes 32 .. 63
+// Chains of one kind: in the forward a thread each; in the backward lanes 0 .. 31 of wave 0, the second kind lanes 32 .. 63.
+constexpr int kLnMaxRows = 256, kLnMaxDxRows = 32;
 
-__device__ __host__ __forceinline__ int ln_pitch(int D) { return ((D + 3) & ~3) + 4; }
+__device__ __host__ __forceinline__ int ln_pitch(int D) { return 4 * (((D + 3) >> 2) | 1); }
 
 struct LnArgs {
 	const float* x;
@@ -738,8 +741,8 @@ __device__ __forceinline__ void ln_dx_body(const LnArgs& a, int block, float* ld
 		}
 	});
 	__syncthreads();
-	if (tid < 64 && (tid & (kLnMaxRows - 1)) < nr) {
-		const int r = tid & (kLnMaxRows - 1), second = tid / kLnMaxRows;
+	if (tid < 64 && (tid & (kLnMaxDxRows - 1)) < nr) {
+		const int r = tid & (kLnMaxDxRows - 1), second = tid / kLnMaxDxRows;
 		st[4 * r + 2 + second] = lds_chain((second ? lb : la) + r * pitch, D);
 	}
 	__syncthreads();
@@ -1012,8 +1015,9 @@ constexpr int kLnMaxD = 1024 * kLnMaxPer;  // longest row a workgroup holds in r
 
 using LnForwardFn = void (*)(const LnArgs);
 using LnBackwardFn = void (*)(const LnArgs, const LnColArgs);
-// [PER 16][VEC]
-const LnForwardFn kLnForward[2][2] = {{ln_forward_rows_kernel<8, false>, ln_forward_rows_kernel<8, true>},
+// [PER 2, 8, 16][VEC]
+const LnForwardFn kLnForward[3][2] = {{ln_forward_rows_kernel<2, false>, ln_forward_rows_kernel<2, true>},
+                                      {ln_forward_rows_kernel<8, false>, ln_forward_rows_kernel<8, true>},
                                       {ln_forward_rows_kernel<16, false>, ln_forward_rows_kernel<16, true>}};
 // [PER 16][VEC][COLS]
 const LnBackwardFn kLnBackward[2][2][3] = {
@@ -1039,19 +1043,19 @@ hipError_t prepare_norm() {
 	raise(reinterpret_cast<const void*>(bn_rows_kernel<kBwd, true, BnLong>));
 	raise(reinterpret_cast<const void*>(bn_rows_kernel<kBwd, false, BnMedium>));
 	raise(reinterpret_cast<const void*>(bn_rows_kernel<kBwd, true, BnMedium>));
-	for (int p = 0; p < 2; ++p)
-		for (int v = 0; v < 2; ++v) {
-			raise(reinterpret_cast<const void*>(kLnForward[p][v]));
+	for (int v = 0; v < 2; ++v) {
+		for (int p = 0; p < 3; ++p) raise(reinterpret_cast<const void*>(kLnForward[p][v]));
+		for (int p = 0; p < 2; ++p)
 			for (int c = 0; c < 3; ++c) raise(reinterpret_cast<const void*>(kLnBackward[p][v][c]));
-		}
+	}
 	done[dev] = e == hipSuccess;
 	return e;
 }
 
 // Rows per workgroup: as many as its registers and chain lanes hold, but few enough for about `blocks` workgroups, and
 // enough that every thread has an element.
-int ln_rows(int64_t R, int D, int blocks) {
-	const int64_t most = std::max<int64_t>(1, std::min<int64_t>(kLnMaxRows, (D <= 8192 ? 8192 : kLnMaxD) / D));
+int ln_rows(int64_t R, int D, int blocks, int max_rows) {
+	const int64_t most = std::max<int64_t>(1, std::min<int64_t>(max_rows, (D <= 8192 ? 8192 : kLnMaxD) / D));
 	return (int)std::max<int64_t>(1, std::min(std::min(most, R), std::max<int64_t>((R + blocks - 1) / blocks, (255 + D) / D)));
 }
 
@@ -1211,8 +1215,14 @@ hipError_t batchnorm_backward(const float* gy, const float* x, const unsigned ch
 hipError_t layernorm_forward(const float* x, const float* gamma, const float* beta, int64_t R, int D, float fd,
                              float eps, float* y, float* mean, float* inv_std, hipStream_t s) {
 	if (R == 0) return hipSuccess;
-	const int rw = ln_rows(R, D, 1024);
-	if (D <= kLnMaxD && R / rw < ((int64_t)1 << 31) - 1) {
+	const bool vec = D % 4 == 0 && aligned16(x) && aligned16(y);
+	// Short rows in workgroups of 2048 floats, two 16-byte groups a thread: with more, each thread issues eight groups (or 32
+	// single floats) however few the rows are, and 32 rows of a few floats are no work for a workgroup. Against 32 rows a
+	// workgroup and eight groups (us): [8192, 5] 4.2 -> 3.2, [262144, 5] 35 -> 5.7, [262144, 32] 22 -> 12.5, unaligned [32768,
+	// 65] 12.3 -> 8.1. Aligned rows above 64 are as fast in larger blocks, all rows above 256 faster ([8192, 1537] 67 against
+	// 95, [1024, 2048] 30.7 against 32.8).
+	const int rw = ln_rows(R, D, 1024, D <= (vec ? 64 : 256) ? std::min(2048 / D, kLnMaxRows) : kLnMaxRows);
+	if (D <= kLnMaxD && R / rw < kMaxGrid) {
 		LnArgs a{};
 		a.x = x;
 		a.gm = gamma;
@@ -1225,17 +1235,16 @@ hipError_t layernorm_forward(const float* x, const float* gamma, const float* be
 		a.rw = rw;
 		a.fd = fd;
 		a.eps = eps;
-		const bool vec = D % 4 == 0 && aligned16(x) && aligned16(y);
 		a.dq = make_fastdiv((unsigned)(vec ? D / 4 : D));
 		const hipError_t e = prepare_norm();
 		if (e != hipSuccess) return e;
-		hipLaunchKernelGGL(kLnForward[D > 8192 ? 1 : 0][vec ? 1 : 0], dim3((unsigned)((R + rw - 1) / rw)), dim3(256),
+		const int per = D <= 256 && rw * D <= 2048 ? 0 : D <= 8192 ? 1 : 2;
+		hipLaunchKernelGGL(kLnForward[per][vec ? 1 : 0], dim3((unsigned)((R + rw - 1) / rw)), dim3(256),
 		                   (size_t)rw * (ln_pitch(D) + 2) * sizeof(float), s, a);
 		return hipGetLastError();
 	}
-	const int vec = D % 4 == 0 && aligned16(x) && aligned16(y) && aligned16(gamma) && aligned16(beta);
 	hipLaunchKernelGGL(ln_forward_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, s, x, gamma, beta, R, D, fd,
-	                   eps, y, mean, inv_std, vec);
+	                   eps, y, mean, inv_std, vec && aligned16(gamma) && aligned16(beta) ? 1 : 0);
 	return hipGetLastError();
 }
 
@@ -1243,7 +1252,7 @@ hipError_t layernorm_backward(const float* gy, const float* x, const float* gamm
                               const float* inv_std, int64_t R, int D, float fd, float* dx, int dx_first,
                               float* dgamma, int dgamma_first, float* dbeta, int dbeta_first, hipStream_t s) {
 	if (R == 0 && !dgamma && !dbeta) return hipSuccess;
-	const int rw = ln_rows(std::max<int64_t>(R, 1), D, 512);
+	const int rw = ln_rows(std::max<int64_t>(R, 1), D, 512, kLnMaxDxRows);
 	const bool cols = dgamma || dbeta;
 	if (D <= kLnMaxD && R / rw < ((int64_t)1 << 31) - D && R > 0) {
 		LnArgs a{};

@@ -43,3 +43,30 @@ def test_rows_and_columns(gpu, oracle, R, D):
                 for t, w, what in zip(got, want, ("dx", "dgamma", "dbeta")):
                     if t is not None:
                         assert_same(t.cpu().numpy(), w, (what, R, D, off, first, parts))
+
+
+@pytest.mark.parametrize("R,D", [(1, 1), (255, 1), (256, 1), (257, 2), (1025, 3), (511, 4), (513, 8), (129, 16), (300, 9), (151, 27),
+                                 (65, 60), (33, 64), (31, 65), (63, 68), (5, 1000), (3, 2047), (3, 2048), (2, 2049), (4100, 25)])
+def test_short_rows(gpu, oracle, R, D):
+    """Rows around those that go up to 256 to a workgroup of 2048 floats, full workgroups and a last row alone."""
+    test_rows_and_columns(gpu, oracle, R, D)
+
+
+def test_more_rows_than_32_a_workgroup_take(gpu):
+    """2^29 + 3 rows of two: with 32 rows a workgroup more than the 2^32 - 1 work-items of a launch. Rows at both ends and on
+    either side of 2^29 against the same arithmetic."""
+    import torch
+
+    import nnh
+    R = (1 << 29) + 3
+    x = torch.empty(R, 2, device="cuda").uniform_(-1, 1, generator=torch.Generator(device="cuda").manual_seed(6))
+    gm, bt = torch.tensor([1.5, -0.75], device="cuda"), torch.tensor([0.25, 2.0], device="cuda")
+    y, mean, inv = nnh.layernorm_forward(x, gm, bt, EPS)
+    for r0, r1 in ((0, 1 << 16), ((1 << 29) - (1 << 16), R)):
+        xs = x[r0:r1].cpu().numpy()
+        mu = (xs[:, 0] + xs[:, 1]) / np.float32(2)
+        d = xs - mu[:, None]
+        iv = np.float32(1) / np.sqrt((d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1]) / np.float32(2) + np.float32(EPS))
+        want = d * iv[:, None] * gm.cpu().numpy() + bt.cpu().numpy()
+        for got, ref, what in ((mean, mu, "mean"), (inv, iv, "inv_std"), (y, want, "y")):
+            assert_same(got[r0:r1].cpu().numpy(), ref, (what, r0))
