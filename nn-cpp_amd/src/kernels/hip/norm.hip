@@ -786,9 +786,10 @@ struct LnColArgs {
 // ring, form g * ((x - mean) * inv_std) exactly as the reference does and write it and g to LDS column by column (a
 // column's rows back to back); wave 0, one chunk behind, adds: lanes 0-15 the products down their column (dgamma),
 // lanes 16-31 g (dbeta), four rows per 16-byte read. One barrier a chunk, two buffers. 16 columns a workgroup keep the
-// loads (64 bytes a row) at a third of what a CU can take. Measured for 8192 rows of 512: 37 us, and 41 with dx beside it
+// loads (64 bytes a row) at a third of what a CU can take. Measured for 8192 rows of 512: 37 us, and 39 with dx beside it
 // (52 and 90 in two launches with 32 columns and fifteen producer waves, where the chain wave shared its SIMD with three
-// producers and read one row at a time); of 64: 30 us against 51.
+// producers and read one row at a time); of 64: 30 us against 51. Wide rows are bound by memory, so the two blocks that share
+// a 128-byte line run on one XCD: 8192 rows of 4096 without dx 81 us in launch order, 50 so (32 columns a workgroup: 54).
 constexpr int kLnCols = 16, kLnAhead = 3, kLnWaveRows = 64, kLnChunk = 3 * kLnWaveRows;
 constexpr int kLnColPitch = kLnChunk + 4;  // 4 mod 64: the chain lanes' 16-byte reads use different banks
 constexpr int kLnColBuf = 2 * kLnCols * kLnColPitch;
@@ -798,7 +799,8 @@ template <bool VEC>
 __device__ __forceinline__ void ln_columns_body(const LnColArgs& d, int block, float* lds) {
 	const int tid = threadIdx.x, lane = tid & 63;
 	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-	const int c0 = block * kLnCols, D = d.D;
+	const int per = d.blocks / 8;  // neighbouring blocks share the rows' cache lines: a contiguous range for each XCD
+	const int c0 = (block < per * 8 ? (block % 8) * per + block / 8 : block) * kLnCols, D = d.D;
 	const int64_t R = d.R, chunks = (R + kLnChunk - 1) / kLnChunk;
 	// a producer's slot u of a chunk: VEC row 16 u + lane / 4, columns 4 (lane % 4) ..; else row 4 u + lane / 16, column
 	// lane % 16 (columns past D read a clamped address: their chains are not stored)
@@ -1254,15 +1256,13 @@ hipError_t layernorm_backward(const float* gy, const float* x, const float* gamm
 	if (R == 0 && !dgamma && !dbeta) return hipSuccess;
 	const int rw = ln_rows(std::max<int64_t>(R, 1), D, 512, kLnMaxDxRows);
 	const bool cols = dgamma || dbeta;
-	if (D <= kLnMaxD && R / rw < ((int64_t)1 << 31) - D && R > 0) {
+	// Column sums alone of up to 1024 wide rows: a thread a column, coalesced, without LDS. The small kernel's four columns a
+	// workgroup read 16 bytes a row: 1 row of 8192 10.1 us against 2.1, 512 rows of 4096 27.5 against 20, 1024 rows 58 against
+	// 50, of 2048 17.5 against 20.
+	const bool wide_cols = !dx && R <= kLnSmallRows && D >= 4096;
+	if (D <= kLnMaxD && R > 0 && !wide_cols) {
 		LnArgs a{};
-		a.g = gy;
-		a.x = x;
 		a.gm = gamma;
-		a.mean_in = mean;
-		a.inv_in = inv_std;
-		a.y = dx;
-		a.R = R;
 		a.D = D;
 		a.rw = rw;
 		a.fd = fd;
@@ -1279,12 +1279,26 @@ hipError_t layernorm_backward(const float* gy, const float* x, const float* gamm
 			return hipGetLastError();
 		}
 		if (cols) d.blocks = small ? (D + kLnMergedCols - 1) / kLnMergedCols : (D + kLnCols - 1) / kLnCols;
-		const int64_t blocks = d.blocks + (dx ? (R + rw - 1) / rw : 0);
 		const size_t lds_dx = dx ? (size_t)rw * (2 * ln_pitch(D) + 4) * sizeof(float) : 0;
 		const size_t lds_cols = !cols ? 0 : small ? kLnMergedLds : kLnColLds;
-		hipLaunchKernelGGL(kLnBackward[D > 8192 ? 1 : 0][vec ? 1 : 0][!cols ? 0 : small ? 1 : 2], dim3((unsigned)blocks), dim3(256),
-		                   std::max(lds_dx, lds_cols), s, a, d);
-		return hipGetLastError();
+		const auto* fns = kLnBackward[D > 8192 ? 1 : 0][vec ? 1 : 0];
+		// the columns and the rows of one launch, then the rows that are left
+		const int64_t most = (kMaxGrid - kLnMaxD) * rw;
+		for (int64_t r0 = 0; r0 < R && (r0 == 0 || dx); r0 += most) {
+			a.g = gy + r0 * D;
+			a.x = x + r0 * D;
+			a.mean_in = mean + r0;
+			a.inv_in = inv_std + r0;
+			a.y = dx ? dx + r0 * D : nullptr;
+			a.R = std::min(most, R - r0);
+			const int64_t blocks = d.blocks + (dx ? (a.R + rw - 1) / rw : 0);
+			hipLaunchKernelGGL(fns[d.blocks == 0 ? 0 : small ? 1 : 2], dim3((unsigned)blocks), dim3(256),
+			                   std::max(lds_dx, lds_cols), s, a, d);
+			e = hipGetLastError();
+			if (e != hipSuccess) return e;
+			d.blocks = 0;
+		}
+		return hipSuccess;
 	}
 	LnBwdArgs a{};
 	a.g = gy;

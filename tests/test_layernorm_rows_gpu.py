@@ -45,6 +45,13 @@ def test_rows_and_columns(gpu, oracle, R, D):
                         assert_same(t.cpu().numpy(), w, (what, R, D, off, first, parts))
 
 
+@pytest.mark.parametrize("R,D", [(1, 4096), (17, 4095), (9, 4100), (1024, 4096), (1025, 4097), (200, 140), (1200, 300), (1030, 16380)])
+def test_wide_columns(gpu, oracle, R, D):
+    """Column sums alone on both sides of where a thread takes a column, and column blocks that do and do not divide by
+    eight."""
+    test_rows_and_columns(gpu, oracle, R, D)
+
+
 @pytest.mark.parametrize("R,D", [(1, 1), (255, 1), (256, 1), (257, 2), (1025, 3), (511, 4), (513, 8), (129, 16), (300, 9), (151, 27),
                                  (65, 60), (33, 64), (31, 65), (63, 68), (5, 1000), (3, 2047), (3, 2048), (2, 2049), (4100, 25)])
 def test_short_rows(gpu, oracle, R, D):
@@ -70,3 +77,16 @@ def test_more_rows_than_32_a_workgroup_take(gpu):
         want = d * iv[:, None] * gm.cpu().numpy() + bt.cpu().numpy()
         for got, ref, what in ((mean, mu, "mean"), (inv, iv, "inv_std"), (y, want, "y")):
             assert_same(got[r0:r1].cpu().numpy(), ref, (what, r0))
+    # the gradient of the same rows: more workgroups than one launch takes
+    g = torch.empty(R, 2, device="cuda").uniform_(-1, 1, generator=torch.Generator(device="cuda").manual_seed(7))
+    dx = y.zero_()
+    nnh.layernorm_backward(g, x, gm, mean, inv, dx=dx)
+    two = np.float32(2)
+    for r0, r1 in ((0, 1 << 16), ((1 << 29) - (1 << 20), (1 << 29) - (1 << 19)), ((1 << 29) - (1 << 16), R)):
+        xs, gs, mu, iv = (t[r0:r1].cpu().numpy() for t in (x, g, mean, inv))
+        xh, dh = (xs - mu[:, None]) * iv[:, None], gs * gm.cpu().numpy()
+        sa = np.float32(0) + dh[:, 0] + dh[:, 1]
+        p = dh * xh
+        sb = np.float32(0) + p[:, 0] + p[:, 1]
+        want = (iv / two)[:, None] * (two * dh - sa[:, None] - xh * sb[:, None])
+        assert_same(dx[r0:r1].cpu().numpy(), want + np.float32(0), ("dx", r0))
