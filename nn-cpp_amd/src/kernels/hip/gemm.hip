@@ -352,7 +352,7 @@ hipError_t gemm_launch_pair(const GemmCall& g0, const GemmCall& g1, hipStream_t 
 	if (g0.batch_count != 1 || g1.batch_count != 1 || g0.batch.ndim != 0 || g1.batch.ndim != 0) return hipSuccess;
 	if (g0.m == 0 || g0.n == 0 || g1.m == 0 || g1.n == 0) return hipSuccess;
 	if (depth_cut(g0.m, g0.n, g0.k) || depth_cut(g1.m, g1.n, g1.k)) return hipSuccess;
-	if (ring_takes_large(g0) || ring_takes_large(g1)) return hipSuccess;
+	if ((ring_takes_large(g0) && ring_takes(g0)) || (ring_takes_large(g1) && ring_takes(g1))) return hipSuccess;
 	const int c0 = pick_config(g0), c1 = pick_config(g1);
 	if (c0 != c1) return hipSuccess;
 	const Config& cf = configs()[c0];

@@ -97,6 +97,7 @@ hipError_t gemm_pieces4_launch(const GemmCall& g, hipStream_t s);
 constexpr int kRingConfigs = 4;
 bool ring_ok(const GemmCall& g);
 bool ring_takes(const GemmCall& g);        // the shapes it is routed for (measured)
+bool ring_takes_gelu(const GemmCall& g);   // those it is routed for with the GELU epilogue
 bool ring_takes_large(const GemmCall& g);  // those of them that take 64 x 64 tiles or larger
 hipError_t gemm_ring_launch(const GemmCall& g, hipStream_t s, int config = -1);
 bool ring_pair_takes(const GemmCall& g0, const GemmCall& g1);  // an A B or A B^T and an A^T B in one grid

@@ -5,6 +5,7 @@
 #include <mutex>
 
 #include "gemm.hpp"
+#include "gemm_valu.hpp"
 
 namespace nnh {
 
@@ -120,7 +121,10 @@ bool ring_takes_large(const GemmCall& g) {
 	return tiles >= 176;
 }
 
-bool ring_takes(const GemmCall& g) {
+namespace {
+
+// Where the ring wins over the tile kernels.
+bool ring_fits(const GemmCall& g) {
 	if (ring_takes_large(g)) return true;
 	// Smaller products, where the 32 x 32 tile's chains are the time. A^T B (a weight gradient) is faster here at every
 	// size: 512 x 512 x 8192 67 -> 52 us, 1024 x 512 x 4096 66 -> 46, 512 x 784 x 256 7.7 -> 5.9 (chain kernel), 256 x 256 x
@@ -135,6 +139,55 @@ bool ring_takes(const GemmCall& g) {
 	if (g.ta && !g.tb) return true;
 	const bool whole = ring_vec(g) && g.m % 32 == 0 && g.n % 32 == 0 && g.k % 64 == 0 && g.ldc % 4 == 0 && aligned16(g.c);
 	return !whole || (!g.ta && !g.tb && tiles <= 256);
+}
+
+}  // namespace
+
+bool ring_takes(const GemmCall& g) {
+	if (!ring_fits(g)) return false;
+	if (g.rowsum) return true;  // the kernels below have none
+	// Where another kernel than the tiles takes the product, or most of a 32 x 32 tile is padding, as products of a few rows
+	// or columns and batches of small ones have it. Two 32 x 32 workgroups share a CU, so past 512 of them a product takes
+	// another round, while the chain kernel needs no LDS and the VALU kernel's blocks are 16 x 16; a depth that leaves the
+	// chain kernel a remainder, or single floats to load, favours the ring. The lines are fitted to 29000 products of 1 to 8192
+	// rows and columns, 96 to 4096 deep, up to 1024 of them; each with examples, the other kernel's us against the ring's.
+	const double m = (double)g.m, n = (double)g.n, batch = (double)g.batch_count;
+	const double tiles = (double)((g.m + 31) / 32) * (double)((g.n + 31) / 32) * batch;
+	const double blocks = (double)((g.m + 15) / 16) * (double)((g.n + 15) / 16) * batch;  // of the VALU kernel
+	const double padded = tiles * 1024 / (m * n * batch);
+	const bool vec = ring_vec(g), one_round = tiles <= 512;
+	if (chain4_takes(g)) {
+		// A^T B: 512 x 784 x 256 8.1, 6.2; 512 x 2048 x 200 11.0, 9.5; 354 x 1744 x 208 8.3, 10.0
+		if (g.ta && !g.tb)
+			return (g.k >= 248 && (one_round || tiles > 768)) || (vec && g.k >= 172 && tiles > 768) ||
+			       (g.k > 100 && one_round && blocks <= 1024 && batch > 1);
+		if (g.ta) return one_round && g.n > 15 && (vec || g.k < 128);
+		// A B^T: 64 x 1500 x 128 5.1, 4.6; 200 of 1 x 128 x 128 7.6, 9.0; 111 of 64 x 126 x 103 17.4, 11.3
+		if (g.tb) return vec ? one_round && padded <= 2 : (g.k > 112 || padded <= 4) && (g.m > 16 || g.n > 16);
+		// A B: 64 x 1500 x 128 4.6, 4.4; 4 of 2 x 4032 x 112 4.8, 5.5; 11 of 5 x 5553 x 112 12.9, 20.2
+		return one_round && g.m > 20 && (vec || (g.k > 112 && g.k < 128));
+	}
+	if (!g.ta && valu_takes(g)) {
+		// A B^T, 16-byte loads: 256 x 512 x 784 10.6, 11.4; 16 x 2930 x 456 7.1, 9.1; 20 x 5352 x 640 10.8, 9.0
+		if (g.tb && vec) return 2.9 * tiles <= blocks && blocks > 512;
+		// one float a lane: 215 of 2 x 168 x 2693 129, 169; 768 x 132 x 3670 39, 32
+		if (g.tb) return (g.k > 480 && 2.9 * tiles <= blocks) || (g.k > 800 && 5 * tiles <= 3 * blocks && tiles >= 160 && one_round);
+		// A B: 256 x 512 x 300 7.5, 6.4; 6 x 2976 x 256 4.5, 5.4; 549 of 4 x 2 x 464 9.1, 18.7
+		return g.n > 16 && g.k > 272 && (blocks > 256 || g.k > 800);
+	}
+	// the tile kernels: 260 of 2 x 1269 x 257 A B^T 145, 201; 435 of 2 x 2874 x 107 A B 297, 368; 300 x 1000 x 512 A B^T 13.8,
+	// 10.6; 200 x 2000 x 1000 A B 22.7, 16.7
+	if (one_round || g.ta) return true;
+	if (g.tb) return padded <= 4;
+	return (g.m > 16 || g.n > 16) && (g.m > 3 || g.k >= 176);
+}
+
+bool ring_takes_gelu(const GemmCall& g) {
+	// The other kernel with the epilogue is the chain kernel, at home where 16-byte loads feed it and its few chunks are in
+	// flight at once: 768 x 399 x 208 9.1 us against 11.1, 187 x 981 x 228 7.5 against 8.9; 8192 x 2048 x 512 far slower.
+	if (!ring_fits(g)) return false;
+	const double tiles = (double)((g.m + 31) / 32) * (double)((g.n + 31) / 32);
+	return !ring_vec(g) || g.k >= 256 || (tiles <= 512 ? tiles > 256 : (double)g.m * (double)g.n > 1.5e6);
 }
 
 namespace {

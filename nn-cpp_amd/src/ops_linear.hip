@@ -121,7 +121,7 @@ int nnh_linear_gelu_forward(const float* x, size_t M, size_t K, const float* w, 
 	int rc = build_gemm(0, 1, M, n, K, x, K, w, K, h, n, 0, nullptr, &ep, g);
 	if (rc != NNH_OK || M == 0 || n == 0) return rc;
 	// the ring kernel (large products) and the chain kernel (small ones) apply the GELU in their epilogue
-	const bool on_ring = ring_takes(g);
+	const bool on_ring = ring_takes_gelu(g);
 	if (on_ring || chain4_ok(g)) {
 		g.ep.gelu_y = y;
 		g.ep.gelu_t = tanh_saved;

@@ -108,3 +108,29 @@ def test_ring_pairs(gpu, oracle, M, K, n, first):
     want = oracle.linear_backward(g, x, w, dx=dx0, dx_first=first, dw=dw0, dw_first=first)
     assert_same(host(da), want[0], ("da", M, K, n, first))
     assert_same(host(dbm), want[1].T, ("db matmul", M, K, n, first))
+
+
+# (ta, tb, batch, m, n, k): both sides of the lines between the ring and the VALU, chain and tile kernels
+ROUTES = [(0, 1, 1, 256, 512, 784), (0, 1, 1, 512, 200, 511), (0, 1, 1, 20, 5352, 320), (0, 1, 70, 5, 5, 300), (0, 1, 1, 33, 1934, 901),
+          (0, 0, 1, 256, 512, 272), (0, 0, 1, 255, 512, 276), (0, 0, 1, 6, 2976, 256), (0, 0, 549, 4, 2, 260), (0, 0, 1, 64, 1500, 128),
+          (0, 0, 4, 2, 4032, 112), (0, 0, 11, 5, 5553, 112), (0, 1, 200, 1, 128, 128), (0, 1, 111, 64, 126, 103), (0, 1, 9, 17, 700, 113),
+          (1, 0, 1, 354, 1744, 208), (1, 0, 1, 512, 784, 256), (1, 0, 1, 516, 2048, 176), (1, 0, 3, 64, 128, 101), (1, 1, 2, 40, 900, 127),
+          (0, 1, 520, 9, 33, 200), (0, 0, 600, 3, 40, 176), (0, 0, 600, 3, 40, 175), (0, 0, 521, 16, 16, 129), (0, 1, 9, 3888, 3, 96)]
+
+
+@pytest.mark.parametrize("ta,tb,batch,m,n,k", ROUTES)
+def test_routes_of_padded_and_small_products(gpu, oracle, ta, tb, batch, m, n, k):
+    import torch
+
+    import nnh
+    a, b = synth.normal(61, (batch,) + ((k, m) if ta else (m, k))), synth.normal(62, (batch,) + ((n, k) if tb else (k, n)))
+    c0 = synth.normal(63, (batch, m, n))
+    ad, bd = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    strides = nnh.make_batch((batch,), (m * k,), (k * n,), (m * n,)) if batch > 1 else None
+    for acc in (0, 1):
+        c = torch.from_numpy(c0).cuda()
+        nnh.sgemm_batched(ta, tb, m, n, k, ad, m if ta else k, bd, k if tb else n, c, n, accumulate=bool(acc), batch=strides)
+        got = host(c)
+        for i in sorted({0, batch // 2, batch - 1}):
+            want = oracle.sgemm(ta, tb, m, n, k, a[i], m if ta else k, b[i], k if tb else n, c0[i].copy(), n, acc)
+            assert_same(got[i], want, (ta, tb, batch, m, n, k, i, acc))
