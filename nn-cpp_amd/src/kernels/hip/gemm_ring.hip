@@ -99,12 +99,20 @@ int ring_pick(const GemmCall& g) {
 	return best;
 }
 
+// A launch holds fewer than 2^32 work-items.
+bool ring_grid_ok(const GemmCall& g) {
+	const RingConfig& c = ring_configs()[ring_pick(g)];
+	return (double)((g.m + c.bm - 1) / c.bm) * (double)((g.n + c.bn - 1) / c.bn) * (double)g.batch_count * c.threads < 4294967296.0;
+}
+
 }  // namespace
 
 bool ring_ok(const GemmCall& g) {
 	// the offsets of a tile's rows are 32-bit byte counts: 256 rows of 2^21 floats stay below 2^31
 	constexpr int64_t kMaxLd = int64_t(1) << 21;
-	if (g.gather || g.k <= 0 || depth_cut(g.m, g.n, g.k) || g.lda >= kMaxLd || g.ldb >= kMaxLd) return false;
+	if (g.gather || g.k <= 0 || depth_cut(g.m, g.n, g.k) || g.lda >= kMaxLd || g.ldb >= kMaxLd ||
+	    g.batch_count >= (int64_t(1) << 31))
+		return false;
 	return !g.rowsum || (g.ta && !g.tb && g.rowsum_outer == 0 && g.batch_count == 1 && g.batch.ndim == 0);
 }
 
@@ -125,7 +133,7 @@ namespace {
 
 // Where the ring wins over the tile kernels.
 bool ring_fits(const GemmCall& g) {
-	if (ring_takes_large(g)) return true;
+	if (ring_takes_large(g)) return ring_grid_ok(g);
 	// Smaller products, where the 32 x 32 tile's chains are the time. A^T B (a weight gradient) is faster here at every
 	// size: 512 x 512 x 8192 67 -> 52 us, 1024 x 512 x 4096 66 -> 46, 512 x 784 x 256 7.7 -> 5.9 (chain kernel), 256 x 256 x
 	// 300 7.0 -> 5.4 (VALU kernel). The other layouts where the tile kernel would check bounds (200 x 2000 x 1000 23 -> 17,
@@ -136,9 +144,9 @@ bool ring_fits(const GemmCall& g) {
 	// few outputs with row sums have no other pipelined kernel (the backward of a 256 -> 10 layer at 256 rows, its dX 4 us of
 	// it: 13.2 us with dW on the tile kernel, 11.1 here)
 	if (tiles < 64) return g.rowsum != nullptr;
-	if (g.ta && !g.tb) return true;
+	if (g.ta && !g.tb) return ring_grid_ok(g);
 	const bool whole = ring_vec(g) && g.m % 32 == 0 && g.n % 32 == 0 && g.k % 64 == 0 && g.ldc % 4 == 0 && aligned16(g.c);
-	return !whole || (!g.ta && !g.tb && tiles <= 256);
+	return (!whole || (!g.ta && !g.tb && tiles <= 256)) && ring_grid_ok(g);
 }
 
 }  // namespace
@@ -228,7 +236,7 @@ hipError_t gemm_ring_launch(const GemmCall& g, hipStream_t s, int config) {
 	const RingConfig& c = ring_configs()[config >= 0 ? config : ring_pick(g)];
 	const GemmArgs p = ring_args(g, c);
 	const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * p.batch_count;
-	if (blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+	if (blocks * c.threads > 0xffffffff) return hipErrorInvalidConfiguration;
 	if (g.ep.gelu_y && (g.ta || !g.tb || g.rowsum)) return hipErrorInvalidValue;
 	const int v = ring_vec(g) ? 1 : 0;
 	const auto fn = g.ep.gelu_y ? c.gelu_fn[v] : g.rowsum ? c.rowsum_fn[v] : c.fn[(g.ta ? 2 : 0) + (g.tb ? 1 : 0)][v];

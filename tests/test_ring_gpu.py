@@ -134,3 +134,20 @@ def test_routes_of_padded_and_small_products(gpu, oracle, ta, tb, batch, m, n, k
         for i in sorted({0, batch // 2, batch - 1}):
             want = oracle.sgemm(ta, tb, m, n, k, a[i], m if ta else k, b[i], k if tb else n, c0[i].copy(), n, acc)
             assert_same(got[i], want, (ta, tb, batch, m, n, k, i, acc))
+
+
+def test_more_tiles_than_one_launch_takes(gpu, oracle):
+    """2^23 products of one 64 x 96 matrix with columns: on 32 x 32 tiles 2^24 workgroups, more than the 2^32 - 1 work-items of
+    a launch."""
+    import torch
+
+    import nnh
+    batch, m, n, k = 1 << 23, 64, 1, 96
+    a = synth.normal(71, (m, k))
+    b = torch.empty(batch, k, device="cuda").uniform_(-1, 1, generator=torch.Generator(device="cuda").manual_seed(8))
+    c = torch.full((batch, m), float(SENTINEL), device="cuda")
+    nnh.sgemm_batched(0, 0, m, n, k, torch.from_numpy(a).cuda(), k, b, n, c, n,
+                      batch=nnh.make_batch((batch,), (0,), (k * n,), (m * n,)))
+    for i in (0, 1, batch // 2, batch - 2, batch - 1):
+        want = oracle.sgemm(0, 0, m, n, k, a, k, b[i].cpu().numpy(), n, np.zeros((m, n), np.float32), n, 0)
+        assert_same(host(c[i]).reshape(m, n), want, i)
