@@ -241,20 +241,26 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 		for (int j = 0; j < J; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 	f32x4 af[2][I], bf[2][J];
 	// Row sums of op(A) (GemmArgs::rowsum): the first column tile's thread tid folds row tid in depth order. Depth past
-	// k was filled with +0, which leaves a sum from +0 unchanged.
-	float rsum = 0.0f;
-	const bool summing = RS && p.rowsum != nullptr && tn == 0 && tid < BM;
+	// k was filled with +0, which leaves a sum from +0 unchanged. With one or four chains a wave, four adds stand at each
+	// step's MFMAs, their operands read with the group's fragments, in whole waves (a tile of 32 rows: the upper lanes repeat the
+	// lower ones'): ahead of a stage's MFMAs its chain of adds took longer than they (4096 rows of a 512 -> 512 layer's
+	// dW and db 61 us, 45 so, and 27 without db; 65536 rows of 64 -> 1088 930, 670, 370). Larger tiles have no registers for
+	// that, and 2048 or more cycles of MFMAs a stage beside the adds.
+	constexpr bool kSpread = I * J <= 4;
+	float rsum = 0.0f, sums[RS && kSpread ? 2 : 1][16];
+	const bool summing = RS && p.rowsum != nullptr && tn == 0 && 64 * wave < BM;  // uniform
+	const int srow = tid & (BM - 1);
+	auto read_sums = [&](int slot, int k, float* v) {  // depths k .. k + 3 of the stage in `slot`
+		const float* As = lds + slot * S::kStage;
+#pragma unroll
+		for (int e = 0; e < 4; ++e) v[e] = As[(k + e) * BM + (srow ^ ring::kswz<BM>(k + e))];
+	};
 
 	// The MFMAs of the stage in `slot`, the fragments of its first group being in set 0; each group's reads are issued
 	// among the MFMAs of the group before, the last group reading the first of the stage in `after` (with has_next). With
 	// `issuing` the loads of the next stage to fetch, into ring slot `fill`, are spread over the whole stage too: issued
 	// in one burst they would stall the wave at the memory unit's rate with the matrix core idle.
-	auto compute = [&](int slot, int after, auto has_next, auto issuing, int fill) {
-		if (RS && summing) {
-			const float* As = lds + slot * S::kStage;
-#pragma unroll 8
-			for (int k = 0; k < BK; ++k) rsum = rsum + As[k * BM + (tid ^ ring::kswz<BM>(k))];
-		}
+	auto compute_stage = [&](int slot, int after, auto has_next, auto issuing, int fill, auto with_sums) {
 		constexpr int kSteps = BK / 4;
 #pragma unroll
 		for (int gi = 0; gi < NG; ++gi) {
@@ -262,6 +268,10 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 #pragma unroll
 			for (int t = 0; t < 4; ++t) {
 				const int step = 4 * gi + t;
+				if constexpr (decltype(with_sums)::value) {
+#pragma unroll
+					for (int e = 0; e < 4; ++e) rsum = rsum + sums[cur][4 * t + e];
+				}
 				if constexpr (decltype(issuing)::value) {
 #pragma unroll
 					for (int q = 0; q < S::L; ++q)
@@ -273,8 +283,13 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 #pragma unroll
 				for (int tt = 0; tt < 4; ++tt) {
 					if (kBurst ? t != 0 : tt != t) continue;
-					if (gi + 1 < NG) read_frags(slot, 16 * (gi + 1), tt, af[cur ^ 1], bf[cur ^ 1]);
-					else if (decltype(has_next)::value) read_frags(after, 0, tt, af[cur ^ 1], bf[cur ^ 1]);
+					if (gi + 1 < NG) {
+						read_frags(slot, 16 * (gi + 1), tt, af[cur ^ 1], bf[cur ^ 1]);
+						if (decltype(with_sums)::value) read_sums(slot, 16 * (gi + 1) + 4 * tt, sums[cur ^ 1] + 4 * tt);
+					} else if (decltype(has_next)::value) {
+						read_frags(after, 0, tt, af[cur ^ 1], bf[cur ^ 1]);
+						if (decltype(with_sums)::value) read_sums(after, 4 * tt, sums[cur ^ 1] + 4 * tt);
+					}
 				}
 #pragma unroll
 				for (int i = 0; i < I; ++i)
@@ -293,6 +308,16 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 			}
 		}
 		if constexpr (decltype(issuing)::value) advance();
+	};
+	auto compute = [&](int slot, int after, auto has_next, auto issuing, int fill) {
+		if constexpr (RS && kSpread) {
+			if (summing) return compute_stage(slot, after, has_next, issuing, fill, std::true_type{});
+		} else if (RS && summing) {
+			const float* As = lds + slot * S::kStage;
+#pragma unroll 8
+			for (int k = 0; k < BK; ++k) rsum = rsum + As[k * BM + (tid ^ ring::kswz<BM>(k))];
+		}
+		compute_stage(slot, after, has_next, issuing, fill, std::false_type{});
 	};
 	auto next = [](int slot) { return slot + 1 == ST ? 0 : slot + 1; };
 
@@ -320,6 +345,10 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 		ready(0, 0);
 #pragma unroll
 		for (int t = 0; t < 4; ++t) read_frags(0, 0, t, af[0], bf[0]);
+		if (RS && kSpread && summing) {
+#pragma unroll
+			for (int t = 0; t < 4; ++t) read_sums(0, 4 * t, sums[0] + 4 * t);
+		}
 		int kt = 0;
 		// whole iterations up to stage `end`, each issuing the (whole) stage ST - 1 ahead
 		auto run = [&](int end) {
@@ -372,7 +401,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 		tail(std::integral_constant<int, 0>{});
 		compute(slot, slot, std::false_type{}, std::false_type{}, 0);
 	}
-	if (RS && summing && m0 + tid < p.m) {
+	if (RS && summing && tid < BM && m0 + tid < p.m) {
 		float* d = p.rowsum + m0 + tid;
 		*d = p.rowsum_combine == 0 ? rsum : (p.rowsum_combine == 1 ? rsum + 0.0f : *d + rsum);
 	}

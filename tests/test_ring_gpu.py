@@ -151,3 +151,11 @@ def test_more_tiles_than_one_launch_takes(gpu, oracle):
     for i in (0, 1, batch // 2, batch - 2, batch - 1):
         want = oracle.sgemm(0, 0, m, n, k, a, k, b[i].cpu().numpy(), n, np.zeros((m, n), np.float32), n, 0)
         assert_same(host(c[i]).reshape(m, n), want, i)
+
+
+@pytest.mark.parametrize("M,K,n", [(128, 512, 512), (129, 300, 301), (191, 512, 128), (192, 256, 260), (320, 256, 256), (321, 255, 257),
+                                   (700, 1000, 900), (701, 1001, 899), (4100, 272, 260)])
+def test_row_sums_among_the_products(gpu, oracle, M, K, n):
+    """db beside dW at depths of two and more stages of each tile, whole and with a remainder: the sums' operands are read a
+    group of 16 depths ahead, across stages."""
+    test_ring_row_sums(gpu, oracle, M, K, n)
