@@ -255,7 +255,11 @@ bool ring_pair_takes(const GemmCall& g0, const GemmCall& g1) {
 	if (g0.batch_count != 1 || g1.batch_count != 1 || g0.batch.ndim != 0 || g1.batch.ndim != 0) return false;
 	if (g0.k < 128 || g1.k < 128 || ring_takes_large(g0) || ring_takes_large(g1)) return false;
 	auto tiles = [](const GemmCall& g) { return (double)((g.m + 31) / 32) * (double)((g.n + 31) / 32); };
-	return tiles(g0) >= 64 && tiles(g1) >= 64;
+	// A narrow dX (2^22 outputs and more, but fewer than 128 columns) counts as small here: beside a weight gradient of few
+	// tiles and a long depth it pays to start both at once (33056, 127, 520 580 -> 307). With row sums its deep aligned form is
+	// better off on its 128 x 64 tiles (48384, 96, 1216 645 us against 745, 40000, 120, 1000 541 against 633).
+	if (narrow(g0) && g1.rowsum && ring_vec(g0) && g0.k >= 1000) return false;
+	return tiles(g0) >= 64 && tiles(g1) >= 64 && tiles(g0) + tiles(g1) < 16777216.0;  // 2^32 work-items
 }
 
 hipError_t gemm_ring_pair_launch(const GemmCall& g0, const GemmCall& g1, hipStream_t s) {
@@ -264,7 +268,7 @@ hipError_t gemm_ring_pair_launch(const GemmCall& g0, const GemmCall& g1, hipStre
 	if (e != hipSuccess) return e;
 	const RingConfig& c = ring_configs()[kRing32x32];
 	const GemmArgs p0 = ring_args(g0, c), p1 = ring_args(g1, c);
-	const int b0 = p0.tiles_m * p0.tiles_n, b1 = p1.tiles_m * p1.tiles_n;  // below 176 x 4 each
+	const int b0 = p0.tiles_m * p0.tiles_n, b1 = p1.tiles_m * p1.tiles_n;
 	const auto fn = ring_pair_32x32(g0.tb ? 2 : g1.rowsum ? 1 : 0, ring_vec(g0) ? 1 : 0, ring_vec(g1) ? 1 : 0);
 	hipLaunchKernelGGL(fn, dim3((unsigned)(b0 + b1)), dim3((unsigned)c.threads), (size_t)c.lds_bytes, s, p0, p1, b0);
 	return hipGetLastError();

@@ -159,3 +159,18 @@ def test_row_sums_among_the_products(gpu, oracle, M, K, n):
     """db beside dW at depths of two and more stages of each tile, whole and with a remainder: the sums' operands are read a
     group of 16 depths ahead, across stages."""
     test_ring_row_sums(gpu, oracle, M, K, n)
+
+
+@pytest.mark.parametrize("M,K,n", [(33056, 127, 520), (41952, 100, 1000)])
+def test_narrow_layer_backward(gpu, oracle, M, K, n):
+    """dX of 2^22 outputs and fewer than 128 columns beside a dW of some 32 x 32 tiles: a pair, and on its own."""
+    import torch
+
+    import nnh
+    x, w, g = synth.normal(81, (M, K)), synth.normal(82, (n, K)), synth.normal(83, (M, n))
+    want = oracle.linear_backward(g, x, w, dx=np.zeros_like(x), dw=np.zeros_like(w), db=np.zeros(n, np.float32))
+    xd, wd, gd = (torch.from_numpy(a).cuda() for a in (x, w, g))
+    dx, dw, db = torch.empty_like(xd), torch.empty_like(wd), torch.empty(n, device="cuda")
+    nnh.linear_backward(gd, xd, wd, dx=dx, dw=dw, db=db)
+    for got, ref, what in ((dx, want[0], "dx"), (dw, want[1], "dw"), (db, want[2], "db")):
+        assert_same(host(got), ref, what)
