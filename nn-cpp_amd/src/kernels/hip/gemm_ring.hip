@@ -171,7 +171,7 @@ bool ring_takes(const GemmCall& g) {
 			       (g.k > 100 && one_round && blocks <= 1024 && batch > 1);
 		if (g.ta) return one_round && g.n > 15 && (vec || g.k < 128);
 		// A B^T: 64 x 1500 x 128 5.1, 4.6; 200 of 1 x 128 x 128 7.6, 9.0; 111 of 64 x 126 x 103 17.4, 11.3
-		if (g.tb) return vec ? one_round && padded <= 2 : (g.k > 112 || padded <= 4) && (g.m > 16 || g.n > 16);
+		if (g.tb) return vec ? padded <= 2 && (one_round || (g.m > 32 && g.n > 32)) : (g.k > 112 || padded <= 4) && (g.m > 16 || g.n > 16);
 		// A B: 64 x 1500 x 128 4.6, 4.4; 4 of 2 x 4032 x 112 4.8, 5.5; 11 of 5 x 5553 x 112 12.9, 20.2
 		return one_round && g.m > 20 && (vec || (g.k > 112 && g.k < 128));
 	}
