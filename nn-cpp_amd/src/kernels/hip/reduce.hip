@@ -2,6 +2,8 @@
 // (bias gradients), the ReLU node, and gradient stores with nn-cpp's first-write rule.
 #include "reduce.hpp"
 
+#include <type_traits>
+
 namespace nnh {
 
 namespace {
@@ -303,11 +305,22 @@ __global__ void __launch_bounds__(256) sum_rows2_quad_kernel(const float* __rest
 #pragma unroll
 				for (int c = 0; c < 4; ++c) acc[c] = acc[c] + v[u][c];
 		}
-		for (; a < r0; ++a) {
-			const f32x4 v = *reinterpret_cast<const f32x4*>(p + a * sa);
+		auto few = [&](auto count) {  // the rest: a batch for each bit of its count
+			constexpr int n = decltype(count)::value;
+			if (!((r0 - a) & n)) return;
+			f32x4 v[n];
 #pragma unroll
-			for (int c = 0; c < 4; ++c) acc[c] = acc[c] + v[c];
-		}
+			for (int u = 0; u < n; ++u) v[u] = *reinterpret_cast<const f32x4*>(p + (a + u) * sa);
+#pragma unroll
+			for (int u = 0; u < n; ++u)
+#pragma unroll
+				for (int c = 0; c < 4; ++c) acc[c] = acc[c] + v[u][c];
+			a += n;
+		};
+		few(std::integral_constant<int, 8>{});
+		few(std::integral_constant<int, 4>{});
+		few(std::integral_constant<int, 2>{});
+		few(std::integral_constant<int, 1>{});
 #pragma unroll
 		for (int c = 0; c < 4; ++c) part[c * kQ2Pitch + b] = acc[c];
 	}
@@ -337,7 +350,12 @@ bool sum_rows2_fits(int64_t r0, int64_t r1, int64_t inner) {
 
 hipError_t sum_rows2(const float* src, int64_t r0, int64_t r1, int64_t inner, float* dst, int combine, hipStream_t s) {
 	if (!sum_rows2_fits(r0, r1, inner)) return hipErrorInvalidValue;
-	if (inner % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0) {
+	// Four columns a workgroup against sixteen (us): [32, 256, 512] 8.6 against 13.4, [8, 24, 512] as fast. Wide rows give the
+	// sixteen enough workgroups, and four leave most of a workgroup idle where axis 1 is short ([5, 18, 7952] 5.1 against 3.5,
+	// [13, 11, 7108] 6.5 against 4.9); past the caches 16-byte pieces of middling rows lose ([194, 95, 2144] 70 against 49).
+	const bool fills = inner <= 3000 || r1 >= 124 || r0 >= 18;
+	const bool cached = r0 * r1 * inner <= 25000000 || inner <= 1024 || inner >= 3600;
+	if (inner % 4 == 0 && fills && cached && reinterpret_cast<uintptr_t>(src) % 16 == 0) {
 		hipLaunchKernelGGL(sum_rows2_quad_kernel, dim3((unsigned)(inner / 4)), dim3(256), 0, s, src, (int)r0, (int)r1,
 		                   (int)inner, dst, combine);
 		return hipGetLastError();

@@ -27,3 +27,11 @@ def test_two_axis_bias_gradient(gpu, oracle, r0, r1, n, first):
         x, w = torch.zeros(r0, r1, 4, device="cuda"), torch.zeros(n, 4, device="cuda")
         nnh.linear_backward(buf[off:].view(r0, r1, n), x, w, db=db, db_first=first)
         assert_same(db.cpu().numpy(), want, (r0, r1, n, first, off))
+
+
+@pytest.mark.parametrize("r0,r1,n", [(1, 2, 2996), (14, 5, 3000), (23, 3, 3004), (17, 123, 3004), (18, 3, 3004), (7, 124, 3004),
+                                     (31, 64, 12), (46, 130, 4184), (46, 140, 3596), (8, 24, 512)])
+@pytest.mark.parametrize("first", [True, False])
+def test_two_axis_bias_gradient_routes(gpu, oracle, r0, r1, n, first):
+    """Both sides of where four columns a workgroup are taken, and every count of a last batch of loads."""
+    test_two_axis_bias_gradient(gpu, oracle, r0, r1, n, first)
