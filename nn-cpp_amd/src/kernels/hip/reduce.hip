@@ -352,10 +352,11 @@ hipError_t sum_rows2(const float* src, int64_t r0, int64_t r1, int64_t inner, fl
 	if (!sum_rows2_fits(r0, r1, inner)) return hipErrorInvalidValue;
 	// Four columns a workgroup against sixteen (us): [32, 256, 512] 8.6 against 13.4, [8, 24, 512] as fast. Wide rows give the
 	// sixteen enough workgroups, and four leave most of a workgroup idle where axis 1 is short ([5, 18, 7952] 5.1 against 3.5,
-	// [13, 11, 7108] 6.5 against 4.9); past the caches 16-byte pieces of middling rows lose ([194, 95, 2144] 70 against 49).
+	// [13, 11, 7108] 6.5 against 4.9); past the caches 16-byte pieces of middling rows lose ([194, 95, 2144] 70 against 49). A
+	// launch holds fewer than 2^24 workgroups.
 	const bool fills = inner <= 3000 || r1 >= 124 || r0 >= 18;
 	const bool cached = r0 * r1 * inner <= 25000000 || inner <= 1024 || inner >= 3600;
-	if (inner % 4 == 0 && fills && cached && reinterpret_cast<uintptr_t>(src) % 16 == 0) {
+	if (inner % 4 == 0 && inner < (1 << 26) && fills && cached && reinterpret_cast<uintptr_t>(src) % 16 == 0) {
 		hipLaunchKernelGGL(sum_rows2_quad_kernel, dim3((unsigned)(inner / 4)), dim3(256), 0, s, src, (int)r0, (int)r1,
 		                   (int)inner, dst, combine);
 		return hipGetLastError();

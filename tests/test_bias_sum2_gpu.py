@@ -35,3 +35,19 @@ def test_two_axis_bias_gradient(gpu, oracle, r0, r1, n, first):
 def test_two_axis_bias_gradient_routes(gpu, oracle, r0, r1, n, first):
     """Both sides of where four columns a workgroup are taken, and every count of a last batch of loads."""
     test_two_axis_bias_gradient(gpu, oracle, r0, r1, n, first)
+
+
+def test_more_columns_than_one_launch_takes_by_four(gpu):
+    """2^26 columns, four of them a workgroup, would be 2^32 work-items."""
+    import torch
+
+    import nnh
+    r0, n = 18, 1 << 26
+    g = torch.empty(r0, 1, n, device="cuda").uniform_(-1, 1, generator=torch.Generator(device="cuda").manual_seed(9))
+    x, w = torch.zeros(r0, 1, 1, device="cuda"), torch.zeros(n, 1, device="cuda")
+    db = torch.empty(n, device="cuda")
+    nnh.linear_backward(g, x, w, db=db)
+    want = torch.zeros(n, device="cuda")
+    for i in range(r0):
+        want += g[i, 0]
+    assert torch.equal(db, want)
