@@ -18,6 +18,9 @@
 // workgroups a CU 85, 32 rows 81, and 74 with a third of the vector instructions taken out (rows summed by one wave
 // for 32 rows at once, V's addresses kept uniform, no division by Tk, one test for 16 exponentials' special cases).
 #include "attention.hpp"
+
+#include <algorithm>
+
 #include "gemm.hpp"
 
 #include "gemm_tile.hpp"
@@ -30,6 +33,7 @@ namespace {
 constexpr int kRows = 32;          // query rows per workgroup
 constexpr int kDh = 64;            // head width
 constexpr int kMaxKeys = 256;     // four waves of 64 keys
+constexpr int64_t kMaxGrid = ((int64_t)1 << 24) - 1;  // workgroups of 256 threads: below 2^32 work-items a launch
 
 struct FusedArgs {
 	const float* q;
@@ -39,7 +43,7 @@ struct FusedArgs {
 	float* probs;
 	const float* pad;  // {N, Tk}, 0 marks a padded key; or null
 	int heads, tq, tk, d;
-	int qblocks, total;
+	int qblocks, total, first;  // blocks of a (sample, head) pair and of this launch, this launch's first block
 	int causal;
 	float scale;
 };
@@ -112,7 +116,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) a
 	__shared__ float rowmax[kRows], rowsum[kRows];
 	__shared__ double rowinv[kRows];
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	const int lid = xcd_remap(blockIdx.x, a.total);  // the query blocks of one head share an XCD's L2
+	const int lid = a.first + xcd_remap(blockIdx.x, a.total);  // the query blocks of one head share an XCD's L2
 	const int nh = lid / a.qblocks, qb = lid - nh * a.qblocks;
 	const int n = nh / a.heads, h = nh - n * a.heads;
 	const int i0 = qb * kRows, nq = min(kRows, a.tq - i0);
@@ -378,7 +382,7 @@ struct DScoresArgs {
 	float* ds;           // {N, heads, Tq, Tk}
 	const float* pad;
 	int heads, tq, tk, d;
-	int qblocks, total;
+	int qblocks, total, first;  // blocks of a (sample, head) pair and of this launch, this launch's first block
 	int causal;
 	float scale;
 };
@@ -394,7 +398,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) a
 	extern __shared__ __align__(16) float sm[];
 	__shared__ float rowdot[kRows];
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	const int lid = xcd_remap(blockIdx.x, a.total);
+	const int lid = a.first + xcd_remap(blockIdx.x, a.total);
 	const int nh = lid / a.qblocks, qb = lid - nh * a.qblocks;
 	const int n = nh / a.heads, h = nh - n * a.heads;
 	const int i0 = qb * kRows, nq = min(kRows, a.tq - i0);
@@ -520,15 +524,20 @@ hipError_t attention_fused_forward(const float* q, const float* k, const float* 
 	a.tk = (int)tk;
 	a.d = (int)d;
 	a.qblocks = (int)qblocks;
-	a.total = (int)total;
 	a.causal = causal ? 1 : 0;
 	a.scale = scale;
 	const int lds = 4 * kRows * score_stride((int)tk);
 	hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_fused_kernel),
 	                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds);
 	if (e != hipSuccess) return e;
-	hipLaunchKernelGGL(attention_fused_kernel, dim3((unsigned)total), dim3(256), lds, s, a);
-	return hipGetLastError();
+	for (int64_t first = 0; first < total; first += kMaxGrid) {
+		a.first = (int)first;
+		a.total = (int)std::min(kMaxGrid, total - first);
+		hipLaunchKernelGGL(attention_fused_kernel, dim3((unsigned)a.total), dim3(256), lds, s, a);
+		e = hipGetLastError();
+		if (e != hipSuccess) return e;
+	}
+	return hipSuccess;
 }
 
 hipError_t attention_fused_dscores(const float* g, const float* v, const float* probs, int64_t n, int64_t tq, int64_t tk,
@@ -548,15 +557,20 @@ hipError_t attention_fused_dscores(const float* g, const float* v, const float* 
 	a.tk = (int)tk;
 	a.d = (int)d;
 	a.qblocks = (int)qblocks;
-	a.total = (int)total;
 	a.causal = causal ? 1 : 0;
 	a.scale = scale;
 	const int lds = 4 * kRows * score_stride((int)tk);
 	hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_dscores_kernel),
 	                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds);
 	if (e != hipSuccess) return e;
-	hipLaunchKernelGGL(attention_dscores_kernel, dim3((unsigned)total), dim3(256), lds, s, a);
-	return hipGetLastError();
+	for (int64_t first = 0; first < total; first += kMaxGrid) {
+		a.first = (int)first;
+		a.total = (int)std::min(kMaxGrid, total - first);
+		hipLaunchKernelGGL(attention_dscores_kernel, dim3((unsigned)a.total), dim3(256), lds, s, a);
+		e = hipGetLastError();
+		if (e != hipSuccess) return e;
+	}
+	return hipSuccess;
 }
 
 }  // namespace nnh
