@@ -50,7 +50,9 @@ struct FusedArgs {
 
 // LDS row stride of the scores: whole groups of 16 keys (four steps of the 16x16x4 product for each lane group) and
 // four floats more, so that the 16-byte reads of 16 rows hit distinct banks.
-__host__ __device__ inline int score_stride(int tk) { return (tk + 15) / 16 * 16 + 4; }
+__host__ __device__ constexpr int score_stride(int tk) { return (tk + 15) / 16 * 16 + 4; }
+
+static_assert(4 * kRows * score_stride(kMaxKeys) <= 64 * 1024, "no launch asks for more LDS than the default limit");
 
 // The 64-float rows' operand of the 16x16x4 product from 16-byte loads: lane (g, i) loads floats 16c + 4g .. + 3 of
 // its row i and needs floats 16c + 4s + g (s = 0..3), the transpose of four registers over the four lane groups.
@@ -527,14 +529,11 @@ hipError_t attention_fused_forward(const float* q, const float* k, const float* 
 	a.causal = causal ? 1 : 0;
 	a.scale = scale;
 	const int lds = 4 * kRows * score_stride((int)tk);
-	hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_fused_kernel),
-	                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-	if (e != hipSuccess) return e;
 	for (int64_t first = 0; first < total; first += kMaxGrid) {
 		a.first = (int)first;
 		a.total = (int)std::min(kMaxGrid, total - first);
 		hipLaunchKernelGGL(attention_fused_kernel, dim3((unsigned)a.total), dim3(256), lds, s, a);
-		e = hipGetLastError();
+		const hipError_t e = hipGetLastError();
 		if (e != hipSuccess) return e;
 	}
 	return hipSuccess;
@@ -560,14 +559,11 @@ hipError_t attention_fused_dscores(const float* g, const float* v, const float* 
 	a.causal = causal ? 1 : 0;
 	a.scale = scale;
 	const int lds = 4 * kRows * score_stride((int)tk);
-	hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_dscores_kernel),
-	                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-	if (e != hipSuccess) return e;
 	for (int64_t first = 0; first < total; first += kMaxGrid) {
 		a.first = (int)first;
 		a.total = (int)std::min(kMaxGrid, total - first);
 		hipLaunchKernelGGL(attention_dscores_kernel, dim3((unsigned)a.total), dim3(256), lds, s, a);
-		e = hipGetLastError();
+		const hipError_t e = hipGetLastError();
 		if (e != hipSuccess) return e;
 	}
 	return hipSuccess;

@@ -18,7 +18,7 @@
 //     holds four consecutive columns of a row of C and stores them as one 16-byte word, with no transpose through LDS.
 //   * V = 1 loads one float per lane instead of four, for rows that are not 16-byte aligned or whose length is not a
 //     multiple of four: four times the load instructions, still far below the MFMAs' issue time.
-// Rows and columns past the edge are read from the last valid ones (their outputs are not stored); depth past k is
+// The depth is at least one (ring_ok). Rows and columns past the edge are read from the last valid ones (their outputs are not stored); depth past k is
 // read from the last valid depth and then overwritten in LDS with the padding.
 #pragma once
 
@@ -42,15 +42,14 @@ struct RingShape {
 	// k-contiguous operands stored in fragment order (ring::kc_index), where one float a lane is loaded anyway. Loading
 	// single floats for its sake cost more than its quarter of the reads gave (512^3 A B on 32 x 32 tiles 7.1 -> 7.7 us).
 	static constexpr bool kFrag = V == 1;
-	static constexpr int VA = !TA && kFrag ? 1 : V, VB = TB && kFrag ? 1 : V;  // floats a lane loads
-	static constexpr int kPerA = 64 * VA, kPerB = 64 * VB;                     // floats a load instruction moves
-	static constexpr int LA = kA / (kPerA * kWaves), LB = kB / (kPerB * kWaves);
+	static constexpr int kPer = 64 * V;  // floats a load instruction moves
+	static constexpr int LA = kA / (kPer * kWaves), LB = kB / (kPer * kWaves);
 	static constexpr int L = LA + LB;        // load instructions of a wave per stage
 	static constexpr int kLdsBytes = ST * kStage * 4;
-	static_assert(LA * kPerA * kWaves == kA && LB * kPerB * kWaves == kB, "a stage splits evenly over the waves");
+	static_assert(LA * kPer * kWaves == kA && LB * kPer * kWaves == kB, "a stage splits evenly over the waves");
 	static_assert(WM % 16 == 0 && WN % 16 == 0 && BM % WM == 0 && BN % WN == 0, "whole 16 x 16 blocks");
 	static_assert(BK % 32 == 0 && kAccAfter % BK == 0, "an even number of 16-deep groups; 256 on a stage boundary");
-	static_assert(ST >= 3 && ST <= 8, "the tail is written out for 8 stages");
+	static_assert(ST >= 3 && ST <= 5, "the tail is written out for 5 stages");
 	// the wait that leaves `stages` whole stages outstanding (a wave counts at most 63 loads: then it waits for more)
 	static constexpr int waits(int stages) { return stages * L < 63 ? stages * L : 63; }
 	static_assert(kLdsBytes <= 160 * 1024, "gfx950 has 160 KiB of LDS per CU");
@@ -148,26 +147,24 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 	unsigned offa[S::LA], offb[S::LB];
 #pragma unroll
 	for (int q = 0; q < S::LA; ++q)
-		offa[q] = ring::src_offset<!TA, S::kFrag, BM, BK, S::VA>(wave * S::LA + q, lane, p.lda, rows_a, BK);
+		offa[q] = ring::src_offset<!TA, S::kFrag, BM, BK, V>(wave * S::LA + q, lane, p.lda, rows_a, BK);
 #pragma unroll
 	for (int q = 0; q < S::LB; ++q)
-		offb[q] = ring::src_offset<TB, S::kFrag, BN, BK, S::VB>(wave * S::LB + q, lane, p.ldb, rows_b, BK);
+		offb[q] = ring::src_offset<TB, S::kFrag, BN, BK, V>(wave * S::LB + q, lane, p.ldb, rows_b, BK);
 
-	auto dma = [&](auto width, const float* src, unsigned off, float* dst) {
-		if constexpr (decltype(width)::value == 4)
+	auto dma = [&](const float* src, unsigned off, float* dst) {
+		if constexpr (V == 4)
 			__builtin_amdgcn_global_load_lds((ring::global_void*)(src + off), (ring::lds_void*)dst, 16, 0, 0);
 		else
 			__builtin_amdgcn_global_load_lds((ring::global_void*)(src + off), (ring::lds_void*)dst, 4, 0, 0);
 	};
-	constexpr std::integral_constant<int, S::VA> va{};
-	constexpr std::integral_constant<int, S::VB> vb{};
 	// The wave's load instruction q (0 .. L - 1) of the next stage, whole, into ring slot `slot`; advance() follows the
 	// last. Stages are issued in order.
 	auto issue_one = [&](int q, int slot) {
-		float* As = lds + slot * S::kStage + wave * S::LA * S::kPerA;
-		float* Bs = lds + slot * S::kStage + S::kA + wave * S::LB * S::kPerB;
-		if (q < S::LA) dma(va, a_next, offa[q < S::LA ? q : 0], As + q * S::kPerA);
-		else dma(vb, b_next, offb[q >= S::LA ? q - S::LA : 0], Bs + (q - S::LA) * S::kPerB);
+		float* As = lds + slot * S::kStage + wave * S::LA * S::kPer;
+		float* Bs = lds + slot * S::kStage + S::kA + wave * S::LB * S::kPer;
+		if (q < S::LA) dma(a_next, offa[q < S::LA ? q : 0], As + q * S::kPer);
+		else dma(b_next, offb[q >= S::LA ? q - S::LA : 0], Bs + (q - S::LA) * S::kPer);
 	};
 	auto advance = [&]() {
 		a_next += a_step;
@@ -176,16 +173,16 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 	// All of stage kt at once; a partial last stage loads nothing past the depth.
 	auto issue = [&](int kt, int slot) {
 		if (krem != BK && kt == nkt - 1) {
-			float* As = lds + slot * S::kStage + wave * S::LA * S::kPerA;
-			float* Bs = lds + slot * S::kStage + S::kA + wave * S::LB * S::kPerB;
+			float* As = lds + slot * S::kStage + wave * S::LA * S::kPer;
+			float* Bs = lds + slot * S::kStage + S::kA + wave * S::LB * S::kPer;
 #pragma unroll
 			for (int q = 0; q < S::LA; ++q)
-				dma(va, a_next, ring::src_offset<!TA, S::kFrag, BM, BK, S::VA>(wave * S::LA + q, lane, p.lda, rows_a, krem),
-				    As + q * S::kPerA);
+				dma(a_next, ring::src_offset<!TA, S::kFrag, BM, BK, V>(wave * S::LA + q, lane, p.lda, rows_a, krem),
+				    As + q * S::kPer);
 #pragma unroll
 			for (int q = 0; q < S::LB; ++q)
-				dma(vb, b_next, ring::src_offset<TB, S::kFrag, BN, BK, S::VB>(wave * S::LB + q, lane, p.ldb, rows_b, krem),
-				    Bs + q * S::kPerB);
+				dma(b_next, ring::src_offset<TB, S::kFrag, BN, BK, V>(wave * S::LB + q, lane, p.ldb, rows_b, krem),
+				    Bs + q * S::kPer);
 			return;
 		}
 #pragma unroll
@@ -336,6 +333,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 					if (row < p.m && col < p.n) acc[i][j][e] = Cp[(int64_t)row * p.ldc + col] + acc[i][j][e];
 				}
 	};
+	// always so; without the test the compiler's code is 2% slower (1000 x 1000 x 100 8.56 us against 8.34)
 	if (nkt > 0) {
 		int fill = 0, slot = 0;  // the slots the next issued and the next computed stage take
 		const int first = min(ST - 1, nkt);
@@ -393,9 +391,6 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 			++kt;
 			add_at_mid();
 		};
-		if constexpr (ST >= 8) tail(std::integral_constant<int, 5>{});
-		if constexpr (ST >= 7) tail(std::integral_constant<int, 4>{});
-		if constexpr (ST >= 6) tail(std::integral_constant<int, 3>{});
 		if constexpr (ST >= 5) tail(std::integral_constant<int, 2>{});
 		if constexpr (ST >= 4) tail(std::integral_constant<int, 1>{});
 		tail(std::integral_constant<int, 0>{});
@@ -429,7 +424,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 				if (old_at_end) {
 					const f32x4 old = *reinterpret_cast<const f32x4*>(Cp + off);
 #pragma unroll
-					for (int e = 0; e < 4; ++e) v[e] = p.k > 0 ? old[e] + v[e] : old[e];
+					for (int e = 0; e < 4; ++e) v[e] = old[e] + v[e];
 				}
 				if (p.ep.bias_mode == kBiasCol) {
 #pragma unroll
@@ -469,7 +464,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& p, int block) {
 			for (int e = 0; e < 4; ++e) {
 				if (e >= nc) continue;
 				float x = v[e];
-				if (old_at_end) x = p.k > 0 ? Cp[off + e] + x : Cp[off + e];
+				if (old_at_end) x = Cp[off + e] + x;
 				if (p.ep.bias_mode == kBiasCol) x = x + p.ep.bias[col + e];
 				else if (p.ep.bias_mode == kBiasRow) x = x + p.ep.bias[row];
 				if (res) x = res[off + e] + x;
