@@ -120,7 +120,7 @@ struct Epilogue {
 	unsigned char* alive;  // optional, addressed like C
 	// optional, addressed like C: added after the bias as res + v, the reference's add(residual, linear(...))
 	const float* res;
-	// optional, addressed like C, the chain kernel only (gemm_direct.hpp): GELU of the stored value (ops.cpp:461-466)
+	// optional, addressed like C, the chain kernel (gemm_direct.hpp) and the ring kernel (gemm_ring.hpp) only: GELU of the stored value (ops.cpp:461-466)
 	// into gelu_y and its tanh into gelu_t, the reference's gelu(linear(...)) with C its input
 	float* gelu_y;
 	float* gelu_t;

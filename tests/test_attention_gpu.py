@@ -107,7 +107,7 @@ def test_baseline_config4(gpu, oracle, causal):
         assert np.all(probs[:, :, tri] == 0.0)
 
 
-# Head width 64, Tk <= 256, Tk % 4 == 0: the fused forward kernel (one workgroup per 64 query rows). Ragged query
+# Head width 64, Tk <= 256, Tk % 4 == 0: the fused forward kernel (one workgroup per 32 query rows). Ragged query
 # blocks, key counts that do not fill a wave's 64 keys, causal rows, padded keys.
 FUSED_SHAPES = [  # (N, Tq, Tk, heads, causal, masked)
     (2, 1, 4, 1, False, False),
@@ -116,7 +116,7 @@ FUSED_SHAPES = [  # (N, Tq, Tk, heads, causal, masked)
     (2, 100, 100, 2, True, True),
     (1, 130, 252, 3, False, True),
     (2, 256, 256, 2, True, True),
-    # Tk a multiple of 16: O = P V on 16x16x4 (ragged and whole 64-row blocks, key counts that are not a multiple of
+    # Tk a multiple of 16: O = P V on 16x16x4 (ragged and whole 32-row blocks, key counts that are not a multiple of
     # 64)
     (2, 48, 160, 2, False, True),
     (1, 16, 16, 1, True, False),

@@ -101,8 +101,8 @@ def test_linear_golden(gpu):
 
 def test_linear_forward_add(gpu, oracle):
     """nnh_linear_forward_add: y = residual + linear(x, w, b), bit for bit the oracle's linear and then the float
-    add, on shapes each GEMM route takes (the tile kernel, the VALU kernel, the chain kernel, the pieces kernels and
-    a cut of more than 16 pieces with its partials), with -0, infinities and NaN in the residual, in place (y is the
+    add, on shapes of each GEMM route but the ring's (the tile kernel, the VALU kernel, the chain kernel, the pieces kernels
+    and a cut of more than 16 pieces with its partials; the ring's are in test_ring_gpu.py), with -0, infinities and NaN in the residual, in place (y is the
     residual), and refused when the residual overlaps y other than in place."""
     import torch
 

@@ -174,3 +174,64 @@ def test_narrow_layer_backward(gpu, oracle, M, K, n):
     nnh.linear_backward(gd, xd, wd, dx=dx, dw=dw, db=db)
     for got, ref, what in ((dx, want[0], "dx"), (dw, want[1], "dw"), (db, want[2], "db")):
         assert_same(host(got), ref, what)
+
+
+@pytest.mark.parametrize("bias", ["none", "col", "row"])
+@pytest.mark.parametrize("relu", [False, True])
+def test_ring_epilogue(gpu, oracle, bias, relu):
+    """Every tile's store with a bias down the columns or along the rows, ReLU with its flags, fresh and accumulated below and
+    past 256 deep: 16-byte aligned rows, ragged ones, and a batch whose C and flags have a stride between matrices."""
+    import torch
+
+    import nnh
+    mode = {"none": nnh.BIAS_NONE, "col": nnh.BIAS_COL, "row": nnh.BIAS_ROW}[bias]
+    seed = 93000
+    for name, cfg in ring_configs().items():
+        bm, bn = (int(v) for v in name.split()[1].split("_")[0].split("x"))
+        for batch, m, n, k, pad in ((1, bm, bn + 4, 40, 0), (1, bm - 1, bn + 3, 300, 1), (3, bm + 5, bn - 2, 33, 3), (2, bm, bn, 288, 0)):
+            lda, ldb, ldc = k + pad, n + pad, n + pad
+            a, b = synth.normal(seed, (batch, m, lda)), synth.normal(seed + 1, (batch, k, ldb))
+            gap = 8  # floats of C between two matrices that belong to neither
+            c0 = synth.normal(seed + 2, (batch, m * ldc + gap))
+            bv = synth.normal(seed + 3, (n if bias == "col" else m,))
+            seed += 4
+            for acc in (0, 1):
+                c, flags = torch.from_numpy(c0).cuda(), torch.full(c0.shape, 7, dtype=torch.uint8, device="cuda")
+                bd = torch.from_numpy(bv).cuda()
+                ep = nnh.make_epilogue(mode, bd if bias != "none" else None, relu, flags if relu else None)
+                nnh.sgemm_batched(0, 0, m, n, k, torch.from_numpy(a).cuda(), lda, torch.from_numpy(b).cuda(), ldb, c, ldc, acc,
+                                  nnh.make_batch((batch,), (m * lda,), (k * ldb,), (m * ldc + gap,)), ep, cfg)
+                want, alive = c0.copy(), np.full(c0.shape, 7, np.uint8)
+                for i in range(batch):
+                    full = oracle.sgemm(0, 0, m, n, k, a[i], lda, b[i], ldb, c0[i, :m * ldc].reshape(m, ldc).copy(), ldc, acc)
+                    v = full[:, :n]
+                    v = v + bv[None, :] if bias == "col" else v + bv[:, None] if bias == "row" else v
+                    if relu:
+                        alive[i, :m * ldc].reshape(m, ldc)[:, :n] = v > 0
+                        v = np.where(v > 0, v, np.float32(0))
+                    want[i, :m * ldc].reshape(m, ldc)[:, :n] = v
+                what = (name, bias, relu, batch, m, n, k, pad, acc)
+                assert_same(host(c), want, what)
+                if relu:
+                    assert np.array_equal(host(flags), alive), what
+
+
+@pytest.mark.parametrize("M,K,n", [(1024, 512, 768), (777, 130, 1021)])
+def test_ring_residual(gpu, oracle, M, K, n):
+    """A layer with its residual through the ring, fresh and in the residual's place, with -0, infinities and NaN in it."""
+    import torch
+
+    import nnh
+    x, w, b, r = synth.normal(41, (M, K)), synth.normal(42, (n, K)), synth.normal(43, (n,)), synth.normal(44, (M, n))
+    r[0, :4] = [-0.0, np.inf, -np.inf, np.nan]
+    want = r + oracle.linear_forward(x, w, b)
+    xd, wd, bd, rd = (torch.from_numpy(a).cuda() for a in (x, w, b, r))
+    assert_same(host(nnh.linear_forward_add(xd, wd, bd, rd)), want, ("residual", M, K, n), nan_equal=True)
+    nnh.linear_forward_add(xd, wd, bd, rd, out=rd)
+    assert_same(host(rd), want, ("in place", M, K, n), nan_equal=True)
+
+
+@pytest.mark.parametrize("M,K,n", [(1000, 256, 900), (300, 160, 900), (1700, 100, 1000), (1000, 252, 900), (61, 128, 900)])
+def test_gelu_routes(gpu, oracle, M, K, n):
+    """Aligned layers with GELU on both sides of the line between the ring and the chain kernel."""
+    test_ring_gelu(gpu, oracle, M, K, n)

@@ -2,7 +2,8 @@
 division, the reference's `o[j] /= sum` (src/autograd/ops.cpp:1203).
 
 The GPU computes q = (double)p * (1 / (double)s), rounds q to float, and takes the float division only for
-positive quotients below 2^-125. numpy's float64 product, float64 reciprocal and float64 -> float32 conversion are
+positive quotients below 2^-125. Where it divides several values of a row at once (div_n_by_row_sum) one look at the
+smallest positive p, below 2^-100, decides whether any of them is looked at: `grouped` models that test. numpy's float64 product, float64 reciprocal and float64 -> float32 conversion are
 the same IEEE operations (round to nearest even, subnormals kept) as the GPU's v_mul_f64, the f64 division and
 v_cvt_f32_f64, so this checks the method itself. The operands are those a softmax row can produce (0 <= p <= s,
 s up to a few thousand) and the hardest ones for the method: quotients within a few double ulps of a float
@@ -85,3 +86,44 @@ def test_special_operands():
     s = np.array([1, 0, nan, nan, 3, 2 ** -149, 2 ** -149, 0.5, 6, 0.75, inf], np.float32)
     check(p, s, "special operands")
     assert method(np.float32(0), np.float32(5)).view(np.uint32) == 0  # +0, as 0 / s
+
+
+def grouped(p, s):
+    """div_n_by_row_sum on groups (rows of p) of values with one sum each."""
+    with np.errstate(divide="ignore", invalid="ignore", over="ignore", under="ignore"):
+        q = p.astype(np.float64) * (1.0 / s.astype(np.float64))[:, None]
+        smallest = (p.view(np.uint32) - np.uint32(1)).min(axis=1)  # p = 0 wraps to the largest
+        looks = smallest < np.uint32(0x0d800000)
+        tiny = looks[:, None] & (q > 0.0) & (q < 2.0 ** -125)
+        return np.where(tiny, p / s[:, None], q.astype(np.float32))
+
+
+def test_one_look_at_a_group():
+    """Groups mixing zeros, subnormals, values around 2^-100 and 2^-125 times the sum, ordinary ones and NaN, for sums from 1 to
+    the longest row: the prefilter lets no quotient that needs the float division through."""
+    rng = np.random.default_rng(23)
+    n, width = 400_000, 16
+    s = random_floats(rng, n, 0x3f800000, 0x4b800000)  # [1, 2^24)
+    s[: n // 4] = 2.0 ** rng.integers(0, 25, n // 4)
+    p = random_floats(rng, n * width, 0x00000001, 0x3f800001).reshape(n, width).copy()
+    kind = rng.integers(0, 8, (n, width))
+    p[kind == 0] = 0.0
+    p[kind == 1] = random_floats(rng, int((kind == 1).sum()), 0x00000001, 0x00800000)  # subnormal
+    near = (0x0d800000 + rng.integers(-4, 5, (n, width))).astype(np.uint32).view(np.float32)  # around 2^-100
+    p = np.where(kind == 2, near, p).astype(np.float32)
+    edge = (s[:, None].astype(np.float64) * 2.0 ** -125 * rng.uniform(0.98, 1.02, (n, width))).astype(np.float32)
+    p = np.where(kind == 3, edge, p).astype(np.float32)
+    p[rng.integers(0, n, 2000), rng.integers(0, width, 2000)] = np.nan
+    got, want = grouped(p, s), ieee(p, s[:, None] + np.zeros_like(p))
+    bad = (got.view(np.uint32) != want.view(np.uint32)) & ~(np.isnan(got) & np.isnan(want))
+    assert not bad.any(), (int(bad.sum()), p[bad][:4], got[bad][:4], want[bad][:4])
+
+
+def test_expf_special_prefilter():
+    """expf_glibc_n looks at the largest |x| of a group as bits above the sign: the same test as expf_is_special on each, for
+    every bit pattern near the limit, the infinities and the NaNs, of both signs."""
+    near = np.concatenate([np.arange(0x42b00000 - 5000, 0x42b00000 + 5000), np.arange(0x7f800000 - 5000, 0x7f800000 + 5000),
+                           np.arange(0, 5000), np.arange(0x7fffffff - 5000, 0x80000000)]).astype(np.uint64)
+    bits = np.concatenate([near, near | 0x80000000]).astype(np.uint32)
+    special = ((bits >> 20) & 0x7ff) >= 0x42b
+    assert np.array_equal((bits << np.uint32(1)) >= np.uint32((0x42b00000 << 1) & 0xffffffff), special)
