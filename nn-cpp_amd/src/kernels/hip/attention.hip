@@ -43,7 +43,7 @@ struct FusedArgs {
 	float* probs;
 	const float* pad;  // {N, Tk}, 0 marks a padded key; or null
 	int heads, tq, tk, d;
-	int qblocks, total, first;  // blocks of a (sample, head) pair and of this launch, this launch's first block
+	int qblocks, total;
 	int causal;
 	float scale;
 };
@@ -118,7 +118,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) a
 	__shared__ float rowmax[kRows], rowsum[kRows];
 	__shared__ double rowinv[kRows];
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	const int lid = a.first + xcd_remap(blockIdx.x, a.total);  // the query blocks of one head share an XCD's L2
+	const int lid = xcd_remap(blockIdx.x, a.total);  // the query blocks of one head share an XCD's L2
 	const int nh = lid / a.qblocks, qb = lid - nh * a.qblocks;
 	const int n = nh / a.heads, h = nh - n * a.heads;
 	const int i0 = qb * kRows, nq = min(kRows, a.tq - i0);
@@ -384,7 +384,7 @@ struct DScoresArgs {
 	float* ds;           // {N, heads, Tq, Tk}
 	const float* pad;
 	int heads, tq, tk, d;
-	int qblocks, total, first;  // blocks of a (sample, head) pair and of this launch, this launch's first block
+	int qblocks, total;
 	int causal;
 	float scale;
 };
@@ -400,7 +400,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) a
 	extern __shared__ __align__(16) float sm[];
 	__shared__ float rowdot[kRows];
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	const int lid = a.first + xcd_remap(blockIdx.x, a.total);
+	const int lid = xcd_remap(blockIdx.x, a.total);
 	const int nh = lid / a.qblocks, qb = lid - nh * a.qblocks;
 	const int n = nh / a.heads, h = nh - n * a.heads;
 	const int i0 = qb * kRows, nq = min(kRows, a.tq - i0);
@@ -504,7 +504,9 @@ bool attention_fused_ok(int64_t tq, int64_t tk, int64_t dh, int64_t d, const voi
 	auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
 	// the kernel runs S = Q K^T and O = P V as whole-depth chains: products that take the depth cut go elsewhere
 	if (depth_cut(tq, tk, dh) || depth_cut(tq, dh, tk)) return false;
-	return dh == kDh && tk >= 1 && tk <= kMaxKeys && tk % 4 == 0 && d % 4 == 0 && tq >= 1 && tq < (1 << 24) &&
+	// one sample's blocks in a launch
+	if (dh != kDh || d / kDh * ((tq + kRows - 1) / kRows) > kMaxGrid) return false;
+	return tk >= 1 && tk <= kMaxKeys && tk % 4 == 0 && d % 4 == 0 && tq >= 1 && tq < (1 << 24) &&
 	       al(q) && al(k) && al(v) && al(out) && al(probs) && (pad == nullptr || al(pad));
 }
 
@@ -515,12 +517,6 @@ hipError_t attention_fused_forward(const float* q, const float* k, const float* 
 	if (total == 0) return hipSuccess;
 	if (total >= ((int64_t)1 << 31) || n * heads * tq * tk >= ((int64_t)1 << 62)) return hipErrorInvalidValue;
 	FusedArgs a;
-	a.q = q;
-	a.k = k;
-	a.v = v;
-	a.out = out;
-	a.probs = probs;
-	a.pad = pad;
 	a.heads = (int)heads;
 	a.tq = (int)tq;
 	a.tk = (int)tk;
@@ -529,9 +525,16 @@ hipError_t attention_fused_forward(const float* q, const float* k, const float* 
 	a.causal = causal ? 1 : 0;
 	a.scale = scale;
 	const int lds = 4 * kRows * score_stride((int)tk);
-	for (int64_t first = 0; first < total; first += kMaxGrid) {
-		a.first = (int)first;
-		a.total = (int)std::min(kMaxGrid, total - first);
+	const int64_t most = kMaxGrid / (heads * qblocks);  // samples of a launch
+	for (int64_t n0 = 0; n0 < n; n0 += most) {
+		const int64_t q0 = n0 * tq * d, k0 = n0 * tk * d, cnt = std::min(most, n - n0);
+		a.q = q + q0;
+		a.k = k + k0;
+		a.v = v + k0;
+		a.out = out + q0;
+		a.probs = probs + n0 * heads * tq * tk;
+		a.pad = pad ? pad + n0 * tk : nullptr;
+		a.total = (int)(cnt * heads * qblocks);
 		hipLaunchKernelGGL(attention_fused_kernel, dim3((unsigned)a.total), dim3(256), lds, s, a);
 		const hipError_t e = hipGetLastError();
 		if (e != hipSuccess) return e;
@@ -546,11 +549,6 @@ hipError_t attention_fused_dscores(const float* g, const float* v, const float* 
 	if (total == 0) return hipSuccess;
 	if (total >= ((int64_t)1 << 31) || n * heads * tq * tk >= ((int64_t)1 << 62)) return hipErrorInvalidValue;
 	DScoresArgs a;
-	a.g = g;
-	a.v = v;
-	a.probs = probs;
-	a.ds = ds;
-	a.pad = pad;
 	a.heads = (int)heads;
 	a.tq = (int)tq;
 	a.tk = (int)tk;
@@ -559,9 +557,15 @@ hipError_t attention_fused_dscores(const float* g, const float* v, const float* 
 	a.causal = causal ? 1 : 0;
 	a.scale = scale;
 	const int lds = 4 * kRows * score_stride((int)tk);
-	for (int64_t first = 0; first < total; first += kMaxGrid) {
-		a.first = (int)first;
-		a.total = (int)std::min(kMaxGrid, total - first);
+	const int64_t most = kMaxGrid / (heads * qblocks);  // samples of a launch
+	for (int64_t n0 = 0; n0 < n; n0 += most) {
+		const int64_t p0 = n0 * heads * tq * tk, cnt = std::min(most, n - n0);
+		a.g = g + n0 * tq * d;
+		a.v = v + n0 * tk * d;
+		a.probs = probs + p0;
+		a.ds = ds + p0;
+		a.pad = pad ? pad + n0 * tk : nullptr;
+		a.total = (int)(cnt * heads * qblocks);
 		hipLaunchKernelGGL(attention_dscores_kernel, dim3((unsigned)a.total), dim3(256), lds, s, a);
 		const hipError_t e = hipGetLastError();
 		if (e != hipSuccess) return e;
