@@ -96,8 +96,9 @@ hipError_t prepare_device() {
 
 // Choice by measured device time on MI355X (every configuration on every BASELINE shape, and the MLP's). Each
 // output element is a K-long chain of dependent MFMAs: a dependent step costs about 64 cycles with 32x32x1 and 44
-// with 16x16x1 or 4x4x1, for one depth index, and 44 with 16x16x4 for four. Large products fill the GPU with
-// 128 x 128 or 128 x 64 tiles of 32x32x1 units (16-deep stages for A B, 32-deep when an operand is transposed);
+// with 16x16x1 or 4x4x1, for one depth index, and 44 with 16x16x4 for four. Large products (those that ring_takes
+// leaves: short ones, gathered ones, very long rows) fill the GPU with 128 x 128 or 128 x 64 tiles of 32x32x1 units
+// (16-deep stages for A B, 32-deep when an operand is transposed);
 // from about 4 million outputs down to 2^20, 128 x 128 and then 64 x 64 workgroups of 16x16x4 units; smaller
 // products use 32 x 32 workgroups of 16x16x4 units (one wave per 16 x 16 block, as many chains as possible), with
 // 64-deep stages (128-deep with op(A) transposed and 512 or more deep, 32-deep up to 32). Measured (us, exact
